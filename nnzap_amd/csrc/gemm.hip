@@ -6,28 +6,20 @@
 // steps (nnmetal/src/transformer.zig:4032-4068), and its only dequant-matmul
 // (`qmm`, compute.metal:2975-3083) stores W as [K x N] for the MNIST network.
 //
-// Design (v_mfma_f32_16x16x32_f16, fp32 accumulate):
-//   * One 64 (tokens) x 64 (W rows) output tile per block of 2 KQ waves:
-//     2 W-row halves x KQ k-phases (KQ = 8 for single matrices whose grid
-//     fits one block per CU, else 4; 2 for the gate/up pair).  Wave (wn, kq) computes a
-//     64 x 32 tile over the k-steps (64 k each) with index = kq mod KQ, so a
-//     W fragment expanded in registers feeds 4 MFMAs, an A fragment read
-//     from LDS feeds 2, and the KQ partial tiles are summed through LDS at
-//     the end.
-//   * A is staged in LDS KQ k-steps (64 KQ k) at a time, double-buffered, with
-//     one barrier per stage, by loads straight into LDS (global_load_lds,
-//     no registers); the 16-byte piece p of row r sits at slot p ^ (r & 15),
-//     so the 16 rows of an MFMA fragment read hit distinct banks.
-//   * W is staged as packed bits (a 16-byte entry per row and k-step: two
-//     code words and the group scale); each lane reads the 8 bits of its B
-//     fragment and expands them in registers to f16 +-s (two ALU operations
-//     per pair of weights).  +-s times an f16
-//     activation is exact in the MFMA, so the result differs from the decode
-//     QMV only in fp32 summation order.
-//   * Blocks are numbered so that those resident on one XCD share their
-//     64-token A tile (the XCD's L2 keeps it) when the token tiles divide by 8.
-//   * Epilogues match the decode kernels: f16 store (Q/K/V), residual += (O,
-//     down), silu(a)*b of a gate/up pair stored as f16.
+// Three kernels on v_mfma_f32_16x16x32_f16 with fp32 accumulation:
+//   * qgemm_kernel, the main one: the presets' weights (1-bit of group size
+//     128, 4-bit of group size 64 with bf16 scales) with K a multiple of 512;
+//   * dq_gemm_kernel (1-bit) and dq4_gemm_kernel (4-bit): every other K and
+//     group size, f16 scales of 4-bit weights, less aligned pointers.
+// In all of them a block owns 64 tokens, its waves are 2 W-row halves x KQ
+// k-phases (a W fragment expanded in registers feeds 4 MFMAs, an A fragment
+// read from LDS feeds 2 or 4, the KQ partial tiles meet in LDS at the end), A
+// goes straight into LDS (global_load_lds) with 16-byte piece p of row r at
+// slot p ^ (r & 15), so the 16 rows of a fragment read hit distinct banks, and
+// there is one barrier per stage.  +-s times an f16 activation is exact in the
+// MFMA, so a 1-bit result differs from the decode QMV only in fp32 summation
+// order.  Epilogues match the decode kernels: f16 store (Q/K/V), residual +=
+// (O, down), silu(a)*b of a gate/up pair stored as f16.
 #include "internal.h"
 
 namespace {
@@ -39,6 +31,10 @@ typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 template <int V> struct IC { static constexpr int value = V; };   // a compile-time index argument
 
 constexpr int BM = 64, BN = 64, BK = 64;
+
+// ---- 1-bit weights of any K and group size (multiples of 64): W staged as
+// packed bits, a 16-byte entry per row and k-step (two code words and the
+// group scale), expanded in registers to f16 +-s.
 // KQ k-phases (2 KQ waves, 128 KQ threads); an LDS stage holds KQ k-steps.
 template <int KQ> constexpr int SK = BK * KQ;        // k per LDS stage
 template <int KQ> constexpr int PIECES = SK<KQ> / 8; // 16-byte pieces per A row and stage
@@ -652,6 +648,494 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(2))) v
     }
 }
 
+// ---------------------------------------------------------------------------
+// The main GEMM kernel: 1-bit weights of group size 128 and 4-bit weights of
+// group size 64 with bf16 scales, K a multiple of 512, 16-byte aligned codes.
+//
+// Block: 64 tokens x NSUB sub-blocks of 64 W rows (a gate/up pair: one of each
+// matrix; a single matrix with NSUB = 2: 128 consecutive rows), 2 KQ waves =
+// 2 row halves x KQ k-phases.  An LDS stage is KQ steps of 64 k; wave (wn, kq)
+// takes step kq of every stage for 32 rows of each sub-block.
+//
+// dq_gemm_kernel and dq4_gemm_kernel above fetch W and its scales 8 and 2
+// bytes per row and step, a 128-byte line each time; with their compute taken
+// out they still took two thirds of their time.  Here everything is loaded
+// straight into LDS (no registers, no LDS stores) in pieces that use the lines
+// they touch: A 128 bytes per row and step, W codes 64 bytes per row (a chunk:
+// 512 k of 1-bit, 128 k of 4-bit codes), scales a dword.  A 4-bit weight is
+// dequantised exactly into its f16 operand (expand_nibbles_scaled), so its
+// accumulators run through K unscaled and only the bias products remain on
+// the VALU.  Measured before -> now, weights rotated: 1-bit gate/up 2 x 6144 x
+// 2048 at P = 512 33.8 -> 30.5 us (845 TFLOP/s), 2 x 9728 x 2560 at P = 3001
+// 295 -> 268 (1113 TFLOP/s; the library's bf16 GEMM of that size without any
+// dequantisation 1161); 2560 x 9728 at P = 3001 195 -> 157, 2560 x 4096 86 ->
+// 68, 6144 x 2560 126 -> 91; 4-bit gate/up 2 x 6144 x 2048 at P = 512 59.7 ->
+// 47, 2 x 9728 x 2560 at P = 1500 290 -> 230.  Bounds now: 1-bit, one round of
+// blocks at P = 512 (first loads and epilogue overlap nothing), at large P the
+// L2-to-LDS rate of A (8.7 TB/s over the chip) and MFMA issue; 4-bit, VALU
+// issue (188 per 40 MFMAs).  Three or four LDS stages in flight instead of
+// two: no faster (2048 x 6144, P = 512: 22.4-22.6 us against 21.7).
+//
+// MFMA k-slot order: lane group q = lane / 16 of the two MFMAs u = 0, 1 of a
+// step takes k = 16 q + 8 u .. + 8 of the step (any assignment is right as long
+// as A and B agree), so a lane's weights of a step are one aligned piece: 16
+// bits (1-bit) or 8 bytes (4-bit).
+// Straight-to-LDS loads from a wave-uniform base plus a 32-bit lane offset.
+// s_nop 4: gfx9 wants five wait states between a VALU write of an SGPR and a
+// memory instruction reading it (the compiler's hazard check does not look
+// into asm, and the base may come from a v_readfirstlane).
+__device__ __forceinline__ void load_lds_b128(const void *sbase, uint32_t voff, uint32_t lds) {
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
+}
+__device__ __forceinline__ void load_lds_b32(const void *sbase, uint32_t voff, uint32_t lds) {
+    asm volatile("s_nop 4\n\tglobal_load_lds_dword %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
+}
+// A wave-uniform pointer as an opaque scalar value: selecting between argument
+// fields through it keeps the compiler from selecting between their addresses,
+// which would copy the argument block to scratch memory.
+template <class T>
+__device__ __forceinline__ T *uniform_ptr(T *p) {
+    // readfirstlane returns int: through uint32_t, or the low half sign-extends
+    const uint64_t v = (uint64_t)p;
+    const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
+    const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
+    return (T *)((uint64_t)hi << 32 | lo);
+}
+template <class T>
+__device__ __forceinline__ uint32_t lds_addr(T *p) {
+    return (uint32_t)(size_t)(__attribute__((address_space(3))) T *)p;
+}
+
+// 16 weight bits -> the two B fragments' f16 values, +s where the bit is set
+// and -s where it is clear.  y carries the bits twice, 15 apart, so that bits
+// 2e and 2e + 1 sit 16 apart and one shift brings them to the sign positions.
+__device__ __forceinline__ void expand_bits16(uint32_t h, uint32_t ns2, half8 &f0, half8 &f1) {
+    uint32_t y;
+    asm("v_lshl_or_b32 %0, %1, 15, %1" : "=v"(y) : "v"(h));
+    u32x4 e, f;
+    e[0] = ((y << 15) & 0x80008000u) ^ ns2;
+    e[1] = ((y << 13) & 0x80008000u) ^ ns2;
+    e[2] = ((y << 11) & 0x80008000u) ^ ns2;
+    e[3] = ((y << 9) & 0x80008000u) ^ ns2;
+    f[0] = ((y << 7) & 0x80008000u) ^ ns2;
+    f[1] = ((y << 5) & 0x80008000u) ^ ns2;
+    f[2] = ((y << 3) & 0x80008000u) ^ ns2;
+    f[3] = ((y << 1) & 0x80008000u) ^ ns2;
+    f0 = __builtin_bit_cast(half8, e);
+    f1 = __builtin_bit_cast(half8, f);
+}
+
+// 8 nibbles -> S (n - 8) 2^-20, exactly: the nibble in bits 4..7 of a half is
+// the (denormal) f16 value n 2^-20, and one fused multiply-add with S and
+// c = -8 S 2^-20 scales and centres it.  A bf16 scale has 8 significant bits
+// and |n - 8| <= 8 three more, or is a power of two: 11 bits, an f16.
+__device__ __forceinline__ half8 expand_nibbles_scaled(uint32_t w, half2v S, half2v c) {
+    const uint32_t lo = (w << 4) & 0xF0F0F0F0u, hi = w & 0xF0F0F0F0u;   // n[2j], n[2j+1] in byte j
+    half8 r;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const uint32_t sel = (uint32_t)j | (0x0Cu << 8) | ((uint32_t)(4 + j) << 16) | (0x0Cu << 24);
+        const half2v v = __builtin_elementwise_fma(__builtin_bit_cast(half2v, __builtin_amdgcn_perm(hi, lo, sel)), S, c);
+        r[2 * j] = v[0];
+        r[2 * j + 1] = v[1];
+    }
+    return r;
+}
+
+struct GemmMat {
+    const void *codes;
+    const uint16_t *scales, *biases;   // biases: 4-bit only
+    void *out;
+    uint32_t rows;
+};
+// m[0..n): row segments of one launch (Q, K, V), each with its own output; a
+// gate/up pair: m[0] and m[1], one output.
+struct GemmArgs {
+    const f16_t *A;
+    GemmMat m0, m1, m2;
+    uint32_t n, P, K, nx;   // nx: W tiles of the launch
+};
+
+template <int BITS, int MODE, int NSUB, int KQ>
+__global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
+    constexpr bool PAIR = MODE == NNZ_GEMM_SILU_PAIR;
+    static_assert(!PAIR || NSUB == 2, "a pair has two sub-blocks");
+    constexpr int SK = BK * KQ, PIECES = SK / 8, THREADS = 128 * KQ, A_LOADS = 4, ROWS = 64 * NSUB;
+    constexpr int CSTEPS = BITS == 1 ? 8 : 2;                    // 64-k steps per W chunk
+    constexpr int CPS = KQ > CSTEPS ? KQ / CSTEPS : 1;           // chunks per buffer
+    constexpr int SPC = CSTEPS > KQ ? CSTEPS / KQ : 1;           // stages per buffer
+    constexpr int W_INSTR = 4 * NSUB * CPS, S_INSTR = 2 * NSUB * CPS, WAVES = 2 * KQ;
+    __shared__ __attribute__((aligned(16))) f16_t As[2][BM * SK];
+    __shared__ __attribute__((aligned(16))) uint32_t Wc[2][CPS][ROWS * 16];
+    __shared__ uint32_t Sc[2][CPS][ROWS * 2];
+    __shared__ int rowexp[BITS == 4 ? ROWS : 1];
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wn = wave & 1, kq = wave >> 1;
+    const int q = lane >> 4, r16 = lane & 15;
+
+    // Workgroups go round-robin over the 8 XCDs: XCD j takes the j-th eighth
+    // of the tiles, W tile fastest, so its L2 holds the few token tiles it
+    // works on and no other XCD reads them.
+    const uint32_t ny = ceil_div(ga.P, (uint32_t)BM), nb = ga.nx * ny;
+    const uint32_t idx = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    if (idx >= nb) return;
+    const uint32_t by = idx / ga.nx, bx = idx % ga.nx, p0 = by * BM;
+    const uint32_t K = ga.K, G = K / (BITS == 1 ? 128 : 64), rowbytes = K / 8 * BITS;
+    uint32_t n0 = bx * (PAIR ? 64u : (uint32_t)ROWS);
+    int seg = 0;
+    if (!PAIR && ga.n > 1) {
+        if (n0 >= ga.m0.rows) {
+            n0 -= ga.m0.rows;
+            seg = 1;
+            if (ga.n > 2 && n0 >= ga.m1.rows) {
+                n0 -= ga.m1.rows;
+                seg = 2;
+            }
+        }
+    }
+    auto pick = [&](auto f) __attribute__((always_inline)) {
+        auto *const v0 = uniform_ptr(f(ga.m0)), *const v1 = uniform_ptr(f(ga.m1)), *const v2 = uniform_ptr(f(ga.m2));
+        return seg == 0 ? v0 : (seg == 1 ? v1 : v2);
+    };
+    const void *const codes = pick([](const GemmMat &m) { return m.codes; });
+    const uint16_t *const scales = pick([](const GemmMat &m) { return m.scales; });
+    const uint16_t *const biases = pick([](const GemmMat &m) { return m.biases; });
+    void *const out = pick([](const GemmMat &m) { return m.out; });
+    const uint32_t r0 = ga.m0.rows, r1 = ga.m1.rows, r2 = ga.m2.rows, out_rows = seg == 0 ? r0 : (seg == 1 ? r1 : r2);
+    const char *const wbase0 = (const char *)codes + (size_t)n0 * rowbytes;
+    const char *const wbase1 = PAIR ? (const char *)ga.m1.codes + (size_t)n0 * rowbytes : wbase0 + (size_t)64 * rowbytes;
+    const uint16_t *const sbase0 = scales + (size_t)n0 * G;
+    const uint16_t *const sbase1 = PAIR ? ga.m1.scales + (size_t)n0 * G : sbase0 + (size_t)64 * G;
+    const uint16_t *const bbase0 = BITS == 4 ? biases + (size_t)n0 * G : nullptr;
+    const uint16_t *const bbase1 = BITS == 4 ? (PAIR ? ga.m1.biases + (size_t)n0 * G : bbase0 + (size_t)64 * G) : nullptr;
+
+    // A: lane's slot lp of rows lr + 16 u holds piece lp ^ (row & 15), so the
+    // 16 rows of a fragment read hit distinct banks; rows past P re-read row
+    // P - 1, their results are not stored.
+    const int lp = tid & (PIECES - 1), lr = tid / PIECES;
+    uint32_t avoff[A_LOADS];
+#pragma unroll
+    for (int u = 0; u < A_LOADS; ++u)
+        avoff[u] = (min(p0 + (uint32_t)(lr + 16 * u), ga.P - 1) - p0) * K * 2u + (uint32_t)(lp ^ (lr & 15)) * 16u;
+    const char *const abase = (const char *)(ga.A + (size_t)p0 * K);
+    // W chunk: 64 bytes per row as 4 pieces, piece p of row r at slot
+    // p ^ ((r >> 2) & 3); instruction i fills rows 16 i .. 16 i + 15.
+    const int wrow = lane >> 2;
+    const uint32_t wvoff = (uint32_t)wrow * rowbytes + (uint32_t)((lane & 3) ^ ((wrow >> 2) & 3)) * 16u;
+
+    auto issue_a = [&](uint32_t st) __attribute__((always_inline)) {
+        const char *const sb = abase + (size_t)st * (SK * 2);
+        const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(As[st & 1] + 8 * (wave * 64)));
+#pragma unroll
+        for (int u = 0; u < A_LOADS; ++u) load_lds_b128(uniform_ptr(sb), avoff[u], l0 + 16u * (uint32_t)(u * THREADS));
+    };
+    // buffer b of W: chunks b CPS .. of every row
+    auto issue_w = [&](uint32_t b) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i0 = 0; i0 < W_INSTR; i0 += WAVES) {
+            const int i = i0 + wave;
+            if (W_INSTR % WAVES == 0 || i < W_INSTR) {   // wave-uniform
+                const int c = i / (4 * NSUB), j = i % (4 * NSUB);
+                const char *const sb = (NSUB == 2 && j >= 4 ? wbase1 : wbase0) + (size_t)(j & 3) * 16 * rowbytes +
+                                       (size_t)(b * CPS + c) * 64;
+                load_lds_b128(uniform_ptr(sb), wvoff, __builtin_amdgcn_readfirstlane(lds_addr(&Wc[b & 1][c][j * 256])));
+            }
+        }
+#pragma unroll
+        for (int i0 = 0; i0 < S_INSTR; i0 += WAVES) {
+            const int i = i0 + (WAVES - 1 - wave);       // the waves with less W first
+            if (S_INSTR % WAVES == 0 || (i >= 0 && i < S_INSTR)) {
+                const int c = i / (2 * NSUB), j = i % (2 * NSUB), sub = j >> 1, h = j & 1;
+                const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(&Sc[b & 1][c][sub * 128 + h * 64]));
+                if constexpr (BITS == 1) {   // 4 scales of a row = 2 dwords: rows 32 h .. of the sub-block
+                    const char *const sb = (const char *)(sub ? sbase1 : sbase0) + (size_t)(b * CPS + c) * 8;
+                    load_lds_b32(uniform_ptr(sb), (uint32_t)(32 * h + (lane >> 1)) * G * 2u + (uint32_t)(lane & 1) * 4u, l0);
+                } else {                     // 2 scales (h = 0) or biases (h = 1) of a row = 1 dword
+                    const uint16_t *const s0 = uniform_ptr(sbase0), *const s1 = uniform_ptr(sbase1);
+                    const uint16_t *const b0 = uniform_ptr(bbase0), *const b1 = uniform_ptr(bbase1);
+                    const uint16_t *const t0 = h ? b0 : s0, *const t1 = h ? b1 : s1;
+                    const char *const sb = (const char *)(sub ? t1 : t0) + (size_t)(b * CPS + c) * 4;
+                    load_lds_b32(uniform_ptr(sb), (uint32_t)lane * G * 2u, l0);
+                }
+            }
+        }
+    };
+
+    float4v acc[NSUB][4][2];
+#pragma unroll
+    for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) acc[s][i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
+
+    const uint32_t nst = K / SK;
+    auto issue = [&](uint32_t st) __attribute__((always_inline)) {   // W before the A of its first stage
+        if (st % SPC == 0) issue_w(st / SPC);
+        issue_a(st);
+    };
+    issue(0);
+    int ex[NSUB][2];
+    if constexpr (BITS == 4) {
+        // Row exponents: S = s 2^e with the row's largest |s| in [2^15, 2^16),
+        // so that S (n - 8) 2^-20 is exact in f16 for scales down to 2^-12 of
+        // the largest; below that weights are rounded at 2^-25, which is 2^-23
+        // of the row's largest weight 8 |s|, a float32 rounding of its terms.  The row's threads scan its scales.
+        constexpr int TPR = THREADS / ROWS;   // threads per row
+        static_assert(TPR == 2 || TPR == 4 || TPR == 8, "a row's threads are lanes of one octet");
+        const int row = tid / TPR, sub = row >> 6;
+        const uint16_t *const s0 = uniform_ptr(sbase0), *const s1 = uniform_ptr(sbase1);
+        const auto *const sp = (const __attribute__((address_space(1))) u32x4 *)((sub ? s1 : s0) + (size_t)(row & 63) * G);
+        uint32_t mx = 0;
+        for (uint32_t p = tid % TPR; p < G / 8; p += 4 * TPR) {
+            u32x4 v[4];   // four loads in flight; past the row's end the last piece again
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[e] = sp[min(p + (uint32_t)(e * TPR), G / 8 - 1)];
+#pragma unroll
+            for (int e = 0; e < 16; ++e) mx = max(mx, max(v[e / 4][e % 4] & 0x7FFFu, (v[e / 4][e % 4] >> 16) & 0x7FFFu));
+        }
+#pragma unroll
+        for (int o = 1; o < TPR; o *= 2) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
+        const int e8 = (int)(min(mx, 0x7F7Fu) >> 7);
+        if (tid % TPR == 0) rowexp[row] = mx ? 142 - e8 : 0;   // 15 - (e8 - 127)
+    }
+    load_barrier();
+    if constexpr (BITS == 4) {
+#pragma unroll
+        for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) ex[s][j] = rowexp[64 * s + 32 * wn + 16 * j + r16];
+    }
+
+    const half8 ones = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f,
+                        (_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f};
+    auto compute = [&](uint32_t st) __attribute__((always_inline)) {
+        const f16_t *const buf = As[st & 1];
+        const uint32_t wb = (st / SPC) & 1;
+        const int step = SPC > 1 ? (int)(st % SPC) * KQ + kq : kq;   // step within the W buffer
+        const int c = step / CSTEPS, cs = step % CSTEPS;
+        half8 af[2][4];
+#pragma unroll
+        for (int u = 0; u < 2; ++u)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                af[u][i] = *(const half8 *)(buf + (i * 16 + r16) * SK + 8 * ((kq * 8 + 2 * q + u) ^ r16));
+        if constexpr (BITS == 1) {
+#pragma unroll
+            for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int row = 64 * s + 32 * wn + 16 * j + r16;
+                    const uint32_t h = *((const uint16_t *)&Wc[wb][c][row * 16 + (((cs >> 1) ^ ((row >> 2) & 3)) << 2)] +
+                                         (cs & 1) * 4 + q);
+                    const uint32_t sc = *((const uint16_t *)&Sc[wb][c][row * 2] + (cs >> 1));
+                    half8 b0, b1;
+                    expand_bits16(h, (sc | (sc << 16)) ^ 0x80008000u, b0, b1);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0][i], b0, acc[s][i][j], 0, 0, 0);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1][i], b1, acc[s][i][j], 0, 0, 0);
+                }
+        } else {
+            const uint16_t *const sp = (const uint16_t *)&Sc[wb][c][0];
+            half2v S[NSUB][2];
+            float b8[NSUB][2];
+#pragma unroll
+            for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int at = s * 256 + (32 * wn + 16 * j + r16) * 2 + cs;
+                    const float sc = __builtin_ldexpf(bf16_to_f32(sp[at]), ex[s][j]);
+                    S[s][j] = __builtin_bit_cast(half2v, __builtin_amdgcn_cvt_pkrtz(sc, sc));
+                    // the centred nibbles miss 8 s: bias b + 8 s times the row sum
+                    b8[s][j] = fmaf((float)S[s][j][0], 0x1p-17f, __builtin_ldexpf(bf16_to_f32(sp[at + 128]), ex[s][j] - 20));
+                }
+            // row sums of A over the step's group (every column of A . ones),
+            // their bias products
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                float4v xs = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0][i], ones, (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                xs = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1][i], ones, xs, 0, 0, 0);
+#pragma unroll
+                for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+#pragma unroll
+                        for (int r = 0; r < 4; ++r) acc[s][i][j][r] = fmaf(b8[s][j], xs[r], acc[s][i][j][r]);
+            }
+#pragma unroll
+            for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int row = 64 * s + 32 * wn + 16 * j + r16;
+                    const u32x2 w = *(const u32x2 *)&Wc[wb][c][row * 16 + (((2 * cs + (q >> 1)) ^ ((row >> 2) & 3)) << 2) +
+                                                                  (q & 1) * 2];
+                    const half2v c8 = S[s][j] * (half2v){(_Float16)-0x1p-17f, (_Float16)-0x1p-17f};
+                    const half8 b0 = expand_nibbles_scaled(w[0], S[s][j], c8);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0][i], b0, acc[s][i][j], 0, 0, 0);
+                    const half8 b1 = expand_nibbles_scaled(w[1], S[s][j], c8);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+                        acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1][i], b1, acc[s][i][j], 0, 0, 0);
+                }
+        }
+    };
+
+    for (uint32_t st = 0; st < nst; ++st) {
+        if (st + 1 < nst) issue(st + 1);   // block-uniform
+        compute(st);
+        load_barrier();
+    }
+
+    // k-phase reduction through the (free) A buffers: phases [h, 2h) hand
+    // their tiles to [0, h) down to phases 0 and 1, which then swap halves
+    // and both finish the block (phase 0 the 16-row tiles i = 0, 1).
+    constexpr int NF = NSUB * 8;
+    float4v *red = (float4v *)&As[0][0];
+    static_assert(KQ / 2 * 2 * NF * 64 * 16 <= (int)sizeof(As), "reduction slots fit the stage buffers");
+#pragma unroll
+    for (int h = KQ / 2; h >= 2; h /= 2) {
+        if (kq >= h && kq < 2 * h) {
+#pragma unroll
+            for (int t = 0; t < NF; ++t) red[(((kq - h) * 2 + wn) * NF + t) * 64 + lane] = acc[t / 8][(t / 2) % 4][t % 2];
+        }
+        __syncthreads();
+        if (kq < h) {
+#pragma unroll
+            for (int t = 0; t < NF; ++t) acc[t / 8][(t / 2) % 4][t % 2] += red[((kq * 2 + wn) * NF + t) * 64 + lane];
+        }
+        __syncthreads();
+    }
+    auto put_half = [&](int slot, auto hh) __attribute__((always_inline)) {
+        constexpr int H = decltype(hh)::value;
+#pragma unroll
+        for (int t = 0; t < NF / 2; ++t)
+            red[(slot * (NF / 2) + t) * 64 + lane] = acc[t / 4][2 * H + (t / 2) % 2][t % 2];
+    };
+    auto add_half = [&](int slot, auto hh) __attribute__((always_inline)) {
+        constexpr int H = decltype(hh)::value;
+#pragma unroll
+        for (int t = 0; t < NF / 2; ++t)
+            acc[t / 4][2 * H + (t / 2) % 2][t % 2] += red[(slot * (NF / 2) + t) * 64 + lane];
+    };
+    if (kq == 0) put_half(2 + wn, IC<1>{});   // phase 1's tiles
+    else if (kq == 1) put_half(wn, IC<0>{});  // phase 0's tiles
+    __syncthreads();
+    if (kq >= 2) return;   // after the last barrier
+    if (kq == 0) add_half(wn, IC<0>{});
+    else add_half(2 + wn, IC<1>{});
+
+    // D layout: lane holds rows 4 q + r, column r16 of each 16 x 16 tile.
+    auto epilogue = [&](auto ti) __attribute__((always_inline)) {
+        constexpr int i = decltype(ti)::value;
+        auto value = [&](int s, int j, int r) __attribute__((always_inline)) {
+            float v = acc[s][i][j][r];
+            if constexpr (BITS == 4) v = __builtin_ldexpf(v, 20 - ex[s][j]);
+            return v;
+        };
+        auto rnd = [&](float v) __attribute__((always_inline)) { return BITS == 4 ? bf16_trunc(v) : v; };
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            const uint32_t p = p0 + i * 16 + 4 * q + r;
+            if (p >= ga.P) continue;
+#pragma unroll
+            for (int s = 0; s < (PAIR ? 1 : NSUB); ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const uint32_t n = n0 + 64 * s + 32 * wn + 16 * j + r16;
+                    const size_t o = (size_t)p * out_rows + n;
+                    const float v = value(s, j, r);
+                    if constexpr (MODE == NNZ_GEMM_STORE_F16) ((f16_t *)out)[o] = (f16_t)rnd(v);
+                    else if constexpr (MODE == NNZ_GEMM_STORE_F32) ((float *)out)[o] = rnd(v);
+                    else if constexpr (MODE == NNZ_GEMM_RESADD) ((float *)out)[o] += rnd(v);
+                    else ((f16_t *)out)[o] = (f16_t)rnd(silu_mul(v, value(NSUB - 1, j, r)));
+                }
+        }
+    };
+    if (kq == 0) {
+        epilogue(IC<0>{});
+        epilogue(IC<1>{});
+    } else {
+        epilogue(IC<2>{});
+        epilogue(IC<3>{});
+    }
+}
+
+// The forms the main kernel takes.  Others (K not a multiple of 512, other
+// group sizes, f16 scales of 4-bit weights, less aligned pointers) run on the
+// kernels above.
+bool qgemm_weight_ok(const nnz_qweight *w, uint32_t K) {
+    return w && K % 512 == 0 && ((uintptr_t)w->codes & 15) == 0 &&
+           (w->bits == 1 ? w->group_size == 128 && ((uintptr_t)w->scales & 3) == 0
+                         : w->group_size == 64 && w->scale_dtype == NNZ_BF16 && ((uintptr_t)w->scales & 15) == 0 &&
+                               ((uintptr_t)w->biases & 3) == 0);
+}
+
+template <int BITS, int MODE, int NSUB, int KQ>
+void qgemm_start(nnz_ctx *ctx, GemmArgs ga, uint32_t rows) {
+    ga.nx = rows / (MODE == NNZ_GEMM_SILU_PAIR ? 64u : 64u * NSUB);
+    const uint32_t nb = ga.nx * ceil_div(ga.P, (uint32_t)BM);
+    qgemm_kernel<BITS, MODE, NSUB, KQ><<<ceil_div(nb, 8u) * 8u, 128 * KQ, 0, ctx->stream>>>(ga);
+}
+
+// Shape of a single-matrix launch (one or more row segments), by how many
+// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (50 / 42 KB of LDS), 2
+// of KQ = 4 (75 KB), one of KQ = 8 (140 KB).  More than one round of 768
+// KQ = 2 blocks: 128-row blocks, half the A traffic (2560 x 4096, P = 3001: 68
+// us against 76 with 64 rows; 6144 x 2560: 91 against 108; 4096 x 2048, P =
+// 1024: 23.5 against 26.6).  512 < g <= 768: one round of KQ = 2 64-row blocks
+// (2048 x 2048, P = 1500: 19.3 us against 21.4 with 128 rows and 23.7 on KQ =
+// 4, which takes a second round; 6144 x 2560, P = 512: 22.6 against 25.1 and
+// 25.0).  Fewer: KQ = 4, more waves per block (2048 x 6144, P = 1024: 33.5
+// against 38.5 on KQ = 2; 2048 x 2048, P = 512: 9.7 against 10.2).  At most one
+// block per CU and K > 2048: KQ = 8 (1-bit; 2048 x 6144, P = 512: 21.7 against
+// 25.4 on KQ = 4; at K = 2048 KQ = 4 is ahead, 9.7 against 10.3; the 4-bit
+// stages of KQ = 8 do not fit LDS).
+template <int BITS, int MODE>
+void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128) {
+    const uint32_t ny = ceil_div(ga.P, (uint32_t)BM);
+    const uint32_t g = rows / 64 * ny;   // blocks of 64 rows
+    if (g > 768) {
+        if (rows128) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
+        else qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
+    } else if (g > 512) {
+        qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
+    } else {
+        if constexpr (BITS == 1) {
+            if (g <= 256 && ga.K > 2048) return qgemm_start<BITS, MODE, 1, 8>(ctx, ga, rows);
+        }
+        qgemm_start<BITS, MODE, 1, 4>(ctx, ga, rows);
+    }
+}
+
+template <int BITS>
+int qgemm_launch(nnz_ctx *ctx, const nnz_qweight *wa, const nnz_qweight *wb, const f16_t *A, uint32_t P, void *out,
+                 int mode, const nnz_qmv_dims &d) {
+    auto mat = [&](const nnz_qweight *w) {
+        return GemmMat{w->codes, (const uint16_t *)w->scales, (const uint16_t *)w->biases, out, d.M};
+    };
+    GemmArgs ga{A, mat(wa), {}, {}, 1, P, d.K, 0};
+    const bool r128 = d.M % 128 == 0;
+    switch (mode) {
+    case NNZ_GEMM_STORE_F16: qgemm_single<BITS, NNZ_GEMM_STORE_F16>(ctx, ga, d.M, r128); break;
+    case NNZ_GEMM_STORE_F32: qgemm_single<BITS, NNZ_GEMM_STORE_F32>(ctx, ga, d.M, r128); break;
+    case NNZ_GEMM_RESADD: qgemm_single<BITS, NNZ_GEMM_RESADD>(ctx, ga, d.M, r128); break;
+    case NNZ_GEMM_SILU_PAIR:
+        ga.m1 = mat(wb);
+        qgemm_start<BITS, NNZ_GEMM_SILU_PAIR, 2, 2>(ctx, ga, d.M);
+        break;
+    default: return nnz_fail(ctx, NNZ_EINVAL, "dequant_gemm: unknown mode %d", mode);
+    }
+    NNZ_LAUNCHED(ctx);
+    return NNZ_OK;
+}
+
 // k-phases and W-row groups of the single-matrix launches.  Measured at P =
 // 512: with a grid of at most one block per CU and K > 2048 (the down
 // projection), 8 k-phases (16 waves, 149 KB of LDS) are faster than 4
@@ -702,6 +1186,8 @@ int gemm4_launch(nnz_ctx *ctx, const nnz_qweight *wa, const nnz_qweight *wb, con
                 NNZ_EUNSUPPORTED,
                 "dequant_gemm: need M %% 64 == 0, K %% 64 == 0, power-of-two group size %% 64 == 0");
     NNZ_REQUIRE(ctx, ((uintptr_t)a & 15) == 0, NNZ_EINVAL, "dequant_gemm: A must be 16-byte aligned");
+    if (qgemm_weight_ok(wa, d.K) && (!pair || qgemm_weight_ok(wb, d.K)))
+        return qgemm_launch<4>(ctx, wa, wb, (const f16_t *)a, P, out, mode, d);
     const uint32_t gl = (uint32_t)__builtin_ctz(d.group_size);
     const uint32_t grid = d.M / BN * ceil_div(P, BM);
     const f16_t *A = (const f16_t *)a;
@@ -770,6 +1256,8 @@ int nnz_gemm_launch(nnz_ctx *ctx, const nnz_qweight *wa, const nnz_qweight *wb, 
     }
     NNZ_REQUIRE(ctx, (d.group_size & (d.group_size - 1)) == 0, NNZ_EUNSUPPORTED,
                 "dequant_gemm: group size must be a power of two");
+    if (qgemm_weight_ok(wa, d.K) && (!pair || qgemm_weight_ok(wb, d.K)))
+        return qgemm_launch<1>(ctx, wa, wb, (const f16_t *)a, P, out, mode, d);
     const uint32_t gl = (uint32_t)__builtin_ctz(d.group_size);
     const uint32_t grid = d.M / BN * ceil_div(P, BM);
     const f16_t *A = (const f16_t *)a;
@@ -815,6 +1303,19 @@ int nnz_gemm_segments_launch(nnz_ctx *ctx, const nnz_qweight *const *w, void *co
         rows[i] = w[i]->packed_count / K;
         NNZ_REQUIRE(ctx, rows[i] % BN == 0, NNZ_EUNSUPPORTED, "gemm_segments: rows %% 64 != 0");
         M += rows[i];
+    }
+    bool main_form = true, r128 = true;
+    for (int i = 0; i < nw; ++i) {
+        main_form = main_form && qgemm_weight_ok(w[i], K);
+        r128 = r128 && rows[i] % 128 == 0;
+    }
+    if (main_form) {
+        GemmArgs ga{(const f16_t *)a, {}, {}, {}, (uint32_t)nw, P, K, 0};
+        GemmMat *const m[3] = {&ga.m0, &ga.m1, &ga.m2};
+        for (int i = 0; i < nw; ++i) *m[i] = GemmMat{w[i]->codes, (const uint16_t *)w[i]->scales, nullptr, out[i], rows[i]};
+        qgemm_single<1, NNZ_GEMM_STORE_F16>(ctx, ga, M, r128);
+        NNZ_LAUNCHED(ctx);
+        return NNZ_OK;
     }
     GemmSegs sg{(uint32_t)nw, rows[0], rows[1],
                 nw > 1 ? (const uint32_t *)w[1]->codes : nullptr,

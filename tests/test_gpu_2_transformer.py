@@ -458,3 +458,55 @@ def test_gemm_row_equals_decode_qmv(dev):
     ops.dispatch_qmv_f16in(dev, dw, tdev(a16[5]), y)
     dev.sync()
     assert_close(host(out)[5], host(y), rtol=1e-4, what="gemm row vs qmv")
+
+
+@pytest.mark.parametrize("bits,P,M,K", [(1, 1, 64, 512), (1, 65, 192, 1536), (1, 64, 128, 4096),
+                                        (1, 1030, 3136, 512), (1, 833, 3840, 512),
+                                        (4, 1, 64, 512), (4, 65, 192, 1536), (4, 64, 128, 4096),
+                                        (4, 1030, 3136, 512), (4, 833, 3840, 512)])
+def test_dequant_gemm_main_shapes(dev, bits, P, M, K):
+    """The main prefill GEMM at the edges of its launch shapes: one token, one
+    past a token tile, one 64-row block, eight and four k-phases, two k-phases
+    on 64-row blocks (rows not a multiple of 128, and up to 768 blocks) and on
+    128-row ones, one W chunk and several.  The 4-bit rows hold scales over
+    eleven octaves, negative and zero ones among them, each row at a size of
+    its own."""
+    from nnzap_amd import formats as fm
+    from nnzap_amd.formats import QWeight
+    rng = np.random.default_rng([bits, P, M, K])
+
+    def weight():
+        if bits == 1:
+            return cf.q1_matrix(M, K, 128, int(rng.integers(1 << 30)), int(rng.integers(1 << 30)))
+        s = np.exp2(rng.uniform(-11, 0, (M, K // 64)) + rng.integers(-20, 20, (M, 1)))
+        s *= rng.choice([-1.0, 0.0, 1.0, 1.0], s.shape)
+        b = 8 * s * rng.uniform(-1.2, 0.2, s.shape)
+        return QWeight(4, M, K, 64, rng.integers(0, 1 << 32, (M, K // 8), dtype=np.uint32),
+                       S.f64_to_bf16_bits(s), S.f64_to_bf16_bits(b), fm.DT_BF16)
+
+    wa, wb = weight(), weight()
+    a16 = (0.5 * rng.standard_normal((P, K))).astype(np.float16)
+    A, da, db = a16.astype(np.float64), ops.DeviceQWeight(dev, wa), ops.DeviceQWeight(dev, wb)
+    Wa, Wb = O.dequant(wa), O.dequant(wb)
+    ra, rb, ad = A @ Wa.T, A @ Wb.T, tdev(a16)
+    out16 = torch.empty(P, M, dtype=torch.float16, device="cuda")
+    out32 = torch.empty(P, M, dtype=torch.float32, device="cuda")
+    ops.dispatch_dequant_gemm(dev, da, ad, out32, L.GEMM_STORE_F32)
+    if bits == 1:
+        ops.dispatch_dequant_gemm(dev, da, ad, out16, L.GEMM_SILU_PAIR, wb=db)
+        dev.sync()
+        # fp32 summation (random walk, 4 sigma) of terms |a| s
+        se = 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ np.abs(Wa).T)
+        assert (np.abs(host(out32) - ra) <= se).all()
+        assert_close(host(out16), O.f16(O.silu(ra) * rb), what="silu pair")
+        return
+    dev.sync()
+    # the sums run over centred weights (n - 8) s and (b + 8 s): their terms
+    # bound the summation error
+    def terms(w):
+        s = S.bf16_bits_to_f32(w.scales).astype(np.float64)[:, :, None]
+        b = S.bf16_bits_to_f32(w.biases).astype(np.float64)[:, :, None]
+        n = fm.unpack_q4(w.codes, K).reshape(M, K // 64, 64).astype(np.float64)
+        return (np.abs((n - 8) * s) + np.abs(b + 8 * s)).reshape(M, K)
+    se = 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ terms(wa).T)
+    assert_bf16_faithful(host(out32), ra, "q4 gemm main", sum_err=se)
