@@ -45,7 +45,7 @@ struct NnzAttnCall {
 };
 
 uint32_t nnz_attn_chunk(uint32_t seq_len, uint32_t hkv);
-uint32_t nnz_attn_fused_chunk(uint32_t max_seq, uint32_t hkv);
+uint32_t nnz_attn_fused_chunk(uint32_t max_seq, uint32_t hq, uint32_t head_dim);
 int nnz_rope_table_launch(nnz_ctx *ctx, float *out, uint32_t head_dim, float theta);
 int nnz_attn_launch_ex(nnz_ctx *ctx, const NnzAttnCall &c);
 // Single-query attention with the partials carved out of `scratch`
@@ -66,8 +66,8 @@ int nnz_argmax_launch(nnz_ctx *ctx, const float *x, uint32_t n, uint32_t *oi, fl
 int nnz_attn_fused1_launch(nnz_ctx *ctx, const void *q, const void *kr, const void *vr,
                            const float *qn, const float *kn, void *kc, void *vc, void *out,
                            float *part_o, float *part_ml, const uint32_t *d_seq, uint32_t max_seq,
-                           uint32_t hq, uint32_t hkv, uint32_t head_dim, uint32_t max_ctx,
-                           float eps, float theta, const float *inv_freq,
+                           uint32_t chunk, uint32_t hq, uint32_t hkv, uint32_t head_dim,
+                           uint32_t max_ctx, float eps, float theta, const float *inv_freq,
                            bool partials_only = false);
 int nnz_qmv_norm_qkv_launch(nnz_ctx *ctx, const nnz_qweight *wq, const nnz_qweight *wk,
                             const nnz_qweight *wv, const float *residual, const float *norm_w,

@@ -463,16 +463,17 @@ int enqueue_decode_step(nnz_model *m, uint32_t max_seq, bool top2 = false) {
         // transformer.zig:3244-3370 encodeAttentionGather: Q/K norm, RoPE, KV
         // append and attention in one launch, then O-proj with residual +=.
         // Up to MERGE chunks of partials, the O-projection merges them itself.
-        const uint32_t nch = ceil_div(max_seq, nnz_attn_fused_chunk(max_seq, c.num_kv_heads));
+        const uint32_t chunk = nnz_attn_fused_chunk(max_seq, c.num_query_heads, c.head_dim);
+        const uint32_t nch = ceil_div(max_seq, chunk);
         const bool merge_in_o = nch <= NNZ_O_MERGE_MAX_CHUNKS;
         RC(nnz_attn_fused1_launch(ctx, m->q, m->k, m->v, Ly.q_norm, Ly.k_norm, Ly.kc, Ly.vc, m->att,
-                                  m->part_o, m->part_ml, m->state + ST_SEQ, max_seq,
+                                  m->part_o, m->part_ml, m->state + ST_SEQ, max_seq, chunk,
                                   c.num_query_heads, c.num_kv_heads, c.head_dim,
                                   c.max_context_length, c.rms_eps, c.rope_theta, m->rope_inv,
                                   merge_in_o));
         if (merge_in_o)
             RC(nnz_qmv_merge_resadd_launch(ctx, &Ly.o.w, m->part_o, m->part_ml, m->state + ST_SEQ,
-                                           max_seq, nch, nnz_attn_fused_chunk(max_seq, c.num_kv_heads),
+                                           max_seq, nch, chunk,
                                            c.head_dim, m->residual, dims_of(m, Ly.o)));
         else if (is_q4(m))
             RC(nnz_dispatch_q4mv_f16io_resadd(ctx, &Ly.o.w, m->att, m->residual, dims_of(m, Ly.o)));
@@ -540,7 +541,7 @@ bool lm_head_top2(const nnz_model *m) {
 }
 
 void decode_plan(const nnz_model *m, uint32_t max_seq, uint32_t *chunk, uint32_t *nch) {
-    *chunk = nnz_attn_fused_chunk(max_seq, m->c.num_kv_heads);
+    *chunk = nnz_attn_fused_chunk(max_seq, m->c.num_query_heads, m->c.head_dim);
     *nch = ceil_div(max_seq, *chunk);
 }
 
@@ -937,7 +938,7 @@ int capture_step(nnz_model *m, uint32_t max_seq, nnz_graph **g) {
 // per run of `per` attention-chunk counts, `per` the smallest that keeps the
 // plan within MAX_STEP_GRAPHS graphs.
 int capture_steps(nnz_model *m, uint32_t first, uint32_t last, StepGraphs &s) {
-    const uint32_t chunk = nnz_attn_fused_chunk(last, m->c.num_kv_heads);
+    const uint32_t chunk = nnz_attn_fused_chunk(last, m->c.num_query_heads, m->c.head_dim);
     const uint32_t c0 = ceil_div(first, chunk), c1 = ceil_div(last, chunk);
     const uint32_t per = ceil_div(c1 - c0 + 1, MAX_STEP_GRAPHS);
     s.first = first;

@@ -1583,9 +1583,8 @@ int nnz_dispatch_qmv_merge_f16io_resadd(nnz_ctx *ctx, const nnz_qweight *w, cons
     NNZ_CHECK_CTX(ctx);
     NNZ_REQUIRE(ctx, seq_len > 0 && head_dim > 0, NNZ_EINVAL, "merge_o_resadd: zero dims");
     NNZ_REQUIRE(ctx, w && w->bits == 1, NNZ_EINVAL, "merge_o_resadd: 1-bit weights");
-    const uint32_t chunk = nnz_attn_fused_chunk(seq_len, 1);
-    return nnz_qmv_merge_resadd_launch(ctx, w, part_o, part_ml, d_seq_len, seq_len,
-                                       ceil_div(seq_len, chunk), chunk, head_dim, residual, dims);
+    const uint32_t nch = nnz_gqa_partial_chunks(seq_len);
+    return nnz_qmv_merge_resadd_launch(ctx, w, part_o, part_ml, d_seq_len, seq_len, nch, 64u, head_dim, residual, dims);
 }
 
 // ---------------------------- Q1 ------------------------------------------

@@ -596,7 +596,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
 //     * scores with 256/FCHUNK lanes per token, one softmax pass for all G
 //       heads, P.V with a thread per (d, token part);
 //     * one chunk: f16 output; several: partials (m, l, o) for
-//       attn_merge_kernel, which folds them with one round of loads.
+//       attn_combine_slice_kernel, which folds them with one round of loads.
 // Caches: f16, K [Hkv][max_ctx][D], V [Hkv][D][max_ctx]; seq_len and
 // position come from device memory (graph replay) when d_seq is set.
 constexpr int FCHUNK = 64;
@@ -620,7 +620,7 @@ struct FusedAttnArgs {
 };
 
 // Offset of partial output (query head qh, chunk c, dim d) in part_o.
-// Head-major (attn_merge_kernel): [Hq][nchunks][D].  Unit-major (the O
+// Head-major (attn_combine_slice_kernel): [Hq][nchunks][D].  Unit-major (the O
 // projection's merge prologue, qmv.hip): chunk by chunk, column k = qh D + d
 // of the K = Hq D columns at ((k >> 2) & 7) K / 8 + (k >> 5) 4 + (k & 3) --
 // nibble n of every 32-column unit together, so a lane per unit reads one
@@ -867,7 +867,7 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(FusedAttnArgs a) {
     }
     __syncthreads();
 
-    // One chunk: final output.  Several: partials for attn_merge_kernel
+    // One chunk: final output.  Several: partials for the combine
     // (merging here would need an agent-scope fence between workgroups,
     // which on a multi-XCD part writes back and invalidates the XCD's L2;
     // a kernel boundary is the cheaper synchronisation).
@@ -1093,52 +1093,297 @@ __global__ __launch_bounds__(256) void attn_fused_wave_kernel(FusedAttnArgs a) {
     }
 }
 
-// Fold the per-chunk partials of attn_fused_kernel: grid Hq, block 128.
-// The first MERGE_PRE chunks' (m, l) pairs and outputs are loaded in one
-// round together with seq_len -- (m, l) by one lane per chunk and shared
-// through LDS, so the loads stay vector loads; longer sequences loop over
-// the rest.
-constexpr int MERGE_PRE = 16;
+// The same for head_dim 128 on the matrix cores (v_mfma_f32_16x16x32_f16): one
+// block per (chunk of 4 KW tokens, KV head, up to GM query heads), wave w on
+// tokens KW w .. of the chunk, two block barriers (queries ready, waves
+// merged).
+//   * Every K and V load is issued before the sequence length is read: rows
+//     are clamped to the cache (max_ctx), not to the live length, so they wait
+//     on nothing; tokens past the length are masked by select (never
+//     multiplied), blocks of chunks past it exit.
+//   * K and V go from memory straight into the MFMA operands, no LDS:
+//     S^T[key][head] = K . Q^T with 16 key rows x 32 dims as A, the heads as
+//     the columns of B (columns past the group are zero), O^T[dim][head] =
+//     V^T . P^T with the probabilities fed from the S^T accumulators.  Row
+//     4 g + r of the key tiles (2 kk, 2 kk + 1) is key 32 kk + 8 g + (0 | 4) + r,
+//     so that lane group g's eight B slots are eight consecutive keys and a
+//     lane's V operand is one 16-byte load of its dim's row.
+//   * q is normalised and rotated by the wave w + 4 n of head w + 4 n (lane l
+//     on dims 2l, 2l + 1, a RoPE pair), scaled by log2(e) / sqrt(D) and split
+//     into f16 hi + lo like the probabilities: with both products accumulated
+//     the scores carry 2^-22 and P.V 2^-20 relative error, below the f16
+//     rounding of the attention output.
+//   * The block whose chunk holds position seq - 1 normalises, rotates and
+//     f16-rounds the new key (wave 3), appends it and the value to the caches
+//     and puts both into their lanes' operands.
+// Bound by one memory round trip, the launch and the chain between the two
+// barriers.  Against the VALU kernel with six barriers that ran these shapes
+// (with its merge, which had one block per head): 32 query and 8 KV heads, 1500
+// tokens 14.3 -> 7.1 us, 3001 23.8 -> 8.1, 8192 57.2 -> 11.5; 16 query heads,
+// 1000 tokens 9.9 -> 6.7, 4096 26.6 -> 8.5.
+template <int GM, int KW>
+__global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
+    typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+    typedef float float4v __attribute__((ext_vector_type(4)));
+    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+    constexpr int D = 128, CH = 4 * KW, NT = KW / 16, NK = KW >= 32 ? KW / 32 : 1, NH = (GM + 3) / 4;
+    constexpr int QP = D + 8;   // LDS pitch (halves) of a query part
+    __shared__ __align__(16) _Float16 qs[GM][2][QP];
+    __shared__ __align__(16) _Float16 knew[D];
+    __shared__ uint16_t vnew[D];
+    __shared__ __align__(16) float osh[4][GM][D];
+    __shared__ float2 mlsh[4][GM];
 
-__global__ __launch_bounds__(128) void attn_merge_kernel(const float *part_o, const float *part_ml,
-                                                         f16_t *out, const uint32_t *d_seq,
-                                                         uint32_t seq_len, uint32_t nchunks,
-                                                         uint32_t D) {
-    __shared__ float2 ml_s[MERGE_PRE];
-    const uint32_t seq = d_seq ? *d_seq : seq_len;
-    const uint32_t qh = blockIdx.x, d = threadIdx.x;
-    const size_t base = (size_t)qh * nchunks;
-    const uint32_t dd = d < D ? d : 0u;
-    const float2 mlv = *(const float2 *)(part_ml + (base + min(d % MERGE_PRE, nchunks - 1)) * 2);
-    float o[MERGE_PRE];
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, g = lane >> 4, c16 = lane & 15;
+    const uint32_t part = blockIdx.x / a.units, u = blockIdx.x % a.units;
+    const uint32_t c = u % a.nchunks, h = u / a.nchunks;
+    const uint32_t qh0 = h * a.gfull + part * GM, heads = min(a.gfull - part * GM, (uint32_t)GM);
+    const uint32_t t0 = c * CH, wt0 = t0 + (uint32_t)(w * KW);
+
+    // ---- loads: q, norm scales, the new K/V projections and the RoPE
+    // frequency first (the prologue waits for these only), then K and V
+    uint32_t qpair[NH];
 #pragma unroll
-    for (int c = 0; c < MERGE_PRE; ++c) {
-        const uint32_t cc = min((uint32_t)c, nchunks - 1);
-        o[c] = part_o[(base + cc) * D + dd];
+    for (int n = 0; n < NH; ++n) {
+        const uint32_t hh = (uint32_t)(w + 4 * n) < heads ? (uint32_t)(w + 4 * n) : 0u;
+        qpair[n] = ((const uint32_t *)(a.q + (size_t)(qh0 + hh) * D))[lane];
     }
-    if (d < MERGE_PRE) ml_s[d] = mlv;
-    __syncthreads();
-    if (d >= D) return;
-    const uint32_t nch = min(nchunks, ceil_div(seq, (uint32_t)FCHUNK));
-    float M = -INFINITY;
+    const float2 qn2 = ((const float2 *)a.qn)[lane];
+    const uint32_t kpair = ((const uint32_t *)(a.kr + (size_t)h * D))[lane];
+    const float2 kn2 = ((const float2 *)a.kn)[lane];
+    const uint32_t vpair = ((const uint32_t *)(a.vr + (size_t)h * D))[lane];
+    // a null table gets an empty range: the load returns 0 without touching
+    // memory (no branch around a load) and the frequency is computed below
+    const float freq_t = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(a.inv_freq), (short)0,
+                                          a.inv_freq ? D * 2 : 0, 0x00020000),
+        lane * 4, 0, 0));
+    const size_t kvh = (size_t)h * a.max_ctx * D;
+    // key of row `row` of tile t, from the wave's first
+    auto key_of = [](int t, int row) __attribute__((always_inline)) {
+        return KW >= 32 ? 32 * (t >> 1) + 8 * (row >> 2) + 4 * (t & 1) + (row & 3) : row;
+    };
+    u32x4 kreg[NT][4];
 #pragma unroll
-    for (int c = 0; c < MERGE_PRE; ++c) M = (uint32_t)c < nch ? fmaxf(M, ml_s[c].x) : M;
-    for (uint32_t c = MERGE_PRE; c < nch; ++c) M = fmaxf(M, part_ml[(base + c) * 2]);
-    float num = 0.f, den = 0.f;
+    for (int t = 0; t < NT; ++t) {
+        const uint32_t key = min(wt0 + (uint32_t)key_of(t, c16), a.max_ctx - 1);
+        const u32x4 *kp = (const u32x4 *)(a.kc + kvh + (size_t)key * D + 8 * g);
 #pragma unroll
-    for (int c = 0; c < MERGE_PRE; ++c) {
-        if ((uint32_t)c < nch) {
-            const float w = expf(ml_s[c].x - M);
-            den = fmaf(w, ml_s[c].y, den);
-            num = fmaf(w, o[c], num);
+        for (int ks = 0; ks < 4; ++ks) kreg[t][ks] = kp[4 * ks];
+    }
+    // V [d][t], dim 16 dt + c16: a group of keys starting at or past max_ctx
+    // (which max_ctx % 8 == 0 keeps whole) reads group 0
+    u32x4 vreg[NK][8];
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk) {
+        const uint32_t vs = wt0 + (uint32_t)(32 * kk + (KW >= 32 ? 8 : 4) * g);
+        const f16_t *vp = a.vc + kvh + (size_t)c16 * a.max_ctx + (vs < a.max_ctx ? vs : 0u);
+#pragma unroll
+        for (int dt = 0; dt < 8; ++dt) {
+            if constexpr (KW >= 32) {
+                vreg[kk][dt] = *(const u32x4 *)(vp + (size_t)(16 * dt) * a.max_ctx);
+            } else {
+                const u32x2 v2 = *(const u32x2 *)(vp + (size_t)(16 * dt) * a.max_ctx);
+                vreg[kk][dt] = (u32x4){v2[0], v2[1], 0u, 0u};
+            }
         }
     }
-    for (uint32_t c = MERGE_PRE; c < nch; ++c) {
-        const float w = expf(part_ml[(base + c) * 2] - M);
-        den = fmaf(w, part_ml[(base + c) * 2 + 1], den);
-        num = fmaf(w, part_o[(base + c) * D + d], num);
+
+    const uint32_t seq = a.d_seq ? *a.d_seq : a.seq_len;
+    if (t0 >= seq) return;   // block-uniform: no barrier is pending
+    const uint32_t pos = seq - 1;
+    const bool own = pos < t0 + CH;                          // block-uniform
+    const bool wnew = pos >= wt0 && pos < wt0 + KW;          // wave-uniform
+
+    const float freq = a.inv_freq ? freq_t : rope_inv_freq(lane, D, a.theta);
+    float sn, cs;
+    sincosf((float)pos * freq, &sn, &cs);
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+        const int hh = w + 4 * n;
+        float q0, q1;
+        unpack2<NNZ_F16>(qpair[n], q0, q1);
+        const float r = rsqrtf(wave_sum(fmaf(q1, q1, q0 * q0)) / (float)D + a.eps);
+        const float x0 = q0 * r * qn2.x, x1 = q1 * r * qn2.y;
+        const float sl = a.scale * 1.44269504088896341f;
+        const float qe = fmaf(x0, cs, -x1 * sn) * sl, qo = fmaf(x0, sn, x1 * cs) * sl;
+        const f16_t he = (f16_t)qe, ho = (f16_t)qo;
+        if (hh < GM) {
+            *(uint32_t *)&qs[hh][0][2 * lane] =
+                (uint32_t)__builtin_bit_cast(uint16_t, he) | (uint32_t)__builtin_bit_cast(uint16_t, ho) << 16;
+            *(uint32_t *)&qs[hh][1][2 * lane] =
+                (uint32_t)__builtin_bit_cast(uint16_t, (f16_t)(qe - (float)he)) |
+                (uint32_t)__builtin_bit_cast(uint16_t, (f16_t)(qo - (float)ho)) << 16;
+        }
     }
-    out[(size_t)qh * D + d] = (f16_t)(num / den);
+    if (own && w == 3) {
+        // the new key: RMSNorm * k_norm, RoPE, f16
+        float k0, k1;
+        unpack2<NNZ_F16>(kpair, k0, k1);
+        const float r = rsqrtf(wave_sum(fmaf(k1, k1, k0 * k0)) / (float)D + a.eps);
+        const float x0 = k0 * r * kn2.x, x1 = k1 * r * kn2.y;
+        const f16_t ke = (f16_t)fmaf(x0, cs, -x1 * sn), ko = (f16_t)fmaf(x0, sn, x1 * cs);
+        const uint32_t kw = (uint32_t)__builtin_bit_cast(uint16_t, ke) | (uint32_t)__builtin_bit_cast(uint16_t, ko) << 16;
+        *(uint32_t *)&knew[2 * lane] = kw;
+        *(uint32_t *)&vnew[2 * lane] = vpair;
+        if (part == 0) {
+            ((uint32_t *)(a.kc + kvh + (size_t)pos * D))[lane] = kw;
+            a.vc[kvh + (size_t)(2 * lane) * a.max_ctx + pos] = __builtin_bit_cast(f16_t, (uint16_t)(vpair & 0xFFFFu));
+            a.vc[kvh + (size_t)(2 * lane + 1) * a.max_ctx + pos] = __builtin_bit_cast(f16_t, (uint16_t)(vpair >> 16));
+        }
+    }
+    __syncthreads();
+
+    // ---- S^T = K . Q^T (log2 units)
+    half8 qh[4], ql[4];
+    {
+        const bool live = (uint32_t)c16 < heads;
+        const int hc = c16 < GM ? c16 : 0;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const half8 zero = {};
+            const half8 hi = *(const half8 *)&qs[hc][0][32 * ks + 8 * g], lo = *(const half8 *)&qs[hc][1][32 * ks + 8 * g];
+            qh[ks] = live ? hi : zero;
+            ql[ks] = live ? lo : zero;
+        }
+    }
+    if (wnew) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            const bool is_new = wt0 + (uint32_t)key_of(t, c16) == pos;
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const u32x4 nk = *(const u32x4 *)&knew[32 * ks + 8 * g];
+                kreg[t][ks] = is_new ? nk : kreg[t][ks];
+            }
+        }
+    }
+    float4v s[NT];
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        s[t] = (float4v){0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const half8 ka = __builtin_bit_cast(half8, kreg[t][ks]);
+            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh[ks], s[t], 0, 0, 0);
+            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[ks], s[t], 0, 0, 0);
+        }
+    }
+    // ---- softmax of head c16 over the wave's tokens
+    const bool tail = wt0 + KW > seq;   // wave-uniform
+    if (tail) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int r = 0; r < 4; ++r)
+                s[t][r] = wt0 + (uint32_t)key_of(t, 4 * g + r) < seq ? s[t][r] : -INFINITY;
+    }
+    float m = s[0][0];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) m = fmaxf(m, s[t][r]);
+    m = fmaxf(m, __shfl_xor(m, 16));
+    m = fmaxf(m, __shfl_xor(m, 32));
+    const float mu = m == -INFINITY ? 0.f : m;   // a wave past the length: p = 2^-inf = 0
+    float l = 0.f;
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            s[t][r] = __builtin_amdgcn_exp2f(s[t][r] - mu);
+            l += s[t][r];
+        }
+    l += __shfl_xor(l, 16);
+    l += __shfl_xor(l, 32);
+
+    // P^T: slot 8 g + e is the wave's key 32 kk + 8 g + e (KW 16: 4 g + e, e < 4)
+    half8 ph[NK], pl[NK];
+#pragma unroll
+    for (int kk = 0; kk < NK; ++kk)
+#pragma unroll
+        for (int sb = 0; sb < 2; ++sb)
+#pragma unroll
+            for (int r = 0; r < 4; r += 2) {
+                const int t = KW >= 32 ? 2 * kk + sb : 0;
+                const bool z = KW < 32 && sb == 1;
+                const float p0 = z ? 0.f : s[t][r], p1 = z ? 0.f : s[t][r + 1];
+                const auto hi = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+                const auto lo = __builtin_amdgcn_cvt_pkrtz(p0 - (float)hi[0], p1 - (float)hi[1]);
+                ph[kk][4 * sb + r] = hi[0];
+                ph[kk][4 * sb + r + 1] = hi[1];
+                pl[kk][4 * sb + r] = lo[0];
+                pl[kk][4 * sb + r + 1] = lo[1];
+            }
+    if (tail || wnew) {
+        // tokens past the length: value 0 (the weight is 0 too; never NaN *
+        // 0); the new token's value from its projection
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+            const uint32_t k0 = wt0 + (uint32_t)(32 * kk + (KW >= 32 ? 8 : 4) * g);
+#pragma unroll
+            for (int dt = 0; dt < 8; ++dt) {
+                const uint32_t nv = vnew[16 * dt + c16];   // read only where this block owns the new token
+#pragma unroll
+                for (int e = 0; e < (KW >= 32 ? 4 : 2); ++e) {
+                    uint32_t v = vreg[kk][dt][e];
+                    const uint32_t ka = k0 + 2u * e;
+                    v = ka < seq ? v : 0u;
+                    v = ka + 1 < seq ? v : v & 0xFFFFu;
+                    v = ka == pos ? (v & 0xFFFF0000u) | nv : v;
+                    v = ka + 1 == pos ? (v & 0xFFFFu) | nv << 16 : v;
+                    vreg[kk][dt][e] = v;
+                }
+            }
+        }
+    }
+    // ---- O^T = V^T . P^T: lane (g, c16) holds dims 16 dt + 4 g + r of head c16
+#pragma unroll
+    for (int dt = 0; dt < 8; ++dt) {
+        float4v o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int kk = 0; kk < NK; ++kk) {
+            const half8 va = __builtin_bit_cast(half8, vreg[kk][dt]);
+            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[kk], o, 0, 0, 0);
+            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[kk], o, 0, 0, 0);
+        }
+        if (c16 < GM) *(float4v *)&osh[w][c16][16 * dt + 4 * g] = o;
+    }
+    if (g == 0 && c16 < GM) mlsh[w][c16] = make_float2(m, l);
+    __syncthreads();
+
+    // ---- the four waves' partials -> the chunk's (m, l, o): dims 2l, 2l + 1
+    // of head w + 4 n
+#pragma unroll
+    for (int n = 0; n < NH; ++n) {
+        const int hh = w + 4 * n;
+        if ((uint32_t)hh >= heads) continue;   // wave-uniform
+        float2 ml[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) ml[i] = mlsh[i][hh];
+        const float M = fmaxf(fmaxf(ml[0].x, ml[1].x), fmaxf(ml[2].x, ml[3].x));
+        float lsum = 0.f, r0 = 0.f, r1 = 0.f;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float wgt = __builtin_amdgcn_exp2f(ml[i].x - M);   // M is finite: token t0 is live
+            const float2 o = *(const float2 *)&osh[i][hh][2 * lane];
+            lsum = fmaf(wgt, ml[i].y, lsum);
+            r0 = fmaf(wgt, o.x, r0);
+            r1 = fmaf(wgt, o.y, r1);
+        }
+        const uint32_t qh_ = qh0 + (uint32_t)hh;
+        if (a.direct) {
+            const f16_t he = (f16_t)(r0 / lsum), ho = (f16_t)(r1 / lsum);
+            ((uint32_t *)(a.out + (size_t)qh_ * D))[lane] =
+                (uint32_t)__builtin_bit_cast(uint16_t, he) | ((uint32_t)__builtin_bit_cast(uint16_t, ho) << 16);
+        } else {
+            // dims 2l, 2l + 1: adjacent in either layout (8-byte aligned);
+            // the maximum in natural units, as the merges take it
+            *(float2 *)(a.part_o + part_o_at(a, qh_, c, 2u * lane, D)) = make_float2(r0, r1);
+            if (lane == 0) ((float2 *)a.part_ml)[part_ml_at(a, qh_, c, D)] = make_float2(M * 0.693147180559945309f, lsum);
+        }
+    }
 }
 
 // ------------------------------------------------- single-query attention --
@@ -2135,18 +2380,36 @@ int nnz_attn_launch(nnz_ctx *ctx, const void *q, int qdt, const void *kc, const 
     return NNZ_OK;
 }
 
-// Chunk length of the fused decode attention (fixed: the kernel prefetches
-// a whole chunk into registers).
-uint32_t nnz_attn_fused_chunk(uint32_t, uint32_t) { return (uint32_t)FCHUNK; }
+// Whether the wave-organised kernel takes a head_dim 128 launch of `chunks`
+// 64-token chunks: while it gives each CU at most one block (one per chunk and
+// query head).  Measured, the attention launch alone, wave / MFMA kernel: 16
+// query and 8 KV heads, 100 tokens 3.52 / 3.96 us, 640 4.02 / 4.29, 1000 4.17 /
+// 4.20; 32 query heads, 200 tokens (128 blocks) 3.65 / 4.13, 640 (320 blocks)
+// 4.85 / 4.37.
+static bool attn_fused_by_wave(uint32_t chunks, uint32_t hq) { return chunks * hq <= 256; }
 
-// Fused decode attention (see attn_fused_kernel).  `max_seq` sizes the grid;
-// the live seq_len is d_seq ? *d_seq : max_seq.  part_o / part_ml hold
-// Hq * nchunks partials for the chunk from nnz_attn_fused_chunk.
+// Chunk length (tokens per partial) of the fused decode attention: 64 while
+// the O projection's merge takes the partials (16 chunks) or the wave kernel
+// runs, 128 beyond -- half the partials: 32 query and 8 KV heads, attention
+// and merge together, 3001 tokens 9.2 -> 8.1 us, 8192 13.9 -> 11.5; 1500 tokens
+// 7.1 -> 7.5, but then its 12 chunks need no merge launch in the decode step.
+// (256-token chunks, 64 per wave: 10.9 us at 3001, 12.5 at 8192.)
+uint32_t nnz_attn_fused_chunk(uint32_t max_seq, uint32_t hq, uint32_t head_dim) {
+    const uint32_t n64 = ceil_div(max_seq, (uint32_t)FCHUNK);
+    if (head_dim != 128 || n64 <= NNZ_O_MERGE_MAX_CHUNKS || attn_fused_by_wave(n64, hq)) return (uint32_t)FCHUNK;
+    return 128u;
+}
+
+// Fused decode attention (see attn_fused_mfma_kernel, and attn_fused_kernel
+// for head_dim 64).  `max_seq` sizes the grid; the live seq_len is d_seq ?
+// *d_seq : max_seq.  `chunk` tokens per partial: 64, or 128 for head_dim 128;
+// part_o / part_ml hold Hq * ceil(max_seq / chunk) partials.
 int nnz_attn_fused1_launch(nnz_ctx *ctx, const void *q, const void *kr, const void *vr,
                            const float *qn, const float *kn, void *kc, void *vc, void *out,
                            float *part_o, float *part_ml, const uint32_t *d_seq, uint32_t max_seq,
-                           uint32_t hq, uint32_t hkv, uint32_t head_dim, uint32_t max_ctx, float eps,
-                           float theta, const float *inv_freq, bool partials_only) {
+                           uint32_t chunk, uint32_t hq, uint32_t hkv, uint32_t head_dim,
+                           uint32_t max_ctx, float eps, float theta, const float *inv_freq,
+                           bool partials_only) {
     NNZ_REQUIRE(ctx, q && kr && vr && qn && kn && kc && vc && (out || partials_only) && part_o && part_ml,
                 NNZ_EINVAL, "gqa_fused_1pass: null buffer");
     NNZ_REQUIRE(ctx, hkv > 0 && hq % hkv == 0 && max_seq > 0 && max_seq <= max_ctx, NNZ_EINVAL,
@@ -2155,7 +2418,12 @@ int nnz_attn_fused1_launch(nnz_ctx *ctx, const void *q, const void *kr, const vo
                 "gqa_fused_1pass: head_dim %u (supported: 64, 128)", head_dim);
     NNZ_REQUIRE(ctx, max_ctx % 8 == 0 && ((uintptr_t)kc & 15) == 0 && ((uintptr_t)vc & 15) == 0,
                 NNZ_EUNSUPPORTED, "gqa_fused_1pass: caches must be 16-byte aligned, max_ctx %% 8 == 0");
+    NNZ_REQUIRE(ctx, chunk == (uint32_t)FCHUNK || (head_dim == 128 && chunk == 128),
+                NNZ_EINVAL, "gqa_fused_1pass: chunk %u", chunk);
     const uint32_t G = hq / hkv;
+    // groups other than 1, 2, 4 and 8 are for short sequences only
+    NNZ_REQUIRE(ctx, G == 1 || G == 2 || G == 4 || G == 8 || ceil_div(max_seq, (uint32_t)FCHUNK) * hkv < 128,
+                NNZ_EUNSUPPORTED, "gqa_fused_1pass: group %u", G);
     FusedAttnArgs a{};
     a.q = (const f16_t *)q;
     a.kr = (const f16_t *)kr;
@@ -2171,7 +2439,7 @@ int nnz_attn_fused1_launch(nnz_ctx *ctx, const void *q, const void *kr, const vo
     a.inv_freq = inv_freq;
     a.seq_len = max_seq;
     a.max_ctx = max_ctx;
-    a.nchunks = ceil_div(max_seq, (uint32_t)FCHUNK);
+    a.nchunks = ceil_div(max_seq, chunk);
     a.direct = a.nchunks == 1 && !partials_only;
     // partials for the O projection's merge: its unit-major layout
     a.unit_major = partials_only ? 1u : 0u;
@@ -2179,33 +2447,53 @@ int nnz_attn_fused1_launch(nnz_ctx *ctx, const void *q, const void *kr, const vo
     a.eps = eps;
     a.theta = theta;
     a.scale = 1.0f / sqrtf((float)head_dim);
-    // Few chunks x KV heads leave CUs idle: split each KV group over blocks
-    // of one query head, placed on one XCD so the K/V repeats hit its L2.
     a.gfull = G;
-    const uint32_t gb = (a.nchunks * hkv < 128) ? 1u : G;
     a.units = a.nchunks * hkv;
-    a.parts = G / gb;
-    const dim3 grid(a.parts == 1 ? a.units : ceil_div(a.units, 8u) * 8u * a.parts);
-#define FUSED(DD, GG) attn_fused_kernel<DD, GG><<<grid, 256, 0, ctx->stream>>>(a)
-    if (gb == 1) {
-        if (head_dim == 128) attn_fused_wave_kernel<<<grid, 256, 0, ctx->stream>>>(a);
-        else FUSED(64, 1);
+    if (head_dim == 128 && chunk == (uint32_t)FCHUNK && attn_fused_by_wave(a.nchunks, hq)) {
+        a.parts = G;
+        attn_fused_wave_kernel<<<ceil_div(a.units, 8u) * 8u * a.parts, 256, 0, ctx->stream>>>(a);
     } else if (head_dim == 128) {
-        if (G == 2) FUSED(128, 2);
-        else if (G == 4) FUSED(128, 4);
-        else if (G == 8) FUSED(128, 8);
-        else return nnz_fail(ctx, NNZ_EUNSUPPORTED, "gqa_fused_1pass: group %u", G);
-    } else {
-        if (G == 2) FUSED(64, 2);
-        else if (G == 4) FUSED(64, 4);
-        else if (G == 8) FUSED(64, 8);
-        else return nnz_fail(ctx, NNZ_EUNSUPPORTED, "gqa_fused_1pass: group %u", G);
-    }
+        a.parts = ceil_div(G, 8u);
+        const dim3 grid(a.units * a.parts);
+#define FUSED(GM, KW) attn_fused_mfma_kernel<GM, KW><<<grid, 256, 0, ctx->stream>>>(a)
+#define FUSED_G(KW)                    \
+    do {                               \
+        if (G <= 2) FUSED(2, KW);      \
+        else if (G <= 4) FUSED(4, KW); \
+        else FUSED(8, KW);             \
+    } while (0)
+        if (chunk == 64) FUSED_G(16);
+        else FUSED_G(32);
+#undef FUSED_G
 #undef FUSED
+    } else {
+        // Few chunks x KV heads leave CUs idle: split each KV group over blocks
+        // of one query head, placed on one XCD so the K/V repeats hit its L2.
+        const uint32_t gb = (a.nchunks * hkv < 128) ? 1u : G;
+        a.parts = G / gb;
+        const dim3 grid(a.parts == 1 ? a.units : ceil_div(a.units, 8u) * 8u * a.parts);
+        if (gb == 1) attn_fused_kernel<64, 1><<<grid, 256, 0, ctx->stream>>>(a);
+        else if (G == 2) attn_fused_kernel<64, 2><<<grid, 256, 0, ctx->stream>>>(a);
+        else if (G == 4) attn_fused_kernel<64, 4><<<grid, 256, 0, ctx->stream>>>(a);
+        else attn_fused_kernel<64, 8><<<grid, 256, 0, ctx->stream>>>(a);
+    }
     NNZ_LAUNCHED(ctx);
     if (a.nchunks > 1 && !partials_only) {
-        attn_merge_kernel<<<hq, 128, 0, ctx->stream>>>(part_o, part_ml, (f16_t *)out, d_seq, max_seq,
-                                                       a.nchunks, head_dim);
+        AttnArgs m{};
+        m.out = out;
+        m.part_o = part_o;
+        m.part_ml = part_ml;
+        m.d_seq = d_seq;
+        m.seq_len = max_seq;
+        m.chunk = chunk;
+        m.nchunks = a.nchunks;
+        m.hq = hq;
+        m.o_stride = hq * head_dim;
+        m.odt = NNZ_F16;
+        // a wave per (head, 8 dims) at any chunk count (7 chunks of 16 heads,
+        // with the attention: 6.9 us through the wave-per-64-dims form)
+        if (head_dim == 128) attn_combine_slice_kernel<128><<<dim3(hq, 16), 64, 0, ctx->stream>>>(m);
+        else attn_combine_slice_kernel<64><<<dim3(hq, 8), 64, 0, ctx->stream>>>(m);
         NNZ_LAUNCHED(ctx);
     }
     return NNZ_OK;
@@ -2440,13 +2728,13 @@ int nnz_dispatch_gqa_attention_fused_1pass(nnz_ctx *ctx, const void *q, void *k_
     const size_t need = nnz_gqa_scratch_bytes(d);
     NNZ_REQUIRE(ctx, scratch && scratch_bytes >= need, NNZ_EINVAL,
                 "gqa_fused_1pass: scratch of %zu bytes needed", need);
-    const uint32_t chunk = nnz_attn_fused_chunk(fd.seq_len, fd.num_kv_heads);
+    const uint32_t chunk = nnz_attn_fused_chunk(fd.seq_len, fd.num_query_heads, fd.head_dim);
     const uint32_t nch = ceil_div(fd.seq_len, chunk);
     float *base = (float *)(((uintptr_t)scratch + 255) & ~(uintptr_t)255);
     float *part_o = base;
     float *part_ml = base + (size_t)fd.num_query_heads * nch * fd.head_dim;
     return nnz_attn_fused1_launch(ctx, q, k_raw, v_raw, q_norm_scale, k_norm_scale, k_cache, v_cache,
-                                  output, part_o, part_ml, d_seq_len, fd.seq_len,
+                                  output, part_o, part_ml, d_seq_len, fd.seq_len, chunk,
                                   fd.num_query_heads, fd.num_kv_heads, fd.head_dim,
                                   fd.max_context_length, fd.eps, fd.rope_theta, nullptr);
 }
@@ -2468,7 +2756,7 @@ int nnz_dispatch_gqa_attention_partials(nnz_ctx *ctx, const void *q, void *k_cac
     NNZ_REQUIRE(ctx, ((uintptr_t)part_o & 15) == 0 && ((uintptr_t)part_ml & 7) == 0, NNZ_EINVAL,
                 "gqa_partials: part_o must be 16-byte and part_ml 8-byte aligned");
     return nnz_attn_fused1_launch(ctx, q, k_raw, v_raw, q_norm_scale, k_norm_scale, k_cache, v_cache,
-                                  nullptr, part_o, part_ml, d_seq_len, fd.seq_len, fd.num_query_heads,
+                                  nullptr, part_o, part_ml, d_seq_len, fd.seq_len, (uint32_t)FCHUNK, fd.num_query_heads,
                                   fd.num_kv_heads, fd.head_dim, fd.max_context_length, fd.eps,
                                   fd.rope_theta, rope_inv_freq, true);
 }

@@ -150,6 +150,43 @@ def test_gqa_fused_1pass_successive_positions(dev, hq, hkv, d):
     assert np.array_equal(host(vcd)[:, :, start:start + 8], vc_ref[:, :, start:start + 8])
 
 
+@pytest.mark.parametrize("hq,hkv,seq,ctx", [(32, 8, 1, 64), (32, 8, 512, 512), (32, 8, 513, 520),
+                                            (32, 8, 576, 576), (32, 8, 1024, 1024), (32, 8, 1025, 1032),
+                                            (16, 8, 1153, 1280), (8, 8, 2113, 2120), (16, 2, 2200, 2304),
+                                            (32, 2, 610, 616), (24, 8, 715, 720), (40, 8, 900, 904)])
+def test_gqa_fused_1pass_kernels(dev, hq, hkv, seq, ctx):
+    """The fused attention where its kernels and chunk lengths change (wave
+    kernel up to 256 (chunk, head) blocks, the MFMA one with 64- and 128-token
+    chunks), at the edges of chunks and of a wave's tokens, with groups of 1,
+    2, 3, 4, 5, 8 and 16 heads (two blocks of eight).  Everything past the
+    live length holds NaN and must not be read into a result."""
+    d, theta, pos = 128, 1e6, seq - 1
+    rng = np.random.default_rng([hq, hkv, seq])
+    qn, kn = ((1 + 0.1 * rng.standard_normal(d)).astype(np.float32) for _ in range(2))
+    kc = np.full((hkv, ctx, d), np.nan, np.float16)
+    vc = np.full((hkv, d, ctx), np.nan, np.float16)
+    kc[:, :pos] = rng.standard_normal((hkv, pos, d))
+    vc[:, :, :pos] = rng.standard_normal((hkv, d, pos))
+    q = rng.standard_normal((hq, d)).astype(np.float16)
+    kr = rng.standard_normal((hkv, d)).astype(np.float16)
+    vr = rng.standard_normal((hkv, d)).astype(np.float16)
+    kcd, vcd, qd, krd, vrd = tdev(kc), tdev(vc), tdev(q), tdev(kr), tdev(vr)
+    dims = L.GQAFusedDims(hq, hkv, d, seq, ctx, hq // hkv, pos, 1e-6, theta)
+    gd = L.GQADims(hq, hkv, d, seq, ctx, hq // hkv)
+    scr = torch.zeros(ops.gqa_scratch_bytes(gd) // 4 + 64, dtype=torch.float32, device="cuda")
+    out = torch.empty(hq, d, dtype=torch.float16, device="cuda")
+    ops.dispatch_gqa_attention_fused_1pass(dev, qd, kcd, vcd, out, krd, vrd, tdev(qn), tdev(kn), scr, dims)
+    dev.sync()
+    kr_, vr_ = kc[:, :seq].astype(np.float64), vc[:, :, :seq].astype(np.float64)
+    ref = O.gqa_fused_step(q.astype(np.float64), kr.astype(np.float64), vr.astype(np.float64),
+                           kr_, vr_, qn, kn, pos, theta, v_transposed=True)
+    assert_close(host(out), O.f16(ref), what=f"1pass {hq}/{hkv} seq={seq}")
+    assert_close(host(kcd)[:, pos], kr_[:, pos], what="k row")
+    assert np.array_equal(host(vcd)[:, :, pos], vr_[:, :, pos])
+    assert np.array_equal(host(kcd)[:, :pos], kr_[:, :pos])
+    assert np.isnan(host(kcd)[:, seq:]).all() and np.isnan(host(vcd)[:, :, seq:]).all()
+
+
 @pytest.mark.parametrize("pos", [30, 700, 1023])
 @pytest.mark.parametrize("freq_table", [False, True])
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (24, 12)])
