@@ -367,8 +367,275 @@ __global__ __launch_bounds__(64 * G * S) void attn_prefill_kernel(PrefillArgs a)
     }
 }
 
+// ---------------------------------------------------------------------------
+// Long prompts, head_dim 128: more queries per staged K/V tile.  (Counters at
+// G = 4, 3001 tokens: MFMA 65 % of the CUs' busy cycles, 300 VALU
+// instructions per 32 queries and 64 keys; a quarter of the time CUs idle as
+// the causal blocks run out.  279 -> 155 us, 4 heads x 8 KV heads; half the
+// flops of the MFMAs are the lo parts.)  The kernel
+// above reads a whole K and V tile from LDS for the 16 queries of a wave and
+// stages it for 16 queries x G heads, so at thousands of keys both the LDS and
+// the L2 bound it.  Here a wave owns 32 queries of one head
+// (v_mfma_f32_32x32x16_f16) and the block's G x NQG waves, 32 NQG queries,
+// share each tile: half the LDS reads per product and a (2 NQG)th of the
+// staging.
+//   * S^T[key][q] = K . Q^T per 32 keys; accumulator register 4 j + r of lane
+//     half hh is row 8 j + 4 hh + r of the tile.  Row m of the A operand is
+//     key m with bits 2 and 3 swapped, which makes the eight B slots of lane
+//     half hh in step s of O^T += V^T . P^T the consecutive keys 16 s + 8 hh ..,
+//     one 16-byte read of the V^T row, and P^T comes straight from the
+//     accumulators.  q and p are split into f16 hi + lo as above.
+//   * Tiles of 64 keys go from memory straight into LDS, double-buffered, one
+//     barrier per tile; piece p of a row sits at slot p ^ row (of 16 or 8
+//     slots), so that neighbouring lanes' 16-byte reads hit distinct banks.
+//   * A tile past the batch end has its V pieces zeroed in LDS (p = 0 must not
+//     meet a non-finite value); its K rows re-read the last key, masked.
+//   * Blocks: the KV head fastest, so with 8 KV heads each XCD's L2 holds one
+//     head's K and V.
+typedef float float16v __attribute__((ext_vector_type(16)));
+
+__device__ __forceinline__ void lds_load16(const void *sbase, uint32_t voff, uint32_t lds) {
+    // five wait states between a VALU write of an SGPR and its use as address
+    asm volatile("s_nop 4\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "{m0}"(lds) : "memory");
+}
+
+// p - (half H of hi), in one instruction (the compiler takes two)
+template <int H, class T>
+__device__ __forceinline__ float minus_half(float p, T hi) {
+    float r;
+    if constexpr (H == 0)
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel_hi:[1,0,0]" : "=v"(r) : "v"(__builtin_bit_cast(uint32_t, hi)), "v"(p));
+    else
+        asm("v_fma_mix_f32 %0, %1, -1.0, %2 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "=v"(r) : "v"(__builtin_bit_cast(uint32_t, hi)), "v"(p));
+    return r;
+}
+
+template <int G, int NQG>
+__global__ __launch_bounds__(64 * G * NQG) __attribute__((amdgpu_waves_per_eu(2))) void attn_prefill_long_kernel(PrefillArgs a) {
+    constexpr int D = 128, NW = G * NQG, NT = 64 * NW, QB = 32 * NQG;
+    constexpr int TILE = KT * D;                   // halves of a K (or V) tile
+    constexpr int LOADS = TILE / 8 / NT;           // 16-byte pieces per thread, K and V each
+    static_assert(TILE / 8 % NT == 0, "staging layout");
+    __shared__ __align__(16) _Float16 Ks[2][TILE];   // [key][D]
+    __shared__ __align__(16) _Float16 Vs[2][TILE];   // [dim][KT]
+
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int hh = lane >> 5, c = lane & 31;
+    const uint32_t hkv = a.hq / G, nqb = (a.n + QB - 1) / QB;
+    // heaviest first; every second batch of 256 blocks (one per CU) in reverse,
+    // so that the CUs' first two blocks weigh the same together
+    uint32_t L = blockIdx.x;
+    if ((L >> 8 & 1) && (L | 255u) < gridDim.x) L ^= 0xF8u;
+    const uint32_t kvh = L % hkv, qb = nqb - 1 - L / hkv;
+    const uint32_t h = kvh * G + (uint32_t)(wave % G), q0 = qb * QB + 32u * (uint32_t)(wave / G);
+    const uint32_t qi = q0 + (uint32_t)c, qc = qi < a.n ? qi : a.n - 1;
+    const uint32_t seq_end = a.start + a.n;
+    auto last_pos = [&](uint32_t q) { return a.start + (q < a.n ? q : a.n - 1); };
+    const uint32_t ntiles = last_pos(qb * QB + QB - 1) / KT + 1u;        // of the block
+    const uint32_t mytiles = q0 < a.n ? last_pos(q0 + 31) / KT + 1u : 0u;   // of the wave
+    const uint32_t qpos = a.start + qc;
+
+    const f16_t *const kbase = a.kc + (size_t)kvh * a.max_ctx * D;
+    const f16_t *const vbase = a.vc + (size_t)kvh * D * a.max_ctx;
+    // thread's pieces: K slot s of row r holds piece s ^ (r & 15); V^T slot s
+    // of row r holds piece s ^ (r & 7)
+    uint32_t krow[LOADS], kcol[LOADS], vrow[LOADS], vcol[LOADS];
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) {
+        const uint32_t p = (uint32_t)(tid + i * NT);
+        krow[i] = p / 16;
+        kcol[i] = ((p % 16) ^ (krow[i] & 15)) * 16u;
+        vrow[i] = p / 8 * a.max_ctx * 2u;
+        vcol[i] = ((p % 8) ^ (p / 8 & 7)) * 8u;
+    }
+    auto stage = [&](uint32_t t) __attribute__((always_inline)) {
+        const uint32_t k0 = t * KT, b = t & 1;
+        const uint32_t lk = __builtin_amdgcn_readfirstlane(
+            (uint32_t)(size_t)(__attribute__((address_space(3))) _Float16 *)(Ks[b] + 8 * 64 * wave));
+        const uint32_t lv = __builtin_amdgcn_readfirstlane(
+            (uint32_t)(size_t)(__attribute__((address_space(3))) _Float16 *)(Vs[b] + 8 * 64 * wave));
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const uint32_t key = min(k0 + krow[i], seq_end - 1);
+            lds_load16(kbase, key * (D * 2u) + kcol[i], lk + 16u * (uint32_t)(i * NT));
+        }
+#pragma unroll
+        for (int i = 0; i < LOADS; ++i) {
+            const uint32_t key = k0 + vcol[i];
+            lds_load16(vbase, vrow[i] + (key < a.max_ctx ? key * 2u : 0u), lv + 16u * (uint32_t)(i * NT));
+        }
+    };
+    stage(0);
+
+    // Q^T: lane (hh, c) holds dims 16 ks + 8 hh .. of query c, hi and lo
+    half8 qh[8], ql[8];
+    {
+        const f16_t *qp = a.q + ((size_t)qc * a.hq + h) * (2 * D);
+#pragma unroll
+        for (int ks = 0; ks < 8; ++ks) {
+            qh[ks] = *(const half8 *)(qp + 16 * ks + 8 * hh);
+            ql[ks] = *(const half8 *)(qp + D + 16 * ks + 8 * hh);
+        }
+    }
+    float16v o[4];
+#pragma unroll
+    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+        for (int e = 0; e < 16; ++e) o[dt][e] = 0.f;
+    float l_run = 0.f;
+    bool started = false;
+    float16v negm;
+#pragma unroll
+    for (int e = 0; e < 16; ++e) negm[e] = 0.f;
+    const int krm = (c & 19) | ((c & 4) << 1) | ((c & 8) >> 1);   // key of A row c
+
+    // the loads into LDS of the tile are waited for, then the barrier
+    auto tile_barrier = [&](uint32_t t) __attribute__((always_inline)) {
+        __builtin_amdgcn_s_waitcnt(7 << 4);   // vmcnt 0, lgkmcnt 0
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (t * KT + KT > seq_end) {   // block-uniform: keys past the batch, V = 0
+            for (uint32_t i = (uint32_t)tid; i < (uint32_t)TILE; i += NT) {
+                const uint32_t r = i / KT, s = i % KT / 8;
+                if (t * KT + ((s ^ (r & 7)) * 8u) + i % 8 >= seq_end) Vs[t & 1][i] = (_Float16)0.f;
+            }
+            __syncthreads();
+        }
+    };
+    tile_barrier(0);
+    for (uint32_t t = 0; t < ntiles; ++t) {
+        if (t + 1 < ntiles) stage(t + 1);   // block-uniform
+        if (t < mytiles) {                  // wave-uniform
+            const uint32_t k0 = t * KT;
+            const _Float16 *const Kt = Ks[t & 1], *const Vt = Vs[t & 1];
+#pragma unroll
+            for (int kt = 0; kt < 2; ++kt) {
+                // scores minus the reference m: the accumulator starts at -m
+                const int row = 32 * kt + krm;
+                half8 kf[8];
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks)
+                    kf[ks] = *(const half8 *)(Kt + row * D + 8 * ((2 * ks + hh) ^ (row & 15)));
+                float16v s = negm;
+#pragma unroll
+                for (int ks = 0; ks < 8; ++ks) {
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], qh[ks], s, 0, 0, 0);
+                    s = __builtin_amdgcn_mfma_f32_32x32x16_f16(kf[ks], ql[ks], s, 0, 0, 0);
+                }
+                half8 vf[4];   // V^T of the first 16-key step
+#pragma unroll
+                for (int dt = 0; dt < 4; ++dt)
+                    vf[dt] = *(const half8 *)(Vt + (32 * dt + c) * KT + 8 * ((4 * kt + hh) ^ (c & 7)));
+                // register e = 4 j + r: key 32 kt + 16 (j >> 1) + 8 hh + 4 (j & 1) + r
+                const uint32_t kk0 = k0 + (uint32_t)(32 * kt);
+                if (kk0 + 31u > a.start + q0) {   // wave-uniform
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        const uint32_t key = kk0 + (uint32_t)(16 * (e >> 3) + 8 * hh + (e & 7));
+                        s[e] = key <= qpos ? s[e] : -INFINITY;
+                    }
+                }
+                float mx = s[0];
+#pragma unroll
+                for (int e = 0; e < 16; ++e) mx = fmaxf(mx, s[e]);
+                const float2 mp = swap32(mx, mx);
+                const float rise = fmaxf(mp.x, mp.y);   // of the maximum over m
+                // The sums are kept relative to m, which follows the maximum
+                // only when that runs ahead by more than 2^8 (p <= 256 costs
+                // neither the f16 pairs nor the float32 sums any precision):
+                // rescaling at every new maximum of one of 32 queries would
+                // run for most tiles.  A query whose keys so far are all
+                // masked has no m yet.
+                if (__builtin_amdgcn_ballot_w64(rise > (started ? 8.f : -INFINITY))) {   // wave-uniform
+                    const bool move = rise > (started ? 8.f : -INFINITY);
+                    const float up = move ? rise : 0.f;
+                    const float alpha = started ? __builtin_amdgcn_exp2f(-up) : 1.f;   // sums are 0 before the start
+                    started = started || move;
+                    l_run *= alpha;
+#pragma unroll
+                    for (int e = 0; e < 16; ++e) {
+                        s[e] -= up;
+                        negm[e] -= up;
+                    }
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+                        for (int e = 0; e < 16; ++e) o[dt][e] *= alpha;
+                }
+                float ls = 0.f;
+#pragma unroll
+                for (int e = 0; e < 16; ++e) {
+                    s[e] = __builtin_amdgcn_exp2f(s[e]);
+                    ls += s[e];
+                }
+                const float2 lp = swap32(ls, ls);
+                l_run += lp.x + lp.y;
+#pragma unroll
+                for (int st = 0; st < 2; ++st) {   // 16 keys: P^T and O^T += V^T . P^T
+                    half8 ph, pl;
+#pragma unroll
+                    for (int e = 0; e < 8; e += 2) {
+                        const float p0 = s[8 * st + e], p1 = s[8 * st + e + 1];
+                        const auto hi = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+                        const auto lo = __builtin_amdgcn_cvt_pkrtz(minus_half<0>(p0, hi), minus_half<1>(p1, hi));
+                        ph[e] = hi[0];
+                        ph[e + 1] = hi[1];
+                        pl[e] = lo[0];
+                        pl[e + 1] = lo[1];
+                    }
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[dt], ph, o[dt], 0, 0, 0);
+#pragma unroll
+                    for (int dt = 0; dt < 4; ++dt) {
+                        o[dt] = __builtin_amdgcn_mfma_f32_32x32x16_f16(vf[dt], pl, o[dt], 0, 0, 0);
+                        if (st == 0) vf[dt] = *(const half8 *)(Vt + (32 * dt + c) * KT + 8 * ((4 * kt + 2 + hh) ^ (c & 7)));
+                    }
+                }
+            }
+        }
+        if (t + 1 < ntiles) tile_barrier(t + 1);   // block-uniform
+    }
+    if (qi < a.n) {
+        const float inv = 1.0f / l_run;
+        f16_t *const op = a.out + ((size_t)qi * a.hq + h) * D;
+#pragma unroll
+        for (int dt = 0; dt < 4; ++dt)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                uint32_t w[2];
+#pragma unroll
+                for (int e = 0; e < 2; ++e)
+                    w[e] = (uint32_t)__builtin_bit_cast(uint16_t, (f16_t)(o[dt][4 * j + 2 * e] * inv)) |
+                           (uint32_t)__builtin_bit_cast(uint16_t, (f16_t)(o[dt][4 * j + 2 * e + 1] * inv)) << 16;
+                *(uint2 *)(op + 32 * dt + 8 * j + 4 * hh) = make_uint2(w[0], w[1]);
+            }
+    }
+}
+
+template <int G, int NQG>
+void launch_long(nnz_ctx *ctx, const PrefillArgs &a, uint32_t hkv) {
+    const uint32_t nqb = (a.n + 32 * NQG - 1) / (32 * NQG);
+    attn_prefill_long_kernel<G, NQG><<<nqb * hkv, 64 * G * NQG, 0, ctx->stream>>>(a);
+}
+
 template <int D>
 int launch_d(nnz_ctx *ctx, const PrefillArgs &a, uint32_t hkv, uint32_t G) {
+    // Measured, 8 KV heads, this kernel / the long one: G = 2 512 tokens (64
+    // blocks of 64 queries) 12.3 / 20.6 us, 1024 (128 blocks) 36.2 / 35.3, 1500
+    // (192) 62.7 / 50.6; G = 4 300 tokens (80 blocks of 32) 14.2 / 16.6, 512
+    // (128) 20.6 / 21.0, 768 (192) 36.3 / 29.7, 1500 98.8 / 62.0, 3001 279 / 155.
+    if constexpr (D == 128) {
+        const uint32_t qb = G == 2 ? 64u : 32u;
+        if ((a.n + qb - 1) / qb * hkv > 128) {
+            if (G == 2) launch_long<2, 2>(ctx, a, hkv);
+            else if (G == 4) launch_long<4, 1>(ctx, a, hkv);
+            else launch_long<8, 1>(ctx, a, hkv);
+            NNZ_LAUNCHED(ctx);
+            return NNZ_OK;
+        }
+    }
     const dim3 grid((a.n + 15) / 16, hkv);
     switch (G) {
     case 2: attn_prefill_kernel<D, 2, S_G2><<<grid, 128 * S_G2, 0, ctx->stream>>>(a); break;

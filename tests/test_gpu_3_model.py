@@ -167,6 +167,32 @@ def test_tiny_long_prefill_matches_oracle(mdev, hq, hkv, hd):
         m.close()
 
 
+@pytest.mark.parametrize("hq,hkv,n1,n2", [(32, 16, 600, 571), (64, 16, 300, 293), (64, 8, 600, 553)])
+def test_tiny_long_kernel_prefill_matches_oracle(mdev, hq, hkv, n1, n2):
+    """Batches of more than 128 (query block, KV head) pairs at head_dim 128
+    run the 32-query prefill attention: groups of 2, 4 and 8 heads, a batch
+    from 0 and one behind it, neither ending at a tile or a query block, over
+    caches that hold NaN everywhere at first."""
+    from nnzap_amd import model as MD
+    cfg = cf.DecoderConfig(**{**cf.TINY.__dict__, "max_context_length": 1200,
+                              "max_prefill_length": 600, "num_query_heads": hq,
+                              "num_kv_heads": hkv, "head_dim": 128})
+    w = cf.decoder_weights(cfg, norm_mode="unit")
+    ids = cf.prompt_ids(cfg, n1 + n2)
+    ref = OracleDecoder(w).forward(list(ids), 0)
+    m = DecoderModel(mdev, cfg)
+    try:
+        m.load(w)
+        nan = np.full(hkv * 1200 * 128, np.nan, np.float16)
+        for l in range(cfg.num_layers):
+            m.upload(MD.T_K_CACHE, l, nan)
+            m.upload(MD.T_V_CACHE, l, nan)
+        assert_close_normwise(m.prefill(ids[:n1], 0), ref[n1 - 1], what=f"{n1}-token prefill")
+        assert_close_normwise(m.prefill(ids[n1:], n1), ref[-1], what=f"prefill at start {n1}")
+    finally:
+        m.close()
+
+
 @pytest.mark.parametrize("use_graph", [True, False])
 def test_tiny_generate_matches_oracle(mdev, tiny, use_graph):
     cfg, w = tiny
