@@ -16,10 +16,15 @@ struct nnz_ctx {
     bool own_stream = false;
     bool capturing = false;
     int q1_matrix_cores = 0;   // NNZ_OPT_Q1_MATRIX_CORES
+    float *gemm_ws = nullptr;  // partial sums of split-K prefill GEMMs [NNZ_GEMM_WS_FLOATS], or null
     std::string err;
     hipEvent_t ev[64] = {};
     bool ev_ok[64] = {};
 };
+
+// The context's GEMM workspace: launches of a context run on its stream, in
+// order, so one buffer serves them all.  256 blocks (one per CU) of 64 x 64.
+constexpr size_t NNZ_GEMM_WS_FLOATS = (size_t)256 * 64 * 64;
 
 struct nnz_graph {
     hipGraph_t graph = nullptr;

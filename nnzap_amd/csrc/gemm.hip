@@ -22,6 +22,8 @@
 // (O, down), silu(a)*b of a gate/up pair stored as f16.
 #include "internal.h"
 
+#include <algorithm>
+
 namespace {
 
 typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -754,12 +756,14 @@ struct GemmArgs {
     const f16_t *A;
     GemmMat m0, m1, m2;
     uint32_t n, P, K, nx;   // nx: W tiles of the launch
+    float *part;            // split-K: partial sums [splits][P][cols], cols = the launch's rows
+    uint32_t splits, cols;
 };
 
-template <int BITS, int MODE, int NSUB, int KQ>
+template <int BITS, int MODE, int NSUB, int KQ, bool SPLIT>
 __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     constexpr bool PAIR = MODE == NNZ_GEMM_SILU_PAIR;
-    static_assert(!PAIR || NSUB == 2, "a pair has two sub-blocks");
+    static_assert(!PAIR || (NSUB == 2 && !SPLIT), "a pair has two sub-blocks, and is not split");
     constexpr int SK = BK * KQ, PIECES = SK / 8, THREADS = 128 * KQ, A_LOADS = 4, ROWS = 64 * NSUB;
     constexpr int CSTEPS = BITS == 1 ? 8 : 2;                    // 64-k steps per W chunk
     constexpr int CPS = KQ > CSTEPS ? KQ / CSTEPS : 1;           // chunks per buffer
@@ -779,8 +783,17 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     // of the tiles, W tile fastest, so its L2 holds the few token tiles it
     // works on and no other XCD reads them.
     const uint32_t ny = ceil_div(ga.P, (uint32_t)BM), nb = ga.nx * ny;
-    const uint32_t idx = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
-    if (idx >= nb) return;
+    uint32_t idx = (blockIdx.x & 7) * (gridDim.x >> 3) + (blockIdx.x >> 3);
+    uint32_t sp = 0, kb = 0, ke = ga.K;   // the block's k range: whole 512-k pieces
+    if constexpr (SPLIT) {
+        if (idx >= nb * ga.splits) return;
+        sp = idx / nb;
+        idx -= sp * nb;
+        kb = ga.K / 512 * sp / ga.splits * 512;
+        ke = ga.K / 512 * (sp + 1) / ga.splits * 512;
+    } else {
+        if (idx >= nb) return;
+    }
     const uint32_t by = idx / ga.nx, bx = idx % ga.nx, p0 = by * BM;
     const uint32_t K = ga.K, G = K / (BITS == 1 ? 128 : 64), rowbytes = K / 8 * BITS;
     uint32_t n0 = bx * (PAIR ? 64u : (uint32_t)ROWS);
@@ -804,12 +817,13 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     const uint16_t *const biases = pick([](const GemmMat &m) { return m.biases; });
     void *const out = pick([](const GemmMat &m) { return m.out; });
     const uint32_t r0 = ga.m0.rows, r1 = ga.m1.rows, r2 = ga.m2.rows, out_rows = seg == 0 ? r0 : (seg == 1 ? r1 : r2);
-    const char *const wbase0 = (const char *)codes + (size_t)n0 * rowbytes;
-    const char *const wbase1 = PAIR ? (const char *)ga.m1.codes + (size_t)n0 * rowbytes : wbase0 + (size_t)64 * rowbytes;
-    const uint16_t *const sbase0 = scales + (size_t)n0 * G;
-    const uint16_t *const sbase1 = PAIR ? ga.m1.scales + (size_t)n0 * G : sbase0 + (size_t)64 * G;
-    const uint16_t *const bbase0 = BITS == 4 ? biases + (size_t)n0 * G : nullptr;
-    const uint16_t *const bbase1 = BITS == 4 ? (PAIR ? ga.m1.biases + (size_t)n0 * G : bbase0 + (size_t)64 * G) : nullptr;
+    const size_t wat = (size_t)n0 * rowbytes + kb / 8 * BITS, sat = (size_t)n0 * G + kb / (BITS == 1 ? 128 : 64);
+    const char *const wbase0 = (const char *)codes + wat;
+    const char *const wbase1 = PAIR ? (const char *)ga.m1.codes + wat : wbase0 + (size_t)64 * rowbytes;
+    const uint16_t *const sbase0 = scales + sat;
+    const uint16_t *const sbase1 = PAIR ? ga.m1.scales + sat : sbase0 + (size_t)64 * G;
+    const uint16_t *const bbase0 = BITS == 4 ? biases + sat : nullptr;
+    const uint16_t *const bbase1 = BITS == 4 ? (PAIR ? ga.m1.biases + sat : bbase0 + (size_t)64 * G) : nullptr;
 
     // A: lane's slot lp of rows lr + 16 u holds piece lp ^ (row & 15), so the
     // 16 rows of a fragment read hit distinct banks; rows past P re-read row
@@ -819,7 +833,7 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
 #pragma unroll
     for (int u = 0; u < A_LOADS; ++u)
         avoff[u] = (min(p0 + (uint32_t)(lr + 16 * u), ga.P - 1) - p0) * K * 2u + (uint32_t)(lp ^ (lr & 15)) * 16u;
-    const char *const abase = (const char *)(ga.A + (size_t)p0 * K);
+    const char *const abase = (const char *)(ga.A + (size_t)p0 * K + kb);
     // W chunk: 64 bytes per row as 4 pieces, piece p of row r at slot
     // p ^ ((r >> 2) & 3); instruction i fills rows 16 i .. 16 i + 15.
     const int wrow = lane >> 2;
@@ -871,7 +885,7 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[s][i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
 
-    const uint32_t nst = K / SK;
+    const uint32_t nst = (ke - kb) / SK;
     auto issue = [&](uint32_t st) __attribute__((always_inline)) {   // W before the A of its first stage
         if (st % SPC == 0) issue_w(st / SPC);
         issue_a(st);
@@ -887,12 +901,13 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
         static_assert(TPR == 2 || TPR == 4 || TPR == 8, "a row's threads are lanes of one octet");
         const int row = tid / TPR, sub = row >> 6;
         const uint16_t *const s0 = uniform_ptr(sbase0), *const s1 = uniform_ptr(sbase1);
-        const auto *const sp = (const __attribute__((address_space(1))) u32x4 *)((sub ? s1 : s0) + (size_t)(row & 63) * G);
+        const auto *const rs = (const __attribute__((address_space(1))) u32x4 *)((sub ? s1 : s0) + (size_t)(row & 63) * G);
         uint32_t mx = 0;
-        for (uint32_t p = tid % TPR; p < G / 8; p += 4 * TPR) {
-            u32x4 v[4];   // four loads in flight; past the row's end the last piece again
+        const uint32_t np = (ke - kb) / 512;   // 16-byte pieces of the row's scales
+        for (uint32_t p = tid % TPR; p < np; p += 4 * TPR) {
+            u32x4 v[4];   // four loads in flight; past the end the last piece again
 #pragma unroll
-            for (int e = 0; e < 4; ++e) v[e] = sp[min(p + (uint32_t)(e * TPR), G / 8 - 1)];
+            for (int e = 0; e < 4; ++e) v[e] = rs[min(p + (uint32_t)(e * TPR), np - 1)];
 #pragma unroll
             for (int e = 0; e < 16; ++e) mx = max(mx, max(v[e / 4][e % 4] & 0x7FFFu, (v[e / 4][e % 4] >> 16) & 0x7FFFu));
         }
@@ -1044,6 +1059,15 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
         for (int r = 0; r < 4; ++r) {
             const uint32_t p = p0 + i * 16 + 4 * q + r;
             if (p >= ga.P) continue;
+            if constexpr (SPLIT) {
+                float *const row = ga.part + ((size_t)sp * ga.P + p) * ga.cols;
+#pragma unroll
+                for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                    for (int j = 0; j < 2; ++j)
+                        row[bx * ROWS + 64 * s + 32 * wn + 16 * j + r16] = value(s, j, r);
+                continue;
+            }
 #pragma unroll
             for (int s = 0; s < (PAIR ? 1 : NSUB); ++s)
 #pragma unroll
@@ -1067,6 +1091,40 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     }
 }
 
+// Sum of the splits' partial results and the epilogue; a thread takes four
+// columns of a token (segments and sub-blocks are multiples of 64 columns).
+template <int BITS, int MODE>
+__global__ __launch_bounds__(256) void qgemm_reduce_kernel(GemmArgs ga) {
+    const uint32_t c4 = ga.cols / 4, e = blockIdx.x * 256 + threadIdx.x;
+    if (e >= ga.P * c4) return;
+    const uint32_t p = e / c4;
+    uint32_t n = e % c4 * 4;
+    const float *src = ga.part + (size_t)p * ga.cols + n;
+    const size_t stride = (size_t)ga.P * ga.cols;
+    float4v v = *(const float4v *)src;
+    for (uint32_t s = 1; s < ga.splits; ++s) v += *(const float4v *)(src + s * stride);
+    void *out = ga.m0.out;
+    uint32_t rows = ga.m0.rows;
+    if (ga.n > 1 && n >= rows) {
+        n -= rows;
+        out = ga.m1.out;
+        rows = ga.m1.rows;
+        if (ga.n > 2 && n >= rows) {
+            n -= rows;
+            out = ga.m2.out;
+            rows = ga.m2.rows;
+        }
+    }
+    const size_t o = (size_t)p * rows + n;
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        const float y = BITS == 4 ? bf16_trunc(v[r]) : v[r];
+        if constexpr (MODE == NNZ_GEMM_STORE_F16) ((f16_t *)out)[o + r] = (f16_t)y;
+        else if constexpr (MODE == NNZ_GEMM_STORE_F32) ((float *)out)[o + r] = y;
+        else ((float *)out)[o + r] += y;
+    }
+}
+
 // The forms the main kernel takes.  Others (K not a multiple of 512, other
 // group sizes, f16 scales of 4-bit weights, less aligned pointers) run on the
 // kernels above.
@@ -1081,7 +1139,27 @@ template <int BITS, int MODE, int NSUB, int KQ>
 void qgemm_start(nnz_ctx *ctx, GemmArgs ga, uint32_t rows) {
     ga.nx = rows / (MODE == NNZ_GEMM_SILU_PAIR ? 64u : 64u * NSUB);
     const uint32_t nb = ga.nx * ceil_div(ga.P, (uint32_t)BM);
-    qgemm_kernel<BITS, MODE, NSUB, KQ><<<ceil_div(nb, 8u) * 8u, 128 * KQ, 0, ctx->stream>>>(ga);
+    qgemm_kernel<BITS, MODE, NSUB, KQ, false><<<ceil_div(nb, 8u) * 8u, 128 * KQ, 0, ctx->stream>>>(ga);
+}
+
+// Whether a launch may use the context's workspace: not under capture, since
+// the graph may be replayed beside the context's own work or after its end.
+bool workspace_free(nnz_ctx *ctx) {
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    return ctx->gemm_ws && hipStreamIsCapturing(ctx->stream, &st) == hipSuccess && st == hipStreamCaptureStatusNone;
+}
+
+// The same with K split over `splits` blocks per tile, their partial sums
+// through the context's workspace (splits x blocks <= 256: it fits).
+template <int BITS, int MODE, int NSUB, int KQ>
+void qgemm_split(nnz_ctx *ctx, GemmArgs ga, uint32_t rows, uint32_t splits) {
+    ga.nx = rows / (64u * NSUB);
+    ga.part = ctx->gemm_ws;
+    ga.splits = splits;
+    ga.cols = rows;
+    const uint32_t nb = ga.nx * ceil_div(ga.P, (uint32_t)BM) * splits;
+    qgemm_kernel<BITS, MODE, NSUB, KQ, true><<<ceil_div(nb, 8u) * 8u, 128 * KQ, 0, ctx->stream>>>(ga);
+    qgemm_reduce_kernel<BITS, MODE><<<ceil_div(ga.P * (rows / 4), 256u), 256, 0, ctx->stream>>>(ga);
 }
 
 // Shape of a single-matrix launch (one or more row segments), by how many
@@ -1101,6 +1179,21 @@ template <int BITS, int MODE>
 void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128) {
     const uint32_t ny = ceil_div(ga.P, (uint32_t)BM);
     const uint32_t g = rows / 64 * ny;   // blocks of 64 rows
+    // Few blocks and a long K: split K so that up to 256 blocks run, four ways
+    // at most (8 ways: 2560 x 9728, P = 45, 18.9 us against 13.0).  Measured
+    // unsplit -> split: 1-bit P = 45 4096 x 12288 29.0 -> 15.9, 2048 x 6144 15.2
+    // -> 9.9, 4096 x 4096 11.7 -> 9.8, 2048 x 2048 7.6 -> 7.5 (not split); two
+    // ways, P = 128 4096 x 12288 32.0 -> 24.8, 4096 x 4096 13.4 -> 14.2 (not
+    // split); 4-bit P = 45 4096 x 12288 46.4 -> 20.2, 2048 x 2048 10.2 -> 8.7,
+    // P = 200 2048 x 2048 11.8 -> 12.5 (not split).  KQ = 8 from 2048 k a block
+    // (9728 / 4: 13.0 against 14.0; 6144 / 4: 10.2 against 9.9).
+    const uint32_t S = std::min(4u, 256u / std::max(g, 1u));
+    if (S >= 2 && ga.K >= (BITS == 1 ? (S == 4 ? 4096u : 6144u) : (S == 4 ? 2048u : 4096u)) && workspace_free(ctx)) {
+        if constexpr (BITS == 1) {
+            if (ga.K / S >= 2048) return qgemm_split<BITS, MODE, 1, 8>(ctx, ga, rows, S);
+        }
+        return qgemm_split<BITS, MODE, 1, 4>(ctx, ga, rows, S);
+    }
     if (g > 768) {
         if (rows128) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
         else qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
@@ -1120,7 +1213,7 @@ int qgemm_launch(nnz_ctx *ctx, const nnz_qweight *wa, const nnz_qweight *wb, con
     auto mat = [&](const nnz_qweight *w) {
         return GemmMat{w->codes, (const uint16_t *)w->scales, (const uint16_t *)w->biases, out, d.M};
     };
-    GemmArgs ga{A, mat(wa), {}, {}, 1, P, d.K, 0};
+    GemmArgs ga{A, mat(wa), {}, {}, 1, P, d.K, 0, nullptr, 1, 0};
     const bool r128 = d.M % 128 == 0;
     switch (mode) {
     case NNZ_GEMM_STORE_F16: qgemm_single<BITS, NNZ_GEMM_STORE_F16>(ctx, ga, d.M, r128); break;
@@ -1128,7 +1221,11 @@ int qgemm_launch(nnz_ctx *ctx, const nnz_qweight *wa, const nnz_qweight *wb, con
     case NNZ_GEMM_RESADD: qgemm_single<BITS, NNZ_GEMM_RESADD>(ctx, ga, d.M, r128); break;
     case NNZ_GEMM_SILU_PAIR:
         ga.m1 = mat(wb);
-        qgemm_start<BITS, NNZ_GEMM_SILU_PAIR, 2, 2>(ctx, ga, d.M);
+        // up to one block per CU: twice the waves per block (2 x 6144 x 2048, P =
+        // 45, 96 blocks: 13.0 -> 11.3 us; 2 x 12288 x 4096, 192: 27.5 -> 21.5; 2 x
+        // 9728 x 2560, P = 128, 304: 23.4 -> 28.3, KQ = 2 there)
+        if (d.M / 64 * ceil_div(P, (uint32_t)BM) <= 256) qgemm_start<BITS, NNZ_GEMM_SILU_PAIR, 2, 4>(ctx, ga, d.M);
+        else qgemm_start<BITS, NNZ_GEMM_SILU_PAIR, 2, 2>(ctx, ga, d.M);
         break;
     default: return nnz_fail(ctx, NNZ_EINVAL, "dequant_gemm: unknown mode %d", mode);
     }
@@ -1310,7 +1407,7 @@ int nnz_gemm_segments_launch(nnz_ctx *ctx, const nnz_qweight *const *w, void *co
         r128 = r128 && rows[i] % 128 == 0;
     }
     if (main_form) {
-        GemmArgs ga{(const f16_t *)a, {}, {}, {}, (uint32_t)nw, P, K, 0};
+        GemmArgs ga{(const f16_t *)a, {}, {}, {}, (uint32_t)nw, P, K, 0, nullptr, 1, 0};
         GemmMat *const m[3] = {&ga.m0, &ga.m1, &ga.m2};
         for (int i = 0; i < nw; ++i) *m[i] = GemmMat{w[i]->codes, (const uint16_t *)w[i]->scales, nullptr, out[i], rows[i]};
         qgemm_single<1, NNZ_GEMM_STORE_F16>(ctx, ga, M, r128);

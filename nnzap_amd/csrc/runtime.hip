@@ -48,6 +48,11 @@ int nnz_ctx_create(int device, void *hip_stream, nnz_ctx **out) {
         delete c;
         return rc;
     }
+    // without it the GEMMs run unsplit
+    if (hipMalloc((void **)&c->gemm_ws, NNZ_GEMM_WS_FLOATS * 4) != hipSuccess) {
+        c->gemm_ws = nullptr;
+        (void)hipGetLastError();
+    }
     *out = c;
     return NNZ_OK;
 }
@@ -58,6 +63,7 @@ int nnz_ctx_destroy(nnz_ctx *ctx) {
     hipStreamSynchronize(ctx->stream);
     for (int i = 0; i < 64; ++i)
         if (ctx->ev_ok[i]) hipEventDestroy(ctx->ev[i]);
+    if (ctx->gemm_ws) hipFree(ctx->gemm_ws);
     if (ctx->own_stream) hipStreamDestroy(ctx->stream);
     delete ctx;
     return NNZ_OK;

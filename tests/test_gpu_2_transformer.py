@@ -483,6 +483,33 @@ def test_dequant_gemm_q4_modes(dev, P, M, K, gs, sdt):
     assert_bf16_faithful(host(pair), O.silu(ra) * rb, "q4 gemm silu pair", sum_err=se_pair)
 
 
+def test_dequant_gemm_split_under_capture(dev):
+    """A launch that would split K over the context's workspace does not while
+    its stream is captured: the graph replays right between eager calls that
+    use the workspace, several times over."""
+    import ctypes as C
+    P, M, K = 45, 192, 4608
+    w = cf.q1_matrix(M, K, 128, 484, 485)
+    a16 = S.normal(486, P * K).astype(np.float16).reshape(P, K)
+    ref = a16.astype(np.float64) @ O.dequant(w).T
+    dw, ad, other = ops.DeviceQWeight(dev, w), tdev(a16), tdev(-a16)
+    eager, graphed = (torch.empty(P, M, dtype=torch.float32, device="cuda") for _ in range(2))
+    dev.call("nnz_graph_begin")
+    ops.dispatch_dequant_gemm(dev, dw, ad, graphed, L.GEMM_STORE_F32)
+    g = C.c_void_p()
+    dev.call("nnz_graph_end", C.byref(g))
+    try:
+        for _ in range(3):
+            graphed.zero_()
+            ops.dispatch_dequant_gemm(dev, dw, other, eager, L.GEMM_STORE_F32)
+            dev.call("nnz_graph_replay", g)
+            dev.sync()
+            assert_close(host(graphed), ref, rtol=1e-4, what="graph replay")
+            assert_close(host(eager), -ref, rtol=1e-4, what="eager beside the graph")
+    finally:
+        L.lib().nnz_graph_destroy(g)
+
+
 def test_gemm_row_equals_decode_qmv(dev):
     """Per-token equivalence: GEMM row p equals the decode QMV of token p."""
     M, K, P = 512, 2048, 8
@@ -499,13 +526,16 @@ def test_gemm_row_equals_decode_qmv(dev):
 
 @pytest.mark.parametrize("bits,P,M,K", [(1, 1, 64, 512), (1, 65, 192, 1536), (1, 64, 128, 4096),
                                         (1, 1030, 3136, 512), (1, 833, 3840, 512),
+                                        (1, 45, 192, 4608), (1, 7, 128, 9728), (1, 130, 2112, 6656),
+                                        (4, 45, 192, 2560), (4, 70, 4096, 4608),
                                         (4, 1, 64, 512), (4, 65, 192, 1536), (4, 64, 128, 4096),
                                         (4, 1030, 3136, 512), (4, 833, 3840, 512)])
 def test_dequant_gemm_main_shapes(dev, bits, P, M, K):
     """The main prefill GEMM at the edges of its launch shapes: one token, one
     past a token tile, one 64-row block, eight and four k-phases, two k-phases
     on 64-row blocks (rows not a multiple of 128, and up to 768 blocks) and on
-    128-row ones, one W chunk and several.  The 4-bit rows hold scales over
+    128-row ones, one W chunk and several, K split four and two ways with
+    parts of unequal length.  The 4-bit rows hold scales over
     eleven octaves, negative and zero ones among them, each row at a size of
     its own."""
     from nnzap_amd import formats as fm
@@ -529,6 +559,12 @@ def test_dequant_gemm_main_shapes(dev, bits, P, M, K):
     out16 = torch.empty(P, M, dtype=torch.float16, device="cuda")
     out32 = torch.empty(P, M, dtype=torch.float32, device="cuda")
     ops.dispatch_dequant_gemm(dev, da, ad, out32, L.GEMM_STORE_F32)
+    # residual += on zeros and the f16 store are the same sums, to the bit
+    res = torch.zeros(P, M, dtype=torch.float32, device="cuda")
+    ops.dispatch_dequant_gemm(dev, da, ad, res, L.GEMM_RESADD)
+    ops.dispatch_dequant_gemm(dev, da, ad, out16, L.GEMM_STORE_F16)
+    dev.sync()
+    assert torch.equal(res, out32) and torch.equal(out16, out32.half())
     if bits == 1:
         ops.dispatch_dequant_gemm(dev, da, ad, out16, L.GEMM_SILU_PAIR, wb=db)
         dev.sync()
