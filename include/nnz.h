@@ -135,8 +135,8 @@ int nnz_graph_replay(nnz_ctx *ctx, nnz_graph *g);
 int nnz_graph_destroy(nnz_graph *g);
 
 /* Context options (new; the reference has no counterpart).
- * NNZ_OPT_Q1_MATRIX_CORES selects the kernel of 1-bit QMVs with K = 2048 and
- * group size 128: 0 = the library's choice by shape (default), 1 = the
+ * NNZ_OPT_Q1_MATRIX_CORES selects the kernel of 1-bit QMVs with group size 128
+ * and K = 2048 (or K = 4096 or 6144, f32 in and out, one matrix): 0 = the library's choice by shape (default), 1 = the
  * block-scaled MFMA kernel wherever it applies, 2 = never it (the VALU
  * kernels).  Results agree to float32 rounding either way; a captured graph
  * keeps the kernels chosen at capture. */

@@ -1116,10 +1116,15 @@ __global__ __launch_bounds__(64 * KS) void qmv1_splitk_kernel(QmvArgs a) {
 // only, where its per-block set-up (a 64 KB fp4 table, the input's digit
 // rows) is amortised over many rows (measured, stacked config-3 pairs: 168
 // against 203 us; the 1-bit LM head, ~4.6 tiles per wave: 16.4 against
-// 14.5 us, so it stays on the VALU kernel).
-bool q1_matrix_cores_wanted(nnz_ctx *ctx, const nnz_qmv_dims &d, bool stacked) {
+// 14.5 us, so it stays on the VALU kernel).  Longer rows (K = 4096, 6144) set
+// up two or three times as much: from 7 MB of codes on (measured, a stack of
+// 2048 x 6144: 4 matrices, 6.3 MB, 10.5 against 9.7 us; 8, 11.1 against 16.4;
+// 256, 87 against 215; of 512 x 4096: 16, 4.2 MB, 9.1 against 7.7; 32, 9.4
+// against 11.9).
+bool q1_matrix_cores_wanted(nnz_ctx *ctx, const nnz_qmv_dims &d, const nnz_qmv_stack *stk) {
     if (!nnz_q1_mfma_supported(d.K, d.group_size) || ctx->q1_matrix_cores == 2) return false;
-    return ctx->q1_matrix_cores == 1 || stacked;
+    if (ctx->q1_matrix_cores == 1) return true;
+    return stk && (d.K <= 2048 || (uint64_t)d.M * (d.K / 8) * stk->count >= (7ull << 20));
 }
 
 // Blocks per matrix of a stacked launch: the caller's choice, else enough
@@ -1295,12 +1300,12 @@ int launch_qmv_ex(nnz_ctx *ctx, const nnz_qweight *const *w, const uint32_t *seg
                     "%s: norm_scale must be 16-byte aligned", name);
     }
 
-    // 1-bit rows of K = 2048, group size 128: the block-scaled MFMA kernel
-    // (qmv_mfma.hip) where the context's policy picks it.
+    // 1-bit rows of K = 2048, 4096 or 6144, group size 128: the block-scaled
+    // MFMA kernels (qmv_mfma.hip) where the context's policy picks them.
     NNZ_REQUIRE(ctx, !top2 || (EPI == EPI_STORE && NMAT == 1 && ODT == NNZ_F32 && nw == 1 && !stk),
                 NNZ_EUNSUPPORTED, "%s: top-2 partials need one f32-output matrix", name);
     if constexpr (BITS == 1 && !FAITH && !MERGE) {
-        if (!top2 && q1_matrix_cores_wanted(ctx, d, stk != nullptr) && (NMAT == 2 || nw == 1)) {
+        if (!top2 && q1_matrix_cores_wanted(ctx, d, stk) && (NMAT == 2 || nw == 1)) {
             NnzQ1Mfma c;
             for (int i = 0; i < NMAT; ++i) {
                 c.codes[i] = w[i]->codes;

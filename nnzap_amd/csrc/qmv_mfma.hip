@@ -2,7 +2,8 @@
 //
 // Same arithmetic as the 1-bit kernels of qmv.hip (qmv_specialized.metal's
 // family: y[r] = sum_g s[r,g] * sum_{c in g} (bit ? +x_c : -x_c), f32
-// accumulation), for rows of K = 2048 with group size 128, computed with one
+// accumulation), for rows of K = 2048 with group size 128 (4096 and 6144: see
+// qmv1_mfma_split_kernel), computed with one
 // v_mfma_scale_f32_16x16x128_f8f6f4 per (16 rows, 128-column group):
 //
 //   B (fp4 e2m1, 128 k x 16 columns = 16 weight rows): the group's bits, bit 1
@@ -59,6 +60,8 @@ constexpr int NS = KG / 4;     // 512-column pieces per row
 template <int NMAT>
 constexpr int threads_of() { return NMAT == 2 ? 512 : 768; }
 constexpr int PREP = KC / 8;   // threads preparing x (8 columns each)
+constexpr int XP = PREP + 4;   // dwords between digit rows in LDS
+constexpr int STG_PITCH = KC / 8 + 16;   // bytes between staged code rows
 
 enum { EPI_STORE = 0, EPI_RESADD = 1, EPI_SILU = 2 };
 enum { XIN_X = 0, XIN_NORM = 1 };
@@ -123,6 +126,48 @@ __device__ __forceinline__ v4f mfma_group(int sel, const v8i &A, const v8i &B, i
     }
 }
 
+// Digit rows of 2048 columns: NDIG signed digits per column, one scale per
+// group.  Row s of group G: d = rint(r / 2^e) with 2^e set by the group's largest
+// |r| (max |r| / 2^e in [2, 4), so |d| <= 4, every such integer exact in e2m1),
+// then r -= d 2^e (exact): |r| drops at least fourfold per row.  Thread t < PREP
+// holds columns 8t..8t+7; a group's 16 threads are one 16-lane row (the maximum
+// by DPP).  Rows NDIG..15 are zero, so every lane loads its A row
+// unconditionally.
+__device__ __forceinline__ void digit_rows(float (&r)[8], uint32_t t, uint32_t *xs4, uint8_t *sc8) {
+    const uint32_t G = t >> 4;
+#pragma unroll
+    for (int s = 0; s < NDIG; ++s) {
+        float mx = 0.f;
+#pragma unroll
+        for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(r[i]));
+        mx = fmaxf(mx, dpp_move<DPP_XOR1>(mx, 0.f));
+        mx = fmaxf(mx, dpp_move<DPP_XOR2>(mx, 0.f));
+        mx = fmaxf(mx, dpp_move<DPP_ROW_HALF_MIRROR>(mx, 0.f));
+        mx = fmaxf(mx, dpp_move<DPP_ROW_MIRROR>(mx, 0.f));
+        int e = 0;
+        if (mx > 0.f) e = max(-126, min(126, __builtin_amdgcn_frexp_expf(mx) - 2));
+        const float inv = __int_as_float((127 - e) << 23), pw = __int_as_float((127 + e) << 23);
+        float d[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            d[i] = rintf(r[i] * inv);
+            r[i] = fmaf(-d[i], pw, r[i]);
+        }
+        // digits are exact in e2m1; the first operand lands in the low nibble
+        uint32_t q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, d[0], d[1], 1.f, 0);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, d[2], d[3], 1.f, 1);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, d[4], d[5], 1.f, 2);
+        q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, d[6], d[7], 1.f, 3);
+        xs4[s * XP + t] = q;
+        if ((t & 15) == 0) sc8[s * KG + G] = (uint8_t)(127 + e);
+    }
+#pragma unroll
+    for (int s = NDIG; s < 16; ++s) {
+        xs4[s * XP + t] = 0u;
+        if ((t & 15) == 0) sc8[s * KG + G] = 127;   // 1.0: finite, the row is zero
+    }
+}
+
 template <int XDT, int NMAT, int XIN, int EPI, int ODT>
 __global__ __launch_bounds__(threads_of<NMAT>()) __attribute__((amdgpu_waves_per_eu(NMAT == 2 ? 2 : 3)))
 void qmv1_mfma_kernel(MqArgs a) {
@@ -139,17 +184,14 @@ void qmv1_mfma_kernel(MqArgs a) {
     __shared__ __align__(16) uint32_t tab[256 * 64];
     // digit rows: row s, columns 8 w .. 8 w + 7 in dword xs4[s * XP + w]
     // (nibble j = column 8 w + j); scales sc8[s * KG + G] (E8M0).
-    // (rows NDIG..15 are zero, so every lane loads its A row unconditionally)
     // The row pitch XP = PREP + 4 dwords puts row n's A reads 4 n banks
     // apart: the 16 lane rows of a 16-byte read cover the 64 banks once (a
     // pitch of PREP, a multiple of 64 banks, made that read 16-way
     // conflicted).
-    constexpr int XP = PREP + 4;
     __shared__ __align__(16) uint32_t xs4[16 * XP];
     __shared__ __align__(16) uint8_t sc8[16 * KG];
     __shared__ float red[16];
     // per-wave staging of one tile's codes: 16 rows at a 272-byte pitch
-    constexpr int STG_PITCH = KC / 8 + 16;
     __shared__ __align__(16) char stage[WAVES * 16 * STG_PITCH];
     char *const stg = stage + wid * 16 * STG_PITCH;
 
@@ -258,46 +300,7 @@ void qmv1_mfma_kernel(MqArgs a) {
         *(u32x4 *)&tab[4 * i] = u32x4{v, v, v, v};
     }
 
-    // ---- digit rows: NDIG signed digits per column, one scale per group ----
-    // Row s of group G: d = rint(r / 2^e) with 2^e set by the group's largest
-    // |r| (max |r| / 2^e in [2, 4), so |d| <= 4, every such integer exact in
-    // e2m1), then r -= d 2^e (exact): |r| drops at least fourfold per row.
-    // Thread t < PREP holds columns 8t..8t+7; a group's 16 threads are one
-    // 16-lane row (the maximum by DPP).
-    if (tid < PREP) {
-        const uint32_t G = (uint32_t)tid >> 4;
-#pragma unroll
-        for (int s = 0; s < NDIG; ++s) {
-            float mx = 0.f;
-#pragma unroll
-            for (int i = 0; i < 8; ++i) mx = fmaxf(mx, fabsf(r[i]));
-            mx = fmaxf(mx, dpp_move<DPP_XOR1>(mx, 0.f));
-            mx = fmaxf(mx, dpp_move<DPP_XOR2>(mx, 0.f));
-            mx = fmaxf(mx, dpp_move<DPP_ROW_HALF_MIRROR>(mx, 0.f));
-            mx = fmaxf(mx, dpp_move<DPP_ROW_MIRROR>(mx, 0.f));
-            int e = 0;
-            if (mx > 0.f) e = max(-126, min(126, __builtin_amdgcn_frexp_expf(mx) - 2));
-            const float inv = __int_as_float((127 - e) << 23), pw = __int_as_float((127 + e) << 23);
-            float d[8];
-#pragma unroll
-            for (int i = 0; i < 8; ++i) {
-                d[i] = rintf(r[i] * inv);
-                r[i] = fmaf(-d[i], pw, r[i]);
-            }
-            // digits are exact in e2m1; the first operand lands in the low nibble
-            uint32_t q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(0u, d[0], d[1], 1.f, 0);
-            q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, d[2], d[3], 1.f, 1);
-            q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, d[4], d[5], 1.f, 2);
-            q = __builtin_amdgcn_cvt_scalef32_pk_fp4_f32(q, d[6], d[7], 1.f, 3);
-            xs4[s * XP + tid] = q;
-            if ((tid & 15) == 0) sc8[s * KG + G] = (uint8_t)(127 + e);
-        }
-#pragma unroll
-        for (int s = NDIG; s < 16; ++s) {
-            xs4[s * XP + tid] = 0u;
-            if ((tid & 15) == 0) sc8[s * KG + G] = 127;   // 1.0: finite, the row is zero
-        }
-    }
+    if (tid < PREP) digit_rows(r, (uint32_t)tid, xs4, sc8);
     __syncthreads();
 
     // ---- A operands (digit rows) and their scales, kept for the whole kernel
@@ -425,6 +428,189 @@ void qmv1_mfma_kernel(MqArgs a) {
     static_for<PERIOD - 1>([&](auto jc) { body(jc, true); });
 }
 
+// Longer rows, K = KS * 2048 (KS = 2, 3), f32 in and out: a wave keeps the
+// digits of one 2048-column part (those of a whole row would take KS times the
+// 64 registers), 12 / KS row groups x KS parts share the block's table.  The
+// part totals of a row meet in LDS once per round of ROUND tiles per wave; the
+// barrier waits for the round's LDS writes only, so the next tiles' loads stay
+// in flight.  Two tiles of registers: a tile's codes go to the staging rows
+// first and the load of the tile after the next takes their place (three
+// spill).  256 stacked 2048 x 6144 matrices (453 MB with the scales): 215-227
+// us on the VALU split-K block, which is bound by issue, 87-90 here, 5.1 TB/s.
+constexpr int ROUND = 4;   // tiles per wave and round (even: two tiles of registers)
+
+template <int KS>
+__global__ __launch_bounds__(768) __attribute__((amdgpu_waves_per_eu(3))) void qmv1_mfma_split_kernel(MqArgs a) {
+    constexpr int THREADS = 768, WAVES = 12, RG = WAVES / KS;
+    constexpr uint32_t K = KS * KC, ROWB = K / 8, SROWB = K / 128 * 2;
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wid = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int n = lane & 15, q = lane >> 4, part = wid % KS, rg = wid / KS;
+    const uint32_t M = a.M, T = ceil_div(M, 16u);
+    __shared__ __align__(16) uint32_t tab[256 * 64];
+    // the digit rows of every part until the A operands are read, then the
+    // waves' staging rows
+    constexpr int XS = KS * 16 * XP * 4, STG = WAVES * 16 * STG_PITCH;
+    __shared__ __align__(16) char smem[XS > STG ? XS : STG];
+    __shared__ __align__(16) uint8_t sc8[KS][16 * KG];
+    __shared__ float sums[2][KS][RG * ROUND * 16];
+    char *const stg = smem + wid * 16 * STG_PITCH;
+
+    const __amdgpu_buffer_rsrc_t cr = rsrc(stk(a.codes0, a.cs)), sr = rsrc(stk(a.scales0, a.ss));
+    const float *const xp = (const float *)stk(a.x, a.xs);
+    float *const out = (float *)stk(a.out, a.os);
+    const uint32_t g0 = blockIdx.x * RG, nw = gridDim.x * RG;   // the block's first row group, all of them
+    const uint32_t gw = g0 + (uint32_t)rg;
+    const uint32_t rounds = g0 < T ? ceil_div(ceil_div(T - g0, nw), (uint32_t)ROUND) : 0u;   // block-uniform
+
+    // tile k of the wave (past the last one: the last row again)
+    auto load = [&](Tile &t, uint32_t k) {
+        const uint32_t row0 = (gw + k * nw) * 16u;
+#pragma unroll
+        for (int S = 0; S < NS; ++S) {
+            const uint32_t row = min(row0 + 4u * S + ((uint32_t)lane >> 4), M - 1u);
+            t.code[S] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                      cr, row * ROWB + ((uint32_t)lane & 15u) * 16u, part * (KC / 8), 2));
+        }
+        const uint32_t so = min(row0 + (uint32_t)n, M - 1u) * SROWB;
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+            t.scl[h] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                     sr, so + (uint32_t)h * 16u, part * (KG * 2), 2));
+    };
+    const uint32_t xt = (uint32_t)tid < K / 8 ? (uint32_t)tid : 0u;
+    const float4 x0 = ((const float4 *)xp)[2 * xt], x1 = ((const float4 *)xp)[2 * xt + 1];
+    __builtin_amdgcn_sched_barrier(0);
+    Tile ring[2];
+    load(ring[0], 0);
+    __builtin_amdgcn_sched_barrier(0);
+    for (uint32_t i = (uint32_t)tid; i < 256u * 16u; i += THREADS) {   // fp4 tables
+        const uint32_t b = i >> 4;
+        const uint32_t v = 0xAAAAAAAAu ^ ((spread4(b & 15u) | (spread4(b >> 4) << 16)) << 3);
+        *(u32x4 *)&tab[4 * i] = u32x4{v, v, v, v};
+    }
+    if ((uint32_t)tid < K / 8) {
+        float r[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
+        digit_rows(r, (uint32_t)tid % PREP, (uint32_t *)smem + tid / PREP * (16 * XP), sc8[tid / PREP]);
+    }
+    // The digits hold finite values only (no e2m1 code is an infinity or NaN):
+    // with any other x the rows are summed as they stand, a thread to a row.
+    const float xsum = (((x0.x + x0.y) + (x0.z + x0.w)) + ((x1.x + x1.y) + (x1.z + x1.w))) * 0.f;
+    if (__syncthreads_or(xsum != 0.f)) {   // 0 * finite is 0; an overflowing sum takes this path too
+        for (uint32_t row = blockIdx.x * THREADS + (uint32_t)tid; row < M; row += gridDim.x * THREADS) {
+            const uint32_t *const cw = stk(a.codes0, a.cs) + (uint64_t)row * (K / 32);
+            const uint16_t *const sw = stk(a.scales0, a.ss) + (uint64_t)row * (K / 128);
+            float y = 0.f;
+            for (uint32_t g = 0; g < K / 128; ++g) {
+                float t = 0.f;
+                for (uint32_t c = 0; c < 128; ++c) {
+                    const float v = xp[g * 128 + c];
+                    t += cw[g * 4 + c / 32] >> (c % 32) & 1u ? v : -v;
+                }
+                y = fmaf((float)__builtin_bit_cast(f16_t, sw[g]), t, y);
+            }
+            out[row] = y;
+        }
+        return;
+    }
+    v4i A[KG];
+    uint32_t sa[KG / 4];
+    {
+        const uint32_t *const xs4 = (const uint32_t *)smem + part * (16 * XP);
+#pragma unroll
+        for (int G = 0; G < KG; ++G) A[G] = __builtin_bit_cast(v4i, *(const u32x4 *)&xs4[n * XP + G * 16 + 4 * q]);
+        const u32x4 sv = *(const u32x4 *)&sc8[part][n * KG];
+        sa[0] = sv.x; sa[1] = sv.y; sa[2] = sv.z; sa[3] = sv.w;
+    }
+    __syncthreads();   // the digit rows become staging
+    load(ring[1], 1);
+    __builtin_amdgcn_sched_barrier(0);
+    const uint32_t lane4 = (uint32_t)lane * 4u;
+    const char *const tb8 = (const char *)tab;
+    // tile k, whose registers then take tile k + 2
+    auto tile_total = [&](Tile &t, uint32_t k) {
+        float acc = 0.f;
+        // the tile's codes into this wave's staging rows (272-byte pitch),
+        // then lane (n, g) reads word g of each group of row n: banks
+        // 4n + 4G + g, all distinct for a read (LDS keeps a wave's order)
+#pragma unroll
+        for (int S = 0; S < NS; ++S)
+            *(u32x4 *)(stg + (4 * S + (lane >> 4)) * STG_PITCH + 16 * (lane & 15)) = t.code[S];
+        const u32x4 scl[2] = {t.scl[0], t.scl[1]};
+        load(t, k + 2);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int S = 0; S < NS; ++S) {
+            uint32_t w[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) w[i] = *(const uint32_t *)(stg + n * STG_PITCH + 16 * (4 * S + i) + 4 * q);
+            // the piece's 16 table reads first (one LDS round trip for four
+            // groups), then its four independent MFMAs, then their sums
+            uint32_t b4[4][4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int bb = 0; bb < 4; ++bb) {
+                    // address = byte bb of the word * 256 + lane * 4
+                    const uint32_t off = __builtin_amdgcn_perm(w[i], lane4, 0x0C0C0000u | ((4u + bb) << 8));
+                    b4[i][bb] = *(const uint32_t *)(tb8 + off);
+                }
+            v4f c[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int G = 4 * S + i;
+                const v8i B = v8i{(int)b4[i][0], (int)b4[i][1], (int)b4[i][2], (int)b4[i][3], 0, 0, 0, 0};
+                const v8i A8 = v8i{A[G][0], A[G][1], A[G][2], A[G][3], 0, 0, 0, 0};
+                c[i] = mfma_group(i, A8, B, (int)sa[G >> 2]);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int G = 4 * S + i;
+                const float tsum = (c[i][0] + c[i][1]) + (c[i][2] + c[i][3]);
+                const uint32_t sw = scl[G >> 3][(G >> 1) & 3];
+                const float sc = (float)__builtin_bit_cast(f16_t, (uint16_t)((G & 1) ? (sw >> 16) : (sw & 0xFFFFu)));
+                acc = fmaf(sc, tsum, acc);
+            }
+            asm volatile("" : "+v"(acc));   // these sums before the next piece: four C tiles live, not 16
+        }
+        // digit rows 4r..4r+3 sit in lane row r: sum the four lane rows (the
+        // swaps' two results are the lower and the upper half or row of each
+        // pair in every lane, so all four lane rows end with the total)
+        const auto hf = __builtin_amdgcn_permlane32_swap(__float_as_int(acc), __float_as_int(acc), false, false);
+        const int t1 = __float_as_int(__int_as_float((int)hf[0]) + __int_as_float((int)hf[1]));
+        const auto rw = __builtin_amdgcn_permlane16_swap(t1, t1, false, false);
+        return __int_as_float((int)rw[0]) + __int_as_float((int)rw[1]);
+    };
+
+    for (uint32_t rd = 0; rd < rounds; ++rd) {
+#pragma unroll 1
+        for (uint32_t h = 0; h < ROUND; h += 2)
+            static_for<2>([&](auto jc) {
+                constexpr int J = decltype(jc)::value;
+                const uint32_t k = rd * ROUND + h + J;
+                if (gw + k * nw < T) {   // wave-uniform
+                    const float tot = tile_total(ring[J], k);
+                    sums[rd & 1][part][((h + J) * RG + rg) * 16 + n] = tot;   // the same from the four lane rows
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        // this wave's LDS writes, then the barrier; loads stay in flight
+        __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        // entry e: row e % 16 of tile g0 + e / 16 % RG + (rd ROUND + e / 16 / RG) nw
+        if (tid < RG * ROUND * 16) {
+            const uint32_t u = (uint32_t)tid >> 4;
+            const uint32_t row = (g0 + u % RG + (rd * ROUND + u / RG) * nw) * 16u + ((uint32_t)tid & 15u);
+            float t = sums[rd & 1][0][tid];
+#pragma unroll
+            for (int p = 1; p < KS; ++p) t += sums[rd & 1][p][tid];
+            if (row < M) out[row] = t;
+        }
+    }
+}
+
 template <int XDT, int NMAT, int XIN, int EPI, int ODT>
 void launch(nnz_ctx *ctx, const MqArgs &a, uint32_t blocks, uint32_t gy) {
     qmv1_mfma_kernel<XDT, NMAT, XIN, EPI, ODT><<<dim3(blocks, gy), threads_of<NMAT>(), 0, ctx->stream>>>(a);
@@ -433,7 +619,7 @@ void launch(nnz_ctx *ctx, const MqArgs &a, uint32_t blocks, uint32_t gy) {
 }  // namespace
 
 bool nnz_q1_mfma_supported(uint32_t K, uint32_t group_size) {
-    return K == (uint32_t)KC && group_size == 128;
+    return (K == KC || K == 2 * KC || K == 3 * KC) && group_size == 128;
 }
 
 // The variants built below (x dtype, pair, input mode, epilogue, output dtype).
@@ -443,6 +629,8 @@ bool nnz_q1_mfma_has_variant(const NnzQ1Mfma &c) {
         {NNZ_F32, 1, XIN_X, EPI_STORE, NNZ_F32},     {NNZ_F16, 1, XIN_X, EPI_STORE, NNZ_F32},
         {NNZ_F32, 1, XIN_NORM, EPI_STORE, NNZ_F32},  {NNZ_F32, 2, XIN_X, EPI_SILU, NNZ_F32},
         {NNZ_F32, 2, XIN_NORM, EPI_SILU, NNZ_F16},   {NNZ_F16, 1, XIN_X, EPI_RESADD, NNZ_F32}};
+    if (c.K != KC)   // longer rows: the f32 store only
+        return c.xdt == NNZ_F32 && c.nmat == 1 && c.xin == XIN_X && c.epi == EPI_STORE && c.odt == NNZ_F32;
     for (const auto &b : built)
         if (b[0] == k[0] && b[1] == k[1] && b[2] == k[2] && b[3] == k[3] && b[4] == k[4]) return true;
     return false;
@@ -450,9 +638,9 @@ bool nnz_q1_mfma_has_variant(const NnzQ1Mfma &c) {
 
 int nnz_q1_mfma_launch(nnz_ctx *ctx, const NnzQ1Mfma &c) {
     NNZ_REQUIRE(ctx, nnz_q1_mfma_supported(c.K, c.group_size), NNZ_EUNSUPPORTED,
-                "q1_mfma: K=%u gs=%u (needs K=%d, gs=128)", c.K, c.group_size, KC);
+                "q1_mfma: K=%u gs=%u (needs K=2048, 4096 or 6144, gs=128)", c.K, c.group_size);
     NNZ_REQUIRE(ctx, c.M >= 1 && (c.nmat == 1 || c.nmat == 2), NNZ_EINVAL, "q1_mfma: bad shape");
-    NNZ_REQUIRE(ctx, (uint64_t)c.M * (KC / 8) < (1ull << 32), NNZ_EUNSUPPORTED,
+    NNZ_REQUIRE(ctx, (uint64_t)c.M * (c.K / 8) < (1ull << 32), NNZ_EUNSUPPORTED,
                 "q1_mfma: matrix of 4 GiB or more");
     MqArgs a{};
     a.codes0 = (const uint32_t *)c.codes[0];
@@ -470,6 +658,14 @@ int nnz_q1_mfma_launch(nnz_ctx *ctx, const NnzQ1Mfma &c) {
     // per lane), about 256 blocks in all, never more than one wave per tile
     const uint32_t gy = c.stack_count ? c.stack_count : 1u;
     uint32_t blocks = c.blocks_per_matrix ? c.blocks_per_matrix : ceil_div(256u, gy);
+    if (c.K != KC) {
+        const uint32_t parts = c.K / KC;
+        blocks = max(1u, min(blocks, ceil_div(tiles, 12u / parts)));
+        if (parts == 2) qmv1_mfma_split_kernel<2><<<dim3(blocks, gy), 768, 0, ctx->stream>>>(a);
+        else qmv1_mfma_split_kernel<3><<<dim3(blocks, gy), 768, 0, ctx->stream>>>(a);
+        NNZ_LAUNCHED(ctx);
+        return NNZ_OK;
+    }
     blocks = min(blocks, ceil_div(tiles, (uint32_t)(c.nmat == 2 ? threads_of<2>() : threads_of<1>()) / 64u));
     blocks = max(blocks, 1u);
 #define MQ(XDT, NMAT, XIN, EPI, ODT)                                                           \

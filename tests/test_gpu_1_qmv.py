@@ -518,6 +518,53 @@ def test_q1_matrix_cores_qmv(dev, q1_cores, M):
     _near_valu(a, b, f"f16in M={M}")
 
 
+@pytest.mark.parametrize("K", [4096, 6144])
+@pytest.mark.parametrize("M", [1, 65, 2048, 20011])
+def test_q1_matrix_cores_long_rows(dev, q1_cores, M, K):
+    """Rows of two and three 2048-column parts (f32 in and out): partial
+    tiles, blocks with one round and with several (20011 rows over 256
+    blocks), the oracle within 1e-3 and the VALU kernel within float32
+    rounding; the error against float64 is that of one rounding per group
+    and part, below 2^-20 of the largest output."""
+    w = cf.q1_matrix(M, K, 128, 720 + M % 97, 721)
+    x = S.normal(722, K).astype(np.float32)
+    x[::5] *= 1e-4   # digits of small columns beside large ones
+    dw, xd = _dw(dev, w), tdev(x)
+
+    def run():
+        y = torch.full((M,), float("nan"), device="cuda")
+        ops.dispatch_qmv(dev, dw, xd, y)
+        dev.sync()
+        return y
+    a, b = _cores_pair(dev, q1_cores, run)
+    ref = O.qmv(w, x)
+    assert_close(host(a), ref, what=f"M={M} K={K}")
+    _near_valu(a, b, f"M={M} K={K}")
+    err = np.max(np.abs(host(a).astype(np.float64) - ref)) / np.max(np.abs(ref))
+    assert err <= 2.0 ** -20, f"M={M} K={K}: {err:.2e} of max |y|"
+
+
+def test_q1_matrix_cores_long_rows_nonfinite(dev, q1_cores):
+    """An infinity or NaN in x reaches the outputs (the digit rows cannot hold
+    one), and only those of its own matrix in a stacked launch."""
+    q1_cores(1)
+    M, K, n = 100, 6144, 4
+    sw = ops.StackedQWeights(dev, M, K, 128, 1, n, 12, (0.01, 0.05))
+    x = torch.randn(n, K, device="cuda", generator=torch.Generator("cuda").manual_seed(15))
+    x[1, 4099] = float("inf")
+    x[2, 7] = float("nan")
+    y = torch.full((n, M), float("nan"), device="cuda")
+    ops.dispatch_qmv_stacked(dev, sw, x, y, 3)
+    dev.sync()
+    y = host(y)
+    for i in (0, 3):
+        assert_close(y[i], O.qmv(sw.host(i), x[i].cpu().numpy()), what=f"matrix {i}")
+    w = sw.host(1)
+    bits = (w.codes.view(np.uint8).reshape(M, K // 8)[:, 4099 // 8] >> (4099 % 8)) & 1
+    assert np.array_equal(y[1], np.where(bits == 1, np.inf, -np.inf))
+    assert np.isnan(y[2]).all()
+
+
 @pytest.mark.parametrize("M", [6144, 151936])
 def test_q1_matrix_cores_norm_lm_head(dev, q1_cores, M):
     """Final RMSNorm + LM head (f16-rounded normalised input, f32 logits) on
