@@ -5,7 +5,8 @@
 // (:3969-3972, Zig std.Random.DefaultPrng).
 //
 // The reference copies the 151k logits to the host and sorts them there.
-// Here the logits never leave HBM; two launches per draw:
+// Here the logits never leave HBM; two launches per draw (top-k of up to 64 out
+// of up to 2^20 logits: sample_maxima_kernel and sample_topk_kernel below):
 //   * selection kernel: one 256-thread block per 1024 logits writes its
 //     maximum scaled logit and its sum of exp(x - max) and, when a filter
 //     needs candidates, every element >= its k-th largest (8-bit radix select
@@ -415,6 +416,7 @@ struct FinSh {
     uint32_t koff[MAX_BLOCKS + 1];
     float wx[64];       // survivors of top-k for the one-wave finish
     uint32_t wi[64];
+    float wq[64];
     float r, prob, cum0;
     uint32_t tok, aux, fallback;
 };
@@ -519,75 +521,75 @@ __device__ __forceinline__ void finish_temperature(const FinishArgs &a, FinSh &S
     __syncthreads();
 }
 
-__device__ __forceinline__ float lane_f(float v, uint32_t j) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), (int)j));
-}
 __device__ __forceinline__ uint32_t lane_u(uint32_t v, uint32_t j) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)j);
+}
+
+// One wave's LDS accesses take effect in program order; this keeps the
+// compiler from moving them.
+__device__ __forceinline__ void wave_lds_fence() {
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+}
+
+constexpr int DPP_WAVE_SHR1 = 0x138;   // lane l takes lane l - 1's value, lane 0 zero
+
+// f(j, lane j's value of v) for j < n, in order and in steps of eight: the
+// lanes from n on have to hold what f ignores.
+template <class F>
+__device__ __forceinline__ void each_lane(uint32_t v, uint32_t n, F f) {
+    for (uint32_t j0 = 0; j0 < n; j0 += 8)
+#pragma unroll
+        for (uint32_t j = 0; j < 8; ++j) f(j0 + j, lane_u(v, j0 + j));
+}
+
+// Sums of lanes 0 .. l in that order, for every lane l < n (zero from n on;
+// the total is lane n - 1's): each step adds a lane to the sum of the lane
+// below it, so lane l has its value after l steps and keeps it.
+__device__ __forceinline__ float ordered_sums(float v, uint32_t n) {
+    float c = v;
+    for (uint32_t j = 1; j < n; j += 8)
+#pragma unroll
+        for (int i = 0; i < 8; ++i)
+            c = v + __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(c), DPP_WAVE_SHR1, 0xF, 0xF, true));
+    return c;
 }
 
 // At most 64 survivors (index order) in S.wx / S.wi, finished by one wave
 // (threads 0..63) with the reference's sequential float32 sums: the top-p
 // softmax (over the survivors, or s_topp > 0: the sum over every logit) and
 // its cumulative walk in descending-probability order (ties by index), the
-// final softmax and the inverse-CDF walk in index order.  Sequential steps
-// read lanes with v_readlane (uniform lane index).
+// final softmax and the inverse-CDF walk in index order.
 __device__ __forceinline__ void finish_wave(const FinishArgs &a, FinSh &S, uint32_t nk, float M,
                                             float s_topp) {
     const uint32_t l = threadIdx.x;
     const bool v = l < nk;
     const float e = v ? expf(S.wx[l] - M) : 0.f;
-    unsigned long long keep = nk >= 64 ? ~0ull : ((1ull << nk) - 1ull);
+    bool keep = v;
     if (a.top_p < 1.0f) {
         float s = s_topp;
-        if (s <= 0.f) {
-            s = 0.f;
-            for (uint32_t j = 0; j < nk; ++j) s += lane_f(e, j);
-        }
+        if (s <= 0.f) s = __uint_as_float(lane_u(__float_as_uint(ordered_sums(e, nk)), nk - 1));
         const float q = e * (1.0f / s);
-        // bitonic sort, ascending on (~q bits, lane): q descending, ties by index
-        unsigned long long key =
-            v ? ((unsigned long long)(~__float_as_uint(q)) << 32) | l : ~0ull;
-        for (uint32_t k = 2; k <= 64; k <<= 1)
-            for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-                const unsigned long long o = __shfl_xor(key, (int)j);
-                const bool take_min = ((l & j) == 0) == ((l & k) == 0);
-                key = take_min ? (key < o ? key : o) : (key > o ? key : o);
-            }
-        const uint32_t src = (uint32_t)(key & 0xFFFFFFFFull) & 63u;  // lane holding the r-th
-        const float qs = __shfl(q, (int)src);
-        float c = 0.f;
-        uint32_t cut = nk - 1;
-        for (uint32_t r = 0; r < nk; ++r) {
-            c += lane_f(qs, r);
-            if (c >= a.top_p) {
-                cut = r;
-                break;
-            }
-        }
-        keep = 0;
-        for (uint32_t r = 0; r <= cut; ++r) keep |= 1ull << lane_u(src, r);
+        // order: q descending (bits, q >= 0), ties by index.  A lane's rank is
+        // the number of survivors before it: nk lane reads, against the 21
+        // dependent exchanges of a 64-lane sort.
+        const uint32_t qb = __float_as_uint(q);
+        uint32_t rank = 0;
+        each_lane(qb, nk, [&](uint32_t j, uint32_t o) { rank += o > qb || (o == qb && j < l); });
+        if (v) S.wq[rank] = q;
+        wave_lds_fence();
+        const float at = ordered_sums(v ? S.wq[l] : 0.f, nk);
+        const unsigned long long over = __ballot(v && at >= a.top_p);
+        const uint32_t cut = over ? (uint32_t)__builtin_ctzll(over) : nk - 1;
+        keep = v && rank <= cut;
     }
-    float s1 = 0.f;
-    for (uint32_t j = 0; j < nk; ++j)
-        if ((keep >> j) & 1ull) s1 += lane_f(e, j);
-    const float p = ((keep >> l) & 1ull) ? e * (1.0f / s1) : 0.f;
-    float c = 0.f;
-    uint32_t tok = 0xFFFFFFFFu;
-    float tp = 0.f;
-    const float r = S.r;
-    for (uint32_t j = 0; j < nk; ++j) {
-        const float pj = lane_f(p, j);
-        c += pj;
-        if (c > r) {
-            tok = j;
-            tp = pj;
-            break;
-        }
-    }
-    if (l == 0 && tok != 0xFFFFFFFFu) {
-        S.tok = S.wi[tok];
-        S.prob = tp;
+    const float s1 = __uint_as_float(lane_u(__float_as_uint(ordered_sums(keep ? e : 0.f, nk)), nk - 1));
+    const float p = keep ? e * (1.0f / s1) : 0.f;
+    const float at = ordered_sums(p, nk);
+    const unsigned long long over = __ballot(v && at > S.r);
+    if (over && l == (uint32_t)__builtin_ctzll(over)) {
+        S.tok = S.wi[l];
+        S.prob = p;
     }
 }
 
@@ -936,6 +938,17 @@ __device__ __forceinline__ void finish_general(const FinishArgs &a, FinSh &S, ui
     __syncthreads();
 }
 
+// The draw's result, by one thread.
+__device__ __forceinline__ void sample_output(const FinishArgs &a, const FinSh &S) {
+    // rounding tail: the reference returns the last index (probs.len - 1)
+    const uint32_t tok = S.tok;
+    const uint32_t out = tok == 0xFFFFFFFFu ? a.n - 1 : tok;
+    const float pr = tok == 0xFFFFFFFFu ? 0.f : S.prob;
+    if (a.out_index) a.out_index[0] = out;
+    if (a.out_prob) a.out_prob[0] = pr;
+    if (a.pick.state) nnz_pick_advance(a.pick, out, pr);
+}
+
 __global__ __launch_bounds__(1024) void sample_finish_kernel(FinishArgs a) {
     __shared__ FinSh S;
     const uint32_t tid = threadIdx.x;
@@ -1008,15 +1021,186 @@ __global__ __launch_bounds__(1024) void sample_finish_kernel(FinishArgs a) {
             }
         }
     }
-    if (tid == 0) {
-        // rounding tail: the reference returns the last index (probs.len - 1)
-        const uint32_t tok = S.tok;
-        const uint32_t out = tok == 0xFFFFFFFFu ? a.n - 1 : tok;
-        const float pr = tok == 0xFFFFFFFFu ? 0.f : S.prob;
-        if (a.out_index) a.out_index[0] = out;
-        if (a.out_prob) a.out_prob[0] = pr;
-        if (a.pick.state) nnz_pick_advance(a.pick, out, pr);
+    if (tid == 0) sample_output(a, S);
+}
+
+// ---- few candidates kept (top-k up to TOPK_FEW) -----------------------------
+//
+// The k-th largest logit is at least the k-th largest of any k or more pieces'
+// maxima: with a threshold under which k maxima lie, only the pieces whose
+// maximum reaches it (about k of them) can hold the top-k set, and about k of
+// their logits reach it too.  So the first kernel writes one maximum per piece
+// and no lists, and the finishing block reads the maxima and some k pieces.
+// Both kernels are bound by their chains of dependent steps (loads, LDS round
+// trips, one block's barriers), not by bandwidth.  Top-20 of 151669 logits:
+// 2.8 + 10.0 us, against 7.1 + 19.7 with the lists (11-bit radix selects in
+// every selection block and over all 2980 candidates in the finishing one);
+// top-1 9.9 us together, top-64 25.1.
+constexpr uint32_t TOPK_FEW = 64;      // survivors one wave finishes
+constexpr uint32_t PIECES = 1024;      // at most: 16 maxima per lane of one wave
+constexpr uint32_t SURV = 1024;        // logits over the threshold held in LDS
+
+// Largest key of each piece of `len` logits (256 times a power of two), a wave
+// to a piece.
+__global__ __launch_bounds__(256) void sample_maxima_kernel(const float *logits, uint32_t n, float inv_t,
+                                                            uint32_t len, uint32_t np, uint32_t *maxima) {
+    const uint32_t piece = blockIdx.x * 4 + (threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (piece >= np) return;
+    uint32_t m = 0;
+    for (uint32_t o = piece * len; o < piece * len + len; o += 256)
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t i = o + 64 * j + lane;
+            if (i < n) m = max(m, fkey(logits[i] * inv_t));
+        }
+    for (int o = 32; o > 0; o >>= 1) m = max(m, (uint32_t)__shfl_xor(m, o));
+    if (lane == 0) maxima[piece] = m;
+}
+
+// Survivors S.sx / S.si (n <= 64, any order): those of the k largest (ties
+// included) into S.wx / S.wi in index order, then finish_wave; one wave.
+__device__ __forceinline__ void finish_few(const FinishArgs &a, FinSh &S, const float *sx, const uint32_t *si,
+                                           uint32_t n) {
+    const uint32_t l = threadIdx.x;
+    const bool v = l < n;
+    const float x = v ? sx[l] : -INFINITY;
+    const uint32_t id = v ? si[l] : 0xFFFFFFFFu, key = v ? fkey(x) : 0u;
+    uint32_t above = 0;
+    each_lane(key, n, [&](uint32_t, uint32_t o) { above += o > key; });
+    const bool kept = v && above < a.k;
+    uint32_t pos = 0;
+    const uint32_t kid = kept ? id : 0xFFFFFFFFu;
+    each_lane(kid, n, [&](uint32_t, uint32_t o) { pos += o < id; });
+    if (kept) {
+        S.wx[pos] = x;
+        S.wi[pos] = id;
     }
+    wave_lds_fence();
+    finish_wave(a, S, (uint32_t)__popcll(__ballot(kept)), wave_max(x), 0.f);
+}
+
+__global__ __launch_bounds__(1024) void sample_topk_kernel(FinishArgs a, const uint32_t *maxima, uint32_t len,
+                                                           uint32_t np) {
+    __shared__ FinSh S;
+    __shared__ float sx[SURV];
+    __shared__ uint32_t si[SURV];
+    __shared__ uint32_t thr, nf, ns;
+    uint32_t *const list = S.koff;   // pieces over the threshold, in index order
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    if (w == 0) {
+        uint32_t key[PIECES / 64];
+#pragma unroll
+        for (uint32_t i = 0; i < PIECES / 64; ++i) key[i] = 64 * i + lane < np ? maxima[64 * i + lane] : 0u;
+        if (lane == 0) ns = 0;
+        // the largest threshold that k maxima reach, bit by bit; a smaller one
+        // that only few more reach does as well
+        uint32_t t = 0;
+        for (int b = 31; b >= 0; --b) {
+            const uint32_t c = t | (1u << b);
+            uint32_t cnt = 0;
+#pragma unroll
+            for (uint32_t i = 0; i < PIECES / 64; ++i) cnt += (uint32_t)__popcll(__ballot(key[i] >= c));
+            if (cnt >= a.k) t = c;
+            if (cnt >= a.k && cnt <= a.k + 2) break;
+        }
+        uint32_t base = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < PIECES / 64; ++i) {
+            const bool in = key[i] >= t && 64 * i + lane < np;
+            const unsigned long long bal = __ballot(in);
+            if (in) list[base + __popcll(bal & ((1ull << lane) - 1ull))] = 64 * i + lane;
+            base += (uint32_t)__popcll(bal);
+        }
+        if (lane == 0) {
+            thr = t;
+            nf = base;
+        }
+    } else if (tid == 64) {
+        uint64_t st[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) st[j] = a.rng[j];
+        S.r = zig_float32(st);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) a.rng[j] = st[j];
+        S.tok = 0xFFFFFFFFu;
+        S.prob = 0.f;
+    }
+    __syncthreads();
+    const uint32_t t = thr, pieces = nf, per = len >> 8;   // 256 logits to a wave's step
+    // f(x, i) for every logit of the pieces
+    auto each_piece = [&](auto f) {
+        for (uint32_t c = w; c < pieces * per; c += FT / 64) {
+            const uint32_t o = list[c / per] * len + (c % per) * 256 + lane;
+            float x[4];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) x[j] = o + 64 * j < a.n ? a.logits[o + 64 * j] * a.inv_t : 0.f;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if (o + 64 * j < a.n) f(x[j], o + 64 * j);
+        }
+    };
+    auto collect = [&](uint32_t least) {
+        each_piece([&](float x, uint32_t i) {
+            if (fkey(x) < least) return;
+            const uint32_t pos = atomicAdd(&ns, 1u);
+            if (pos < SURV) {
+                sx[pos] = x;
+                si[pos] = i;
+            }
+        });
+    };
+    // that many pieces are ties among the maxima: more of them than a wave takes
+    const bool tied = pieces > 2 * TOPK_FEW;
+    if (!tied) collect(t);
+    __syncthreads();
+    uint32_t n = tied ? pieces : ns;
+    if (n > TOPK_FEW && !tied) {   // block-uniform: the exact k-th largest, and only what reaches it
+        const bool v = tid < n;
+        const float x = v && n <= SURV ? sx[tid] : 0.f;
+        const uint32_t id = v && n <= SURV ? si[tid] : 0u;
+        const uint32_t kmin = radix_kth_largest<FT, FIN_W>(
+            [&](auto f) {
+                if (n > SURV) each_piece([&](float y, uint32_t) { f(fkey(y)); });
+                else if (v) f(fkey(x));
+            },
+            a.k, S.hist, S.R);
+        if (tid == 0) ns = 0;
+        __syncthreads();
+        if (n > SURV) {
+            collect(kmin);
+        } else if (v && fkey(x) >= kmin) {
+            const uint32_t pos = atomicAdd(&ns, 1u);
+            sx[pos] = x;
+            si[pos] = id;
+        }
+        __syncthreads();
+        n = ns;
+    }
+    if (n <= TOPK_FEW) {
+        if (w == 0) finish_few(a, S, sx, si, n);
+    } else {
+        // many ties at the k-th largest: the pieces (or every logit), which
+        // hold all that the threshold lets pass
+        const uint32_t sh = (uint32_t)__builtin_ctz(len);
+        if (pieces == np)
+            finish_general(
+                a, S, a.n,
+                [&](uint32_t i, float &x, uint32_t &idx) {
+                    x = a.logits[i] * a.inv_t;
+                    idx = i;
+                },
+                true, 0.f);
+        else
+            finish_general(
+                a, S, pieces * len,
+                [&](uint32_t e, float &x, uint32_t &idx) {
+                    idx = list[e >> sh] * len + (e & (len - 1));
+                    x = idx < a.n ? a.logits[idx] * a.inv_t : -INFINITY;
+                },
+                true, 0.f);
+    }
+    __syncthreads();
+    if (tid == 0) sample_output(a, S);
 }
 
 // Zig std.Random.SplitMix64.next, used by Xoshiro256.init to expand the seed.
@@ -1107,6 +1291,22 @@ int nnz_sample_launch(nnz_ctx *ctx, const float *logits, uint32_t n, const nnz_s
         a.mode = MODE_TEMP;
     }
     a.kc = kc;
+    // Few kept of many: piece maxima.  At least 2 k pieces, so that the pieces
+    // over the threshold are a fraction of the logits (top-20 of 10240 logits,
+    // 40 pieces: 12.3 against 23.7 us a draw with the lists); pieces of at most
+    // 1024 logits, as one block reads k of them (top-20 / top-64 of 1M: 17 / 34
+    // against 37 / 43 us; of 4M, pieces of 4096: 79 / 145 against 63 / 68 or more).
+    uint32_t len = 256;   // logits per piece
+    while (ceil_div(n, len) > PIECES) len *= 2;
+    const uint32_t np = ceil_div(n, len);
+    if (a.mode == MODE_TOPK && a.k <= TOPK_FEW && np >= 2 * a.k && len <= 1024) {
+        uint32_t *const maxima = (uint32_t *)(w + L.cx);   // the lists' space
+        sample_maxima_kernel<<<ceil_div(np, 4u), 256, 0, ctx->stream>>>(logits, n, inv_t, len, np, maxima);
+        NNZ_LAUNCHED(ctx);
+        sample_topk_kernel<<<1, FT, 0, ctx->stream>>>(a, maxima, len, np);
+        NNZ_LAUNCHED(ctx);
+        return NNZ_OK;
+    }
     sample_select_kernel<<<nb, 256, 0, ctx->stream>>>(
         logits, n, inv_t, kc, (float *)(w + L.blk_max), (float *)(w + L.blk_sum),
         (uint32_t *)(w + L.blk_cnt), (uint32_t *)(w + L.blk_kth), (float *)(w + L.cx),

@@ -122,6 +122,62 @@ def test_sample_matches_oracle(sdev, V, T, k, p, kind, draws):
     assert _state(rng) == prng.s
 
 
+FEW = [
+    # (vocab, top_k, top_p, kind): the piece maxima take over at 2 k pieces
+    (10240, 20, 0.95, "normal"),       # 40 pieces of 256: the smallest for k = 20
+    (10239, 20, 0.95, "normal"),       # ragged last piece
+    (9984, 20, 0.95, "normal"),        # 39 pieces: the lists
+    (32768, 64, 1.0, "normal"),        # 64 kept, the most one wave finishes
+    (151669, 1, 1.0, "normal"),
+    (151669, 20, 0.95, "clustered"),   # 200 of the largest in one piece
+    (151669, 20, 0.95, "ordered"),     # whole pieces over the threshold
+    (151669, 20, 0.9, "ties"),
+    (151669, 20, 0.95, "equal"),
+    (151669, 20, 0.95, "masked"),      # ten finite logits, the rest -inf
+    (262144, 40, 0.95, "normal"),      # 1024 pieces of 256
+    (262145, 40, 0.95, "clustered"),   # pieces of 512
+    (1048576, 40, 0.95, "ordered"),    # 1024 pieces of 1024, the longest
+    (1048577, 40, 0.95, "normal"),     # the lists
+]
+
+
+@pytest.mark.parametrize("V,k,p,kind", FEW)
+def test_sample_few_kept(sdev, V, k, p, kind):
+    """Top-k draws from piece maxima: every route of the finishing block (one
+    wave at once, after an exact k-th largest, over the pieces), piece lengths
+    and the smallest count that takes it, against the oracle."""
+    x = _logits(V, V, kind)
+    if kind == "clustered":
+        x[5000:5200] += 14.0
+    elif kind == "ordered":
+        x = -np.sort(-x)
+    elif kind == "equal":
+        x[:] = 1.5
+    elif kind == "masked":
+        x[np.random.default_rng(5).permutation(V)[10:]] = -np.inf
+    draws = 8
+    ws, rng, out, prob = _buffers(V, draws)
+    logits = torch.from_numpy(x).cuda()
+    ops.rng_seed(sdev, V + k, rng)
+    print(f"sample V={V} k={k} p={p} {kind}", flush=True)
+    for i in range(draws):
+        ops.dispatch_sample(sdev, logits, out[i:i + 1], rng, ws, 0.6, k, p, out_prob=prob[i:i + 1])
+    sdev.sync()
+    got, gp = out.cpu().numpy(), prob.cpu().numpy()
+    prng = SM.ZigPrng(V + k)
+    tol = SM.summation_tolerance(V)
+    if kind == "equal":   # the oracle's V additions of one value to a sum below 1 may all
+        tol = V * 2.0 ** -25   # round the same way, by up to 2^-25 each
+    for i in range(draws):
+        d = SM.sample_token(x, 0.6, k, p, prng)
+        if d.margin >= tol:
+            assert got[i] == d.token, (i, got[i], d.token, d.margin)
+            assert abs(gp[i] - d.prob) <= 1e-4 * max(d.prob, 1e-3) + 1e-6, (i, gp[i], d.prob)
+        else:
+            assert d.within(int(got[i]), tol + 2 * d.q_cut), (i, got[i], d.token, d.margin)
+    assert _state(rng) == prng.s
+
+
 def test_sample_distribution(sdev):
     V, T, k, p, n = 40, 0.9, 12, 0.85, 6000
     x = _logits(V, 3, "normal")
