@@ -1428,7 +1428,26 @@ int launch_qmv_ex(nnz_ctx *ctx, const nnz_qweight *const *w, const uint32_t *seg
     // that over several row-steps per wave (measured: the normalised gate/up
     // pair at 512 blocks instead of 768, 4.37 -> 3.81 us; the plain pair and
     // single matrices do best uncapped up to 2048 / 1024).
-    const uint32_t max_blocks = NORM ? (NMAT == 2 ? 512u : 1024u) : 2048u;
+    uint32_t max_blocks = NORM ? (NMAT == 2 ? 512u : 1024u) : 2048u;
+    if (NORM && lut && nv <= 2) {
+        // Every block builds its tables (32 KB, 64 KB for K > 2048), so no more
+        // blocks than the chip holds at once: three per CU (by registers), two
+        // with 64 KB.  LM heads, 1024 blocks -> these: 151669 x 2560 26.5 -> 23.3
+        // us, x 4096 29.4 -> 24.9 (768 blocks: 31), 32000 x 4096 13.4 -> 10.8,
+        // 70001 x 2048 10.0 -> 9.4.  Rows too few to give each wave of 512 blocks
+        // a step of four: one block per CU (Q/K/V of 6144 rows, 384 -> 256
+        // blocks: K = 4096 6.0 -> 5.2 us, 512 in two-row steps 5.6; K = 2560 5.13
+        // -> 5.05).
+        if (NMAT == 1 && nv == 2 && R >= 4) max_blocks = d.M <= 4u * 4u * 512u ? 256u : 512u;
+        if (NMAT == 1 && nv == 1 && R == 8) max_blocks = 768u;
+        // a pair's 2048 waves: two-row steps where they come out as fewer rows
+        // (9728 x 2560: three steps of two against two of four, 7.4 -> 6.6 us;
+        // 12288 x 4096 8.3 either way)
+        if (NMAT == 2 && nv == 2 && R == 4 && blocks > max_blocks && ceil_div(d.M, 4096u) * 2 < ceil_div(d.M, 8192u) * 4) {
+            R = 2;
+            blocks = ceil_div(d.M, 4u * R * rpw);
+        }
+    }
     if (blocks > max_blocks) blocks = max_blocks;
     if (MERGE) {
         // every block re-reads all partials: fewer, fuller blocks

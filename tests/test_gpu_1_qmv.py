@@ -218,6 +218,41 @@ def test_norm_lm_head_vocabulary_rows_ragged(dev):
     assert_close(host(y), O.qmv(w, O.norm_to_half(res, nw)), what="vocabulary rows")
 
 
+@pytest.mark.parametrize("M,K", [(4097, 2560), (8192, 4096), (8193, 4096), (65536 + 13, 2560), (9728, 2560), (8200, 4096)])
+def test_fused_norm_long_rows_grids(dev, M, K):
+    """Norm + QMV and norm + gate/up of K > 2048 around the lines of the grid
+    rule: one or two blocks per CU, several steps per wave, two-row steps of a
+    pair, ragged last steps."""
+    wa, wb = cf.q1_matrix(M, K, 128, 394, 395), cf.q1_matrix(M, K, 128, 396, 397)
+    res = S.normal(398, K).astype(np.float32)
+    nw = (1.0 + 0.1 * S.normal(399, K)).astype(np.float32)
+    xn = O.norm_to_half(res, nw)
+    a, b, rd, nd = _dw(dev, wa), _dw(dev, wb), tdev(res), tdev(nw)
+    y = torch.full((M,), float("nan"), dtype=torch.float32, device="cuda")
+    h = torch.full((M,), float("nan"), dtype=torch.float16, device="cuda")
+    ops.dispatch_fused_norm_qmv_f16in(dev, a, rd, y, nd)
+    ops.dispatch_fused_norm_pair_silu_f16io(dev, a, b, rd, h, nd)
+    dev.sync()
+    ya = O.qmv(wa, xn)
+    assert_close(host(y), ya, what="norm qmv")
+    assert_close(host(h), _f16(O.qmv_pair_silu(wa, wb, xn)), what="norm pair silu")
+
+
+@pytest.mark.parametrize("qrows,kvrows,K", [(4096, 1024, 4096), (4096, 1024, 2560), (8192, 64, 4096)])
+def test_fused_norm_qkv_long_rows(dev, qrows, kvrows, K):
+    """Norm + Q/K/V of K > 2048: fewer blocks than steps, segments met in one
+    wave's successive steps."""
+    w = [cf.q1_matrix(m, K, 128, 400 + i, 410 + i) for i, m in enumerate((qrows, kvrows, kvrows))]
+    res = S.normal(420, K).astype(np.float32)
+    nw = (1.0 + 0.1 * S.normal(421, K)).astype(np.float32)
+    xn = O.norm_to_half(res, nw)
+    out = [torch.full((x.M,), float("nan"), dtype=torch.float16, device="cuda") for x in w]
+    ops.dispatch_fused_norm_qkv_f16io(dev, *[_dw(dev, x) for x in w], tdev(res), *out, tdev(nw))
+    dev.sync()
+    for x, y in zip(w, out):
+        assert_close(host(y), _f16(O.qmv(x, xn)), what="qkv")
+
+
 @pytest.mark.parametrize("M", [6145, 5, 1])
 def test_q4_qmv_ragged_rows(dev, M):
     """4-bit QMV on an f32 input (two rows per wave step) with row counts
