@@ -1109,18 +1109,22 @@ __global__ __launch_bounds__(256) void attn_fused_wave_kernel(FusedAttnArgs a) {
 //     so that lane group g's eight B slots are eight consecutive keys and a
 //     lane's V operand is one 16-byte load of its dim's row.
 //   * q is normalised and rotated by the wave w + 4 n of head w + 4 n (lane l
-//     on dims 2l, 2l + 1, a RoPE pair), scaled by log2(e) / sqrt(D) and split
-//     into f16 hi + lo like the probabilities: with both products accumulated
-//     the scores carry 2^-22 and P.V 2^-20 relative error, below the f16
-//     rounding of the attention output.
+//     on dims 2l, 2l + 1, a RoPE pair) and scaled by log2(e) / sqrt(D).  Its
+//     24 bits go into three f16 parts, and so do the probabilities': scaled by
+//     a power of two first (q by one that its largest possible value, from the
+//     norm weights, allows; p by 2^15), so that the last parts stay above the
+//     smallest f16 and the three products add up to the float32 ones.  Error
+//     of the merged partials against float64, three parts / float32 on the VALU
+//     / two parts: 16 query heads, 1500 tokens 2.1e-7 / 2.3e-7 / 3.1e-7; 32,
+//     3001 2.4e-7 / 2.3e-7 / 3.2e-7 (the third parts cost 0.35-0.4 us).
 //   * The block whose chunk holds position seq - 1 normalises, rotates and
 //     f16-rounds the new key (wave 3), appends it and the value to the caches
 //     and puts both into their lanes' operands.
 // Bound by one memory round trip, the launch and the chain between the two
 // barriers.  Against the VALU kernel with six barriers that ran these shapes
 // (with its merge, which had one block per head): 32 query and 8 KV heads, 1500
-// tokens 14.3 -> 7.1 us, 3001 23.8 -> 8.1, 8192 57.2 -> 11.5; 16 query heads,
-// 1000 tokens 9.9 -> 6.7, 4096 26.6 -> 8.5.
+// tokens 14.8 -> 8.0 us, 3001 23.9 -> 8.3, 8192 57.4 -> 11.4; 16 query heads,
+// 1025 tokens 10.5 -> 7.4, 4096 26.8 -> 8.9.
 template <int GM, int KW>
 __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     typedef _Float16 half8 __attribute__((ext_vector_type(8)));
@@ -1129,7 +1133,8 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     constexpr int D = 128, CH = 4 * KW, NT = KW / 16, NK = KW >= 32 ? KW / 32 : 1, NH = (GM + 3) / 4;
     constexpr int QP = D + 8;   // LDS pitch (halves) of a query part
-    __shared__ __align__(16) _Float16 qs[GM][2][QP];
+    constexpr float PSC = 0x1p15f;   // of the probabilities' f16 parts
+    __shared__ __align__(16) _Float16 qs[GM][3][QP];
     __shared__ __align__(16) _Float16 knew[D];
     __shared__ uint16_t vnew[D];
     __shared__ __align__(16) float osh[4][GM][D];
@@ -1199,6 +1204,11 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     const float freq = a.inv_freq ? freq_t : rope_inv_freq(lane, D, a.theta);
     float sn, cs;
     sincosf((float)pos * freq, &sn, &cs);
+    // |normalised q| <= sqrt(D), a rotated pair at most sqrt(2) times its
+    // larger part: |q| log2(e) / sqrt(D) < 2.05 max |q_norm|, times 2^qexp
+    // below 2^15.04
+    const int qexp = min(14 - __builtin_amdgcn_frexp_expf(wave_max(fmaxf(fabsf(qn2.x), fabsf(qn2.y)))), 100);
+    const float sl = __builtin_ldexpf(a.scale * 1.44269504088896341f, qexp);
 #pragma unroll
     for (int n = 0; n < NH; ++n) {
         const int hh = w + 4 * n;
@@ -1206,15 +1216,16 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
         unpack2<NNZ_F16>(qpair[n], q0, q1);
         const float r = rsqrtf(wave_sum(fmaf(q1, q1, q0 * q0)) / (float)D + a.eps);
         const float x0 = q0 * r * qn2.x, x1 = q1 * r * qn2.y;
-        const float sl = a.scale * 1.44269504088896341f;
-        const float qe = fmaf(x0, cs, -x1 * sn) * sl, qo = fmaf(x0, sn, x1 * cs) * sl;
-        const f16_t he = (f16_t)qe, ho = (f16_t)qo;
+        float qe = fmaf(x0, cs, -x1 * sn) * sl, qo = fmaf(x0, sn, x1 * cs) * sl;
         if (hh < GM) {
-            *(uint32_t *)&qs[hh][0][2 * lane] =
-                (uint32_t)__builtin_bit_cast(uint16_t, he) | (uint32_t)__builtin_bit_cast(uint16_t, ho) << 16;
-            *(uint32_t *)&qs[hh][1][2 * lane] =
-                (uint32_t)__builtin_bit_cast(uint16_t, (f16_t)(qe - (float)he)) |
-                (uint32_t)__builtin_bit_cast(uint16_t, (f16_t)(qo - (float)ho)) << 16;
+#pragma unroll
+            for (int i = 0; i < 3; ++i) {
+                const f16_t he = (f16_t)qe, ho = (f16_t)qo;
+                *(uint32_t *)&qs[hh][i][2 * lane] =
+                    (uint32_t)__builtin_bit_cast(uint16_t, he) | (uint32_t)__builtin_bit_cast(uint16_t, ho) << 16;
+                qe -= (float)he;
+                qo -= (float)ho;
+            }
         }
     }
     if (own && w == 3) {
@@ -1236,17 +1247,17 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     __syncthreads();
 
     // ---- S^T = K . Q^T (log2 units)
-    half8 qh[4], ql[4];
+    half8 qf[3][4];
     {
         const bool live = (uint32_t)c16 < heads;
         const int hc = c16 < GM ? c16 : 0;
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) {
-            const half8 zero = {};
-            const half8 hi = *(const half8 *)&qs[hc][0][32 * ks + 8 * g], lo = *(const half8 *)&qs[hc][1][32 * ks + 8 * g];
-            qh[ks] = live ? hi : zero;
-            ql[ks] = live ? lo : zero;
-        }
+        for (int i = 0; i < 3; ++i)
+#pragma unroll
+            for (int ks = 0; ks < 4; ++ks) {
+                const half8 zero = {}, v = *(const half8 *)&qs[hc][i][32 * ks + 8 * g];
+                qf[i][ks] = live ? v : zero;
+            }
     }
     if (wnew) {
 #pragma unroll
@@ -1262,13 +1273,18 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     float4v s[NT];
 #pragma unroll
     for (int t = 0; t < NT; ++t) {
+        float4v lo = {0.f, 0.f, 0.f, 0.f};
         s[t] = (float4v){0.f, 0.f, 0.f, 0.f};
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const half8 ka = __builtin_bit_cast(half8, kreg[t][ks]);
-            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qh[ks], s[t], 0, 0, 0);
-            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, ql[ks], s[t], 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[2][ks], lo, 0, 0, 0);
+            s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[0][ks], s[t], 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[1][ks], lo, 0, 0, 0);
         }
+        const float unit = __builtin_ldexpf(1.f, -qexp);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) s[t][r] = (s[t][r] + lo[r]) * unit;
     }
     // ---- softmax of head c16 over the wave's tokens
     const bool tail = wt0 + KW > seq;   // wave-uniform
@@ -1299,7 +1315,7 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     l += __shfl_xor(l, 32);
 
     // P^T: slot 8 g + e is the wave's key 32 kk + 8 g + e (KW 16: 4 g + e, e < 4)
-    half8 ph[NK], pl[NK];
+    half8 pf[3][NK];
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk)
 #pragma unroll
@@ -1308,13 +1324,15 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
             for (int r = 0; r < 4; r += 2) {
                 const int t = KW >= 32 ? 2 * kk + sb : 0;
                 const bool z = KW < 32 && sb == 1;
-                const float p0 = z ? 0.f : s[t][r], p1 = z ? 0.f : s[t][r + 1];
-                const auto hi = __builtin_amdgcn_cvt_pkrtz(p0, p1);
-                const auto lo = __builtin_amdgcn_cvt_pkrtz(p0 - (float)hi[0], p1 - (float)hi[1]);
-                ph[kk][4 * sb + r] = hi[0];
-                ph[kk][4 * sb + r + 1] = hi[1];
-                pl[kk][4 * sb + r] = lo[0];
-                pl[kk][4 * sb + r + 1] = lo[1];
+                float p0 = z ? 0.f : s[t][r] * PSC, p1 = z ? 0.f : s[t][r + 1] * PSC;
+#pragma unroll
+                for (int i = 0; i < 3; ++i) {
+                    const auto v = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+                    pf[i][kk][4 * sb + r] = v[0];
+                    pf[i][kk][4 * sb + r + 1] = v[1];
+                    p0 -= (float)v[0];
+                    p1 -= (float)v[1];
+                }
             }
     if (tail || wnew) {
         // tokens past the length: value 0 (the weight is 0 too; never NaN *
@@ -1345,8 +1363,8 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk) {
             const half8 va = __builtin_bit_cast(half8, vreg[kk][dt]);
-            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, ph[kk], o, 0, 0, 0);
-            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pl[kk], o, 0, 0, 0);
+#pragma unroll
+            for (int i = 2; i >= 0; --i) o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pf[i][kk], o, 0, 0, 0);
         }
         if (c16 < GM) *(float4v *)&osh[w][c16][16 * dt + 4 * g] = o;
     }
@@ -1369,8 +1387,8 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
             const float wgt = __builtin_amdgcn_exp2f(ml[i].x - M);   // M is finite: token t0 is live
             const float2 o = *(const float2 *)&osh[i][hh][2 * lane];
             lsum = fmaf(wgt, ml[i].y, lsum);
-            r0 = fmaf(wgt, o.x, r0);
-            r1 = fmaf(wgt, o.y, r1);
+            r0 = fmaf(wgt * (1.f / PSC), o.x, r0);
+            r1 = fmaf(wgt * (1.f / PSC), o.y, r1);
         }
         const uint32_t qh_ = qh0 + (uint32_t)hh;
         if (a.direct) {
@@ -1379,9 +1397,13 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
                 (uint32_t)__builtin_bit_cast(uint16_t, he) | ((uint32_t)__builtin_bit_cast(uint16_t, ho) << 16);
         } else {
             // dims 2l, 2l + 1: adjacent in either layout (8-byte aligned);
-            // the maximum in natural units, as the merges take it
-            *(float2 *)(a.part_o + part_o_at(a, qh_, c, 2u * lane, D)) = make_float2(r0, r1);
-            if (lane == 0) ((float2 *)a.part_ml)[part_ml_at(a, qh_, c, D)] = make_float2(M * 0.693147180559945309f, lsum);
+            // the maximum in natural units, as the merges take it, and what
+            // its rounding leaves out (M - Mn log2(e), log2(e) in two parts)
+            // as a factor of the sums
+            const float Mn = M * 0.693147180559945309f;
+            const float f = __builtin_amdgcn_exp2f(fmaf(-Mn, 1.92596299e-8f, fmaf(-Mn, 1.44269502f, M)));
+            *(float2 *)(a.part_o + part_o_at(a, qh_, c, 2u * lane, D)) = make_float2(r0 * f, r1 * f);
+            if (lane == 0) ((float2 *)a.part_ml)[part_ml_at(a, qh_, c, D)] = make_float2(Mn, lsum * f);
         }
     }
 }
@@ -2385,7 +2407,7 @@ int nnz_attn_launch(nnz_ctx *ctx, const void *q, int qdt, const void *kc, const 
 // query head).  Measured, the attention launch alone, wave / MFMA kernel: 16
 // query and 8 KV heads, 100 tokens 3.52 / 3.96 us, 640 4.02 / 4.29, 1000 4.17 /
 // 4.20; 32 query heads, 200 tokens (128 blocks) 3.65 / 4.13, 640 (320 blocks)
-// 4.85 / 4.37.
+// 4.85 / 4.37 (the MFMA kernel before its third f16 parts, now 0.35 more).
 static bool attn_fused_by_wave(uint32_t chunks, uint32_t hq) { return chunks * hq <= 256; }
 
 // Chunk length (tokens per partial) of the fused decode attention: 64 while
@@ -2393,7 +2415,8 @@ static bool attn_fused_by_wave(uint32_t chunks, uint32_t hq) { return chunks * h
 // runs, 128 beyond -- half the partials: 32 query and 8 KV heads, attention
 // and merge together, 3001 tokens 9.2 -> 8.1 us, 8192 13.9 -> 11.5; 1500 tokens
 // 7.1 -> 7.5, but then its 12 chunks need no merge launch in the decode step.
-// (256-token chunks, 64 per wave: 10.9 us at 3001, 12.5 at 8192.)
+// (256-token chunks, 64 per wave: 10.9 us at 3001, 12.5 at 8192; all of these
+// before the third f16 parts, which cost every length 0.35-0.4 us.)
 uint32_t nnz_attn_fused_chunk(uint32_t max_seq, uint32_t hq, uint32_t head_dim) {
     const uint32_t n64 = ceil_div(max_seq, (uint32_t)FCHUNK);
     if (head_dim != 128 || n64 <= NNZ_O_MERGE_MAX_CHUNKS || attn_fused_by_wave(n64, hq)) return (uint32_t)FCHUNK;

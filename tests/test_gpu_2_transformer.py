@@ -187,6 +187,51 @@ def test_gqa_fused_1pass_kernels(dev, hq, hkv, seq, ctx):
     assert np.isnan(host(kcd)[:, seq:]).all() and np.isnan(host(vcd)[:, :, seq:]).all()
 
 
+@pytest.mark.parametrize("form,qscale,kscale", [("plain", 1.0, 1.0), ("small norms", 2.0 ** -10, 2.0 ** 10),
+                                                ("large norms", 2.0 ** 20, 2.0 ** -17), ("sink", 1.0, 1.0)])
+def test_attention_partials_precision(dev, form, qscale, kscale):
+    """The matrix-core decode attention holds float32 queries and weights: its
+    float32 partials (288 blocks: 16 heads x 18 chunks), merged here in float64,
+    against the oracle.  Norm weights far from 1 against keys that bring the
+    scores back to size (16-bit parts of q would lose their last bits, or
+    overflow), and a sink: one token without a value takes the weight, the rest
+    (2^-20 of it each) is what is left to see.
+
+    Tolerance, relative in the 2-norm: 1e-5.  The scores (up to 14) are float32
+    sums, a few 14 2^-24 = 8e-7 off, which is their weights' relative error;
+    the weights are kept to 2^-40 of the largest, 2^-20 of the sink's others."""
+    hq, hkv, d, seq, theta, ctx = 16, 8, 128, 1100, 1e6, 1104
+    pos = seq - 1
+    rng = np.random.default_rng(2201)
+    qn = (qscale * (1 + 0.1 * rng.standard_normal(d))).astype(np.float32)
+    kn = (kscale * (1 + 0.1 * rng.standard_normal(d))).astype(np.float32)
+    kc = np.zeros((hkv, ctx, d), np.float16)
+    vc = np.zeros((hkv, d, ctx), np.float16)
+    kc[:, :pos] = kscale * rng.standard_normal((hkv, pos, d))
+    vc[:, :, :pos] = rng.standard_normal((hkv, d, pos))
+    q = rng.standard_normal((hkv, 1, d)).repeat(hq // hkv, 1).reshape(hq, d).astype(np.float16)
+    kr, vr = (rng.standard_normal((hkv, d)).astype(np.float16) for _ in range(2))
+    if form == "sink":
+        kc[:, 0] = 1.25 * O.head_norm_rope(q.astype(np.float64), qn, pos, theta)[::hq // hkv]
+        vc[:, :, 0] = 0.0
+    n = ops.gqa_partial_chunks(seq)
+    part_o = torch.empty(n, hq * d, dtype=torch.float32, device="cuda")
+    part_ml = torch.empty(n, hq, 2, dtype=torch.float32, device="cuda")
+    dims = L.GQAFusedDims(hq, hkv, d, seq, ctx, hq // hkv, pos, 1e-6, theta)
+    ops.dispatch_gqa_attention_partials(dev, tdev(q), tdev(kc), tdev(vc), tdev(kr), tdev(vr), tdev(qn), tdev(kn),
+                                        part_o, part_ml, dims, rope_inv_freq=tdev(O.rope_inv_freq(d, theta)))
+    dev.sync()
+    k = np.arange(hq * d)
+    at = ((k >> 2) & 7) * (hq * d // 8) + (k >> 5) * 4 + (k & 3)   # unit-major columns
+    o, ml = host(part_o)[:, at].reshape(n, hq, d), host(part_ml)
+    w = np.exp(ml[..., 0] - ml[..., 0].max(0))
+    got = (w[..., None] * o).sum(0) / (w * ml[..., 1]).sum(0)[..., None]
+    ref = O.gqa_fused_step(q.astype(np.float64), kr.astype(np.float64), vr.astype(np.float64),
+                           kc[:, :seq].astype(np.float64), vc[:, :, :seq].astype(np.float64), qn, kn, pos, theta)
+    e = np.linalg.norm(got - ref) / np.linalg.norm(ref)
+    assert e <= 1e-5, f"{form}: relative error {e:.2e}"
+
+
 @pytest.mark.parametrize("pos", [30, 700, 1023])
 @pytest.mark.parametrize("freq_table", [False, True])
 @pytest.mark.parametrize("hq,hkv", [(16, 8), (24, 12)])
