@@ -178,6 +178,90 @@ def test_sample_few_kept(sdev, V, k, p, kind):
     assert _state(rng) == prng.s
 
 
+CROWDED = [
+    # (vocab, top_k, top_p, kind): more logits over the maxima's threshold than LDS holds, or more
+    # ties at the k-th largest than a wave finishes
+    (33000, 64, 0.9, "hump"),         # the threshold from around the largest logit
+    (300000, 50, 1.0, "hump"),        # pieces of 512: one of two windows
+    (33005, 20, 0.95, "tail"),        # the largest in the last piece, which is shorter than k
+    (33000, 64, 0.95, "coarse"),      # 65..1024 survivors, finished in LDS in index order
+    (151669, 50, 0.95, "coarse"),
+    (33000, 40, 0.95, "teeth"),       # no window's threshold narrows it to 1024: exact k-th largest
+    (151669, 50, 0.95, "plateau"),    # more than 1024 ties at the k-th largest, below a few larger
+]
+
+
+def _crowded(V, kind):
+    x = _logits(V, V, "normal")
+    i = np.arange(V)
+    if kind == "hump":
+        x = (8.0 - np.abs(i - V // 3) / 1000.0).astype(np.float32)
+    elif kind == "tail":
+        x[-3:] += 30.0
+        x[1000:4000] += 15.0
+    elif kind == "coarse":
+        x = np.round(x / 2.5).astype(np.float32)
+    elif kind == "teeth":
+        x = (8.0 - (i % 256) / 64.0 - i / 1e5).astype(np.float32)
+    elif kind == "plateau":
+        x[2000:6000] = 14.0
+        x[7000:7005] = 14.5
+    return x
+
+
+@pytest.mark.parametrize("V,k,p,kind", CROWDED)
+def test_sample_few_kept_crowded(sdev, V, k, p, kind):
+    """Top-k draws from piece maxima where the pieces over the threshold are full
+    of logits that reach it, against the oracle."""
+    x = _crowded(V, kind)
+    draws = 8
+    ws, rng, out, prob = _buffers(V, draws)
+    logits = torch.from_numpy(x).cuda()
+    ops.rng_seed(sdev, V + k, rng)
+    print(f"sample V={V} k={k} p={p} {kind}", flush=True)
+    for i in range(draws):
+        ops.dispatch_sample(sdev, logits, out[i:i + 1], rng, ws, 0.6, k, p, out_prob=prob[i:i + 1])
+    sdev.sync()
+    got, gp = out.cpu().numpy(), prob.cpu().numpy()
+    prng = SM.ZigPrng(V + k)
+    tol = SM.summation_tolerance(V)
+    if kind == "plateau":   # 4000 equal terms added to a sum below 1, each rounding the same way by up to 2^-25
+        tol = max(tol, 4000 * 2.0 ** -25)
+    for i in range(draws):
+        d = SM.sample_token(x, 0.6, k, p, prng)
+        if d.margin >= tol:
+            assert got[i] == d.token, (i, got[i], d.token, d.margin)
+            assert abs(gp[i] - d.prob) <= 1e-4 * max(d.prob, 1e-3) + 1e-6, (i, gp[i], d.prob)
+        else:
+            assert d.within(int(got[i]), tol + 2 * d.q_cut), (i, got[i], d.token, d.margin)
+    assert _state(rng) == prng.s
+
+
+@pytest.mark.parametrize("kind", ["hump", "coarse"])
+def test_sample_few_kept_crowded_time(sdev, kind):
+    """Neighbouring or tied large logits cost a draw no multiple of what scattered
+    ones do (top-64 of 33000: 20 us scattered, 28 to 34 crowded; 89 to 97 where
+    the finishing block went through every logit of the pieces)."""
+    V = 33000
+    ws, rng, out, _ = _buffers(V, 1)
+    ops.rng_seed(sdev, 1, rng)
+
+    def time_us(x):
+        logits = torch.from_numpy(x).cuda()
+        torch.cuda.synchronize()
+        best = []
+        for _ in range(5):
+            sdev.mark(0)
+            for _ in range(40):
+                ops.dispatch_sample(sdev, logits, out, rng, ws, 0.6, 64, 1.0)
+            sdev.mark(1)
+            sdev.sync()
+            best.append(sdev.elapsed_ms(0, 1) * 1e3 / 40)
+        return min(best)
+
+    assert time_us(_crowded(V, kind)) <= 2.5 * time_us(_logits(V, V, "normal"))
+
+
 def test_sample_distribution(sdev):
     V, T, k, p, n = 40, 0.9, 12, 0.85, 6000
     x = _logits(V, 3, "normal")
