@@ -760,6 +760,17 @@ struct GemmArgs {
     uint32_t splits, cols;
 };
 
+// LDS of a block, and the blocks that the shape rules below count on per CU.
+template <int BITS, int NSUB, int KQ>
+constexpr size_t qgemm_lds() {
+    constexpr int cpb = KQ > (BITS == 1 ? 8 : 2) ? KQ / (BITS == 1 ? 8 : 2) : 1;
+    return 2 * (size_t)(BM * BK * KQ) * 2 + 2 * (size_t)cpb * (64 * NSUB) * (64 + 8) + (BITS == 4 ? 4 * 64 * NSUB : 4);
+}
+constexpr size_t LDS_CU = 160 * 1024;
+static_assert(qgemm_lds<1, 1, 8>() <= LDS_CU && 2 * qgemm_lds<1, 1, 4>() <= LDS_CU && 3 * qgemm_lds<1, 2, 2>() <= LDS_CU &&
+              qgemm_lds<4, 2, 4>() <= LDS_CU && 2 * qgemm_lds<4, 1, 4>() > LDS_CU && 3 * qgemm_lds<4, 2, 2>() <= LDS_CU,
+              "blocks per CU");
+
 template <int BITS, int MODE, int NSUB, int KQ, bool SPLIT>
 __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     constexpr bool PAIR = MODE == NNZ_GEMM_SILU_PAIR;
@@ -773,6 +784,7 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     __shared__ __attribute__((aligned(16))) uint32_t Wc[2][CPS][ROWS * 16];
     __shared__ uint32_t Sc[2][CPS][ROWS * 2];
     __shared__ int rowexp[BITS == 4 ? ROWS : 1];
+    static_assert(sizeof(As) + sizeof(Wc) + sizeof(Sc) + sizeof(rowexp) == qgemm_lds<BITS, NSUB, KQ>(), "the shape rules' LDS");
 
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1163,15 +1175,20 @@ void qgemm_split(nnz_ctx *ctx, GemmArgs ga, uint32_t rows, uint32_t splits) {
 }
 
 // Shape of a single-matrix launch (one or more row segments), by how many
-// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (50 / 42 KB of LDS), 2
-// of KQ = 4 (75 KB), one of KQ = 8 (140 KB).  More than one round of 768
+// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (42 KB of LDS, 128 rows
+// 51), of KQ = 4 two 1-bit ones (75 KB) or one 4-bit one (84 KB), one of KQ = 8
+// (140 KB).  More than one round of 768
 // KQ = 2 blocks: 128-row blocks, half the A traffic (2560 x 4096, P = 3001: 68
 // us against 76 with 64 rows; 6144 x 2560: 91 against 108; 4096 x 2048, P =
-// 1024: 23.5 against 26.6).  512 < g <= 768: one round of KQ = 2 64-row blocks
+// 1024: 23.5 against 26.6).  Up to 768, from 512 (1-bit) or 256 (4-bit), where
+// KQ = 4 takes a second round: one round of KQ = 2 64-row blocks
 // (2048 x 2048, P = 1500: 19.3 us against 21.4 with 128 rows and 23.7 on KQ =
-// 4, which takes a second round; 6144 x 2560, P = 512: 22.6 against 25.1 and
-// 25.0).  Fewer: KQ = 4, more waves per block (2048 x 6144, P = 1024: 33.5
-// against 38.5 on KQ = 2; 2048 x 2048, P = 512: 9.7 against 10.2).  At most one
+// 4; 6144 x 2560, P = 512: 22.6 against 25.1 and 25.0; 4-bit 4096 x 2560, P =
+// 400: 21.7 against 26.3 on KQ = 4, 2560 x 9728, P = 512: 65.8 against 79.7,
+// 2048 x 2048, P = 1024: 18.1 against 22.1).  Fewer: KQ = 4, more waves per
+// block (2048 x 6144, P = 1024: 33.5
+// against 38.5 on KQ = 2; 2048 x 2048, P = 512: 9.7 against 10.2; 4-bit 2048 x
+// 6144, P = 512: 29.2 against 41.9).  At most one
 // block per CU and K > 2048: KQ = 8 (1-bit; 2048 x 6144, P = 512: 21.7 against
 // 25.4 on KQ = 4; at K = 2048 KQ = 4 is ahead, 9.7 against 10.3; the 4-bit
 // stages of KQ = 8 do not fit LDS).
@@ -1197,7 +1214,7 @@ void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128)
     if (g > 768) {
         if (rows128) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
         else qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
-    } else if (g > 512) {
+    } else if (g > (BITS == 1 ? 512u : 256u)) {
         qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
     } else {
         if constexpr (BITS == 1) {
