@@ -10,7 +10,8 @@
 //   * qgemm_kernel, the main one: the presets' weights (1-bit of group size
 //     128, 4-bit of group size 64 with bf16 scales) with K a multiple of 512;
 //   * dq_gemm_kernel (1-bit) and dq4_gemm_kernel (4-bit): every other K and
-//     group size, f16 scales of 4-bit weights, less aligned pointers.
+//     group size, f16 scales of 4-bit weights, less aligned pointers, short
+//     1-bit launches (qgemm_short).
 // In all of them a block owns 64 tokens, its waves are 2 W-row halves x KQ
 // k-phases (a W fragment expanded in registers feeds 4 MFMAs, an A fragment
 // read from LDS feeds 2 or 4, the KQ partial tiles meet in LDS at the end), A
@@ -1147,6 +1148,19 @@ bool qgemm_weight_ok(const nnz_qweight *w, uint32_t K) {
                                ((uintptr_t)w->biases & 3) == 0);
 }
 
+// A single 1-bit launch of K <= 2048 and at most one block per CU (of K = 512,
+// two) stays on dq_gemm_kernel: too few stages for the main kernel's longer
+// first loads.  Measured, dq_gemm_kernel / main: 4096 x 2048, P = 200 (256
+// blocks) 8.75 / 9.88 us, P = 320 (320) 12.86 / 12.15; 2048 x 2048, P = 400
+// (224) 8.47 / 9.23, P = 512 (256) 9.27 / 9.54, P = 640 (320) 12.85 / 12.01;
+// 2048 x 1024, P = 400 5.96 / 6.44, P = 640 8.36 / 8.35; 2048 x 512, P = 1024
+// (512) 6.54 / 6.75.  (The one size seen ahead below the line: 1024 x 2048, P =
+// 1024, 9.47 / 8.99.)
+bool qgemm_short(uint32_t rows, uint32_t P, uint32_t K) {
+    const uint32_t g = rows / 64 * ceil_div(P, (uint32_t)BM);
+    return K <= 2048 && g <= (K <= 512 ? 512u : 256u);
+}
+
 template <int BITS, int MODE, int NSUB, int KQ>
 void qgemm_start(nnz_ctx *ctx, GemmArgs ga, uint32_t rows) {
     ga.nx = rows / (MODE == NNZ_GEMM_SILU_PAIR ? 64u : 64u * NSUB);
@@ -1187,11 +1201,10 @@ void qgemm_split(nnz_ctx *ctx, GemmArgs ga, uint32_t rows, uint32_t splits) {
 // 400: 21.7 against 26.3 on KQ = 4, 2560 x 9728, P = 512: 65.8 against 79.7,
 // 2048 x 2048, P = 1024: 18.1 against 22.1).  Fewer: KQ = 4, more waves per
 // block (2048 x 6144, P = 1024: 33.5
-// against 38.5 on KQ = 2; 2048 x 2048, P = 512: 9.7 against 10.2; 4-bit 2048 x
-// 6144, P = 512: 29.2 against 41.9).  At most one
-// block per CU and K > 2048: KQ = 8 (1-bit; 2048 x 6144, P = 512: 21.7 against
-// 25.4 on KQ = 4; at K = 2048 KQ = 4 is ahead, 9.7 against 10.3; the 4-bit
-// stages of KQ = 8 do not fit LDS).
+// against 38.5 on KQ = 2; 4-bit 2048 x 6144, P = 512: 29.2 against 41.9).  At
+// most one block per CU: KQ = 8 (1-bit of K > 2048, see qgemm_short; 2048 x
+// 6144, P = 512: 21.7 against 25.4 on KQ = 4; the 4-bit stages of KQ = 8 do not
+// fit LDS).
 template <int BITS, int MODE>
 void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128) {
     const uint32_t ny = ceil_div(ga.P, (uint32_t)BM);
@@ -1218,7 +1231,7 @@ void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128)
         qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
     } else {
         if constexpr (BITS == 1) {
-            if (g <= 256 && ga.K > 2048) return qgemm_start<BITS, MODE, 1, 8>(ctx, ga, rows);
+            if (g <= 256) return qgemm_start<BITS, MODE, 1, 8>(ctx, ga, rows);
         }
         qgemm_start<BITS, MODE, 1, 4>(ctx, ga, rows);
     }
@@ -1370,7 +1383,7 @@ int nnz_gemm_launch(nnz_ctx *ctx, const nnz_qweight *wa, const nnz_qweight *wb, 
     }
     NNZ_REQUIRE(ctx, (d.group_size & (d.group_size - 1)) == 0, NNZ_EUNSUPPORTED,
                 "dequant_gemm: group size must be a power of two");
-    if (qgemm_weight_ok(wa, d.K) && (!pair || qgemm_weight_ok(wb, d.K)))
+    if (qgemm_weight_ok(wa, d.K) && (pair ? qgemm_weight_ok(wb, d.K) : !qgemm_short(d.M, P, d.K)))
         return qgemm_launch<1>(ctx, wa, wb, (const f16_t *)a, P, out, mode, d);
     const uint32_t gl = (uint32_t)__builtin_ctz(d.group_size);
     const uint32_t grid = d.M / BN * ceil_div(P, BM);
@@ -1423,7 +1436,7 @@ int nnz_gemm_segments_launch(nnz_ctx *ctx, const nnz_qweight *const *w, void *co
         main_form = main_form && qgemm_weight_ok(w[i], K);
         r128 = r128 && rows[i] % 128 == 0;
     }
-    if (main_form) {
+    if (main_form && !qgemm_short(M, P, K)) {
         GemmArgs ga{(const f16_t *)a, {}, {}, {}, (uint32_t)nw, P, K, 0, nullptr, 1, 0};
         GemmMat *const m[3] = {&ga.m0, &ga.m1, &ga.m2};
         for (int i = 0; i < nw; ++i) *m[i] = GemmMat{w[i]->codes, (const uint16_t *)w[i]->scales, nullptr, out[i], rows[i]};

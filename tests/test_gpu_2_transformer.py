@@ -628,3 +628,25 @@ def test_dequant_gemm_main_shapes(dev, bits, P, M, K):
         return (np.abs((n - 8) * s) + np.abs(b + 8 * s)).reshape(M, K)
     se = 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ terms(wa).T)
     assert_bf16_faithful(host(out32), ra, "q4 gemm main", sum_err=se)
+
+
+@pytest.mark.parametrize("P,M,K", [(256, 4096, 2048), (320, 3072, 2048), (321, 2880, 2048), (1, 64, 1536),
+                                   (512, 4096, 512), (513, 3648, 512), (130, 192, 2560)])
+def test_dequant_gemm_short_launches(dev, P, M, K):
+    """Single 1-bit launches on both sides of the line between the short ones
+    (K <= 2048 on up to 256 blocks, K = 512 on up to 512) and the main kernel:
+    every store, the fp32 sums within the random-walk bound."""
+    w = cf.q1_matrix(M, K, 128, 500, 501)
+    a16 = (0.5 * S.normal(502, P * K)).astype(np.float16).reshape(P, K)
+    A, W = a16.astype(np.float64), O.dequant(w)
+    dw, ad = ops.DeviceQWeight(dev, w), tdev(a16)
+    out32 = torch.empty(P, M, dtype=torch.float32, device="cuda")
+    res = torch.zeros(P, M, dtype=torch.float32, device="cuda")
+    out16 = torch.empty(P, M, dtype=torch.float16, device="cuda")
+    ops.dispatch_dequant_gemm(dev, dw, ad, out32, L.GEMM_STORE_F32)
+    ops.dispatch_dequant_gemm(dev, dw, ad, res, L.GEMM_RESADD)
+    ops.dispatch_dequant_gemm(dev, dw, ad, out16, L.GEMM_STORE_F16)
+    dev.sync()
+    se = 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ np.abs(W).T)
+    assert (np.abs(host(out32) - A @ W.T) <= se).all()
+    assert torch.equal(res, out32) and torch.equal(out16, out32.half())
