@@ -768,7 +768,7 @@ constexpr size_t qgemm_lds() {
     return 2 * (size_t)(BM * BK * KQ) * 2 + 2 * (size_t)cpb * (64 * NSUB) * (64 + 8) + (BITS == 4 ? 4 * 64 * NSUB : 4);
 }
 constexpr size_t LDS_CU = 160 * 1024;
-static_assert(qgemm_lds<1, 1, 8>() <= LDS_CU && 2 * qgemm_lds<1, 1, 4>() <= LDS_CU && 3 * qgemm_lds<1, 2, 2>() <= LDS_CU &&
+static_assert(qgemm_lds<1, 1, 8>() <= LDS_CU && 2 * qgemm_lds<1, 1, 4>() <= LDS_CU && 3 * qgemm_lds<1, 1, 2>() <= LDS_CU && 2 * qgemm_lds<1, 2, 2>() <= LDS_CU &&
               qgemm_lds<4, 2, 4>() <= LDS_CU && 2 * qgemm_lds<4, 1, 4>() > LDS_CU && 3 * qgemm_lds<4, 2, 2>() <= LDS_CU,
               "blocks per CU");
 
@@ -897,6 +897,17 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[s][i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
+    // 1-bit launches on two k-phases keep a second set, for the u = 1 MFMAs, so
+    // that a float32 chain is no longer than four k-phases make it: with one
+    // set the result was 1.4 times as far from float64 (2048 x 6144, P = 1500:
+    // 3.5e-7 against 2.5e-7).  On 128-row blocks (179 registers) that leaves
+    // two blocks per CU instead of three.
+    constexpr bool TWO = BITS == 1 && KQ == 2 && !PAIR;
+    float4v acc1[TWO ? NSUB : 1][4][2];
+    if constexpr (TWO) {
+#pragma unroll
+        for (int t = 0; t < NSUB * 8; ++t) acc1[t / 8][(t / 2) % 4][t % 2] = (float4v){0.f, 0.f, 0.f, 0.f};
+    }
 
     const uint32_t nst = (ke - kb) / SK;
     auto issue = [&](uint32_t st) __attribute__((always_inline)) {   // W before the A of its first stage
@@ -964,9 +975,10 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
                         acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0][i], b0, acc[s][i][j], 0, 0, 0);
+                    auto &a1 = [&]() -> auto & { if constexpr (TWO) return acc1; else return acc; }();
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
-                        acc[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1][i], b1, acc[s][i][j], 0, 0, 0);
+                        a1[s][i][j] = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1][i], b1, a1[s][i][j], 0, 0, 0);
                 }
         } else {
             const uint16_t *const sp = (const uint16_t *)&Sc[wb][c][0];
@@ -1019,6 +1031,10 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
         if (st + 1 < nst) issue(st + 1);   // block-uniform
         compute(st);
         load_barrier();
+    }
+    if constexpr (TWO) {
+#pragma unroll
+        for (int t = 0; t < NSUB * 8; ++t) acc[t / 8][(t / 2) % 4][t % 2] += acc1[t / 8][(t / 2) % 4][t % 2];
     }
 
     // k-phase reduction through the (free) A buffers: phases [h, 2h) hand
@@ -1189,22 +1205,26 @@ void qgemm_split(nnz_ctx *ctx, GemmArgs ga, uint32_t rows, uint32_t splits) {
 }
 
 // Shape of a single-matrix launch (one or more row segments), by how many
-// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (42 KB of LDS, 128 rows
-// 51), of KQ = 4 two 1-bit ones (75 KB) or one 4-bit one (84 KB), one of KQ = 8
-// (140 KB).  More than one round of 768
-// KQ = 2 blocks: 128-row blocks, half the A traffic (2560 x 4096, P = 3001: 68
-// us against 76 with 64 rows; 6144 x 2560: 91 against 108; 4096 x 2048, P =
-// 1024: 23.5 against 26.6).  Up to 768, from 512 (1-bit) or 256 (4-bit), where
-// KQ = 4 takes a second round: one round of KQ = 2 64-row blocks
-// (2048 x 2048, P = 1500: 19.3 us against 21.4 with 128 rows and 23.7 on KQ =
-// 4; 6144 x 2560, P = 512: 22.6 against 25.1 and 25.0; 4-bit 4096 x 2560, P =
-// 400: 21.7 against 26.3 on KQ = 4, 2560 x 9728, P = 512: 65.8 against 79.7,
-// 2048 x 2048, P = 1024: 18.1 against 22.1).  Fewer: KQ = 4, more waves per
-// block (2048 x 6144, P = 1024: 33.5
-// against 38.5 on KQ = 2; 4-bit 2048 x 6144, P = 512: 29.2 against 41.9).  At
-// most one block per CU: KQ = 8 (1-bit of K > 2048, see qgemm_short; 2048 x
-// 6144, P = 512: 21.7 against 25.4 on KQ = 4; the 4-bit stages of KQ = 8 do not
-// fit LDS).
+// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (42 KB of LDS; of 128
+// rows two 1-bit ones, by registers, or three 4-bit ones), of KQ = 4 two 1-bit
+// ones (75 KB) or one 4-bit one (84 KB), one of KQ = 8 (140 KB).
+//   * More than one round of KQ = 2 64-row blocks: 128-row blocks, half the A
+//     traffic (1-bit 2560 x 4096, P = 3001: 66 us against 72 with 64 rows; 6144
+//     x 2560 97 against 104; 2560 x 9728, P = 1500 77 against 104) -- except
+//     1-bit grids of 1025 to 1536, whose 513 to 768 128-row blocks leave the
+//     second round of 512 half empty (6144 x 2560, P = 768: 31.1 us on 64 rows
+//     against 36.9; 4096 x 12288, P = 1280 139 against 156; at 1536, P = 1024,
+//     37.2 against 37.1).
+//   * Up to 768, from 512 (1-bit) or 256 (4-bit), where KQ = 4 takes a second
+//     round: one round of KQ = 2 64-row blocks (2048 x 2048, P = 1500: 18.0 us
+//     against 23.7 on KQ = 4; 6144 x 2560, P = 512: 22.6 against 25.0; 4-bit
+//     4096 x 2560, P = 400: 21.7 against 26.3, 2560 x 9728, P = 512: 65.8
+//     against 79.7, 2048 x 2048, P = 1024: 18.1 against 22.1).
+//   * Fewer: KQ = 4, more waves per block (2048 x 6144, P = 1024: 33.5 against
+//     38.5 on KQ = 2; 4-bit 2048 x 6144, P = 512: 29.2 against 41.9).
+//   * 1-bit, at most one block per CU: KQ = 8 (K > 2048, see qgemm_short; 2048
+//     x 6144, P = 512: 21.7 against 25.4 on KQ = 4; the 4-bit stages of KQ = 8
+//     do not fit LDS).
 template <int BITS, int MODE>
 void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128) {
     const uint32_t ny = ceil_div(ga.P, (uint32_t)BM);
@@ -1225,7 +1245,7 @@ void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128)
         return qgemm_split<BITS, MODE, 1, 4>(ctx, ga, rows, S);
     }
     if (g > 768) {
-        if (rows128) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
+        if (rows128 && (BITS == 4 || g <= 1024 || g > 1536)) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
         else qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
     } else if (g > (BITS == 1 ? 512u : 256u)) {
         qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);

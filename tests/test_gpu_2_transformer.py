@@ -650,3 +650,27 @@ def test_dequant_gemm_short_launches(dev, P, M, K):
     se = 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ np.abs(W).T)
     assert (np.abs(host(out32) - A @ W.T) <= se).all()
     assert torch.equal(res, out32) and torch.equal(out16, out32.half())
+
+
+def test_dequant_gemm_precision_over_shapes(dev):
+    """The launch shape does not cost precision: the fp32 sums of the same 640
+    tokens on two k-phases (64-row blocks at 672 and 1280 blocks, 128-row ones
+    at 1024) are no further from float64 than on four (320 blocks).  A chain of
+    half the roundings is 1 / sqrt(2) of the error, so a launch whose chains are
+    twice as long shows as 1.4; 1.1 leaves room for the sample (1.3M sums, the
+    ratio of two such norms good to 0.1 %)."""
+    M, K, n = 2048, 2560, 640
+    w = cf.q1_matrix(M, K, 128, 510, 511)
+    dw, W = ops.DeviceQWeight(dev, w), tdev(O.dequant(w))
+    a = tdev((0.5 * S.normal(512, 2500 * K)).astype(np.float16).reshape(2500, K))
+    ref = a[:n].double() @ W.T
+
+    def error(P):
+        out = torch.empty(P, M, dtype=torch.float32, device="cuda")
+        ops.dispatch_dequant_gemm(dev, dw, a[:P], out, L.GEMM_STORE_F32)
+        dev.sync()
+        return float((out[:n].double() - ref).norm() / ref.norm())
+
+    base = error(n)
+    for P in (1300, 2048, 2500):
+        assert error(P) <= 1.1 * base, (P, error(P), base)
