@@ -666,13 +666,14 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(2))) v
 // straight into LDS (no registers, no LDS stores) in pieces that use the lines
 // they touch: A 128 bytes per row and step, W codes 64 bytes per row (a chunk:
 // 512 k of 1-bit, 128 k of 4-bit codes), scales a dword.  A 4-bit weight is
-// dequantised exactly into its f16 operand (expand_nibbles_scaled), so its
+// dequantised exactly into its f16 operand (expand_nibbles_scaled; waves with a
+// row whose scales don't allow that take a loop of their own), so its
 // accumulators run through K unscaled and only the bias products remain on
 // the VALU.  Measured before -> now, weights rotated: 1-bit gate/up 2 x 6144 x
 // 2048 at P = 512 33.8 -> 30.5 us (845 TFLOP/s), 2 x 9728 x 2560 at P = 3001
 // 295 -> 268 (1113 TFLOP/s; the library's bf16 GEMM of that size without any
-// dequantisation 1161); 2560 x 9728 at P = 3001 195 -> 157, 2560 x 4096 86 ->
-// 68, 6144 x 2560 126 -> 91; 4-bit gate/up 2 x 6144 x 2048 at P = 512 59.7 ->
+// dequantisation 1161); 2560 x 9728 at P = 3001 190 -> 148, 2560 x 4096 82 ->
+// 68, 6144 x 2560 120 -> 97; 4-bit gate/up 2 x 6144 x 2048 at P = 512 59.7 ->
 // 47, 2 x 9728 x 2560 at P = 1500 290 -> 230.  Bounds now: 1-bit, one round of
 // blocks at P = 512 (first loads and epilogue overlap nothing), at large P the
 // L2-to-LDS rate of A (8.7 TB/s over the chip) and MFMA issue; 4-bit, VALU
@@ -728,10 +729,12 @@ __device__ __forceinline__ void expand_bits16(uint32_t h, uint32_t ns2, half8 &f
     f1 = __builtin_bit_cast(half8, f);
 }
 
-// 8 nibbles -> S (n - 8) 2^-20, exactly: the nibble in bits 4..7 of a half is
+// 8 nibbles -> S (n - 8) 2^-20, exact where it is an f16: the nibble in bits 4..7 of a half is
 // the (denormal) f16 value n 2^-20, and one fused multiply-add with S and
 // c = -8 S 2^-20 scales and centres it.  A bf16 scale has 8 significant bits
-// and |n - 8| <= 8 three more, or is a power of two: 11 bits, an f16.
+// and |n - 8| <= 8 three more, or is a power of two: 11 bits, an f16 down to
+// S = 2^3 (below, the last bits fall under the smallest f16).
+constexpr int ROW_WIDE = 0x40000000;
 __device__ __forceinline__ half8 expand_nibbles_scaled(uint32_t w, half2v S, half2v c) {
     const uint32_t lo = (w << 4) & 0xF0F0F0F0u, hi = w & 0xF0F0F0F0u;   // n[2j], n[2j+1] in byte j
     half8 r;
@@ -916,36 +919,62 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     };
     issue(0);
     int ex[NSUB][2];
+    bool wide = false;   // wave-uniform: the wave's weights don't fit f16 scaled
     if constexpr (BITS == 4) {
         // Row exponents: S = s 2^e with the row's largest |s| in [2^15, 2^16),
         // so that S (n - 8) 2^-20 is exact in f16 for scales down to 2^-12 of
-        // the largest; below that weights are rounded at 2^-25, which is 2^-23
-        // of the row's largest weight 8 |s|, a float32 rounding of its terms.  The row's threads scan its scales.
+        // the largest.  A row whose nonzero scales spread further, or whose
+        // largest is outside 2^-21 .. 2^12 (where the scaled sums might leave
+        // float32's range before the results do: within, that takes results
+        // of 2^111), infinite or NaN is wide: its wave multiplies the nibbles
+        // as they are and applies scales and biases in float32 per group.  The
+        // row's threads scan its scales.
         constexpr int TPR = THREADS / ROWS;   // threads per row
         static_assert(TPR == 2 || TPR == 4 || TPR == 8, "a row's threads are lanes of one octet");
         const int row = tid / TPR, sub = row >> 6;
         const uint16_t *const s0 = uniform_ptr(sbase0), *const s1 = uniform_ptr(sbase1);
         const auto *const rs = (const __attribute__((address_space(1))) u32x4 *)((sub ? s1 : s0) + (size_t)(row & 63) * G);
-        uint32_t mx = 0;
+        uint32_t mx = 0, mn1 = 0xFFFFFFFFu;    // largest |s|, smallest nonzero |s| less 1 (bits)
         const uint32_t np = (ke - kb) / 512;   // 16-byte pieces of the row's scales
         for (uint32_t p = tid % TPR; p < np; p += 4 * TPR) {
             u32x4 v[4];   // four loads in flight; past the end the last piece again
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[e] = rs[min(p + (uint32_t)(e * TPR), np - 1)];
 #pragma unroll
-            for (int e = 0; e < 16; ++e) mx = max(mx, max(v[e / 4][e % 4] & 0x7FFFu, (v[e / 4][e % 4] >> 16) & 0x7FFFu));
+            for (int e = 0; e < 16; ++e) {
+                const uint32_t a = v[e / 4][e % 4] & 0x7FFFu, b = (v[e / 4][e % 4] >> 16) & 0x7FFFu;
+                mx = max(mx, max(a, b));
+                mn1 = min(mn1, min(a - 1u, b - 1u));
+            }
         }
 #pragma unroll
-        for (int o = 1; o < TPR; o *= 2) mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
-        const int e8 = (int)(min(mx, 0x7F7Fu) >> 7);
-        if (tid % TPR == 0) rowexp[row] = mx ? 142 - e8 : 0;   // 15 - (e8 - 127)
+        for (int o = 1; o < TPR; o *= 2) {
+            mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
+            mn1 = min(mn1, (uint32_t)__shfl_xor((int)mn1, o, 64));
+        }
+        if (tid % TPR == 0) {
+            const uint32_t hi = mx >> 7, lo = (mn1 + 1u) >> 7;   // exponent fields
+            // all zero: the sums of the biases as they are
+            rowexp[row] = mx == 0 ? 20 : (hi >= 106 && hi < 139 && hi - lo <= 12 ? 142 - (int)hi : ROW_WIDE);   // 15 - (hi - 127)
+        }
     }
     load_barrier();
     if constexpr (BITS == 4) {
+        bool any = false;
 #pragma unroll
         for (int s = 0; s < NSUB; ++s)
 #pragma unroll
-            for (int j = 0; j < 2; ++j) ex[s][j] = rowexp[64 * s + 32 * wn + 16 * j + r16];
+            for (int j = 0; j < 2; ++j) {
+                ex[s][j] = rowexp[64 * s + 32 * wn + 16 * j + r16];
+                any = any || ex[s][j] == ROW_WIDE;
+            }
+        wide = __builtin_amdgcn_ballot_w64(any) != 0;
+        if (wide) {
+#pragma unroll
+            for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) ex[s][j] = 20;
+        }
     }
 
     const half8 ones = {(_Float16)1.f, (_Float16)1.f, (_Float16)1.f, (_Float16)1.f,
@@ -1027,11 +1056,51 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
         }
     };
 
-    for (uint32_t st = 0; st < nst; ++st) {
-        if (st + 1 < nst) issue(st + 1);   // block-uniform
-        compute(st);
-        load_barrier();
-    }
+    // 4-bit, a wide wave: products of the nibbles (as n 2^-5) with A, then s and
+    // b per group
+    auto compute_wide = [&](uint32_t st) __attribute__((always_inline)) {
+        const f16_t *const buf = As[st & 1];
+        const uint32_t wb = (st / SPC) & 1;
+        const int step = SPC > 1 ? (int)(st % SPC) * KQ + kq : kq;
+        const int c = step / CSTEPS, cs = step % CSTEPS;
+        const uint16_t *const sp = (const uint16_t *)&Sc[wb][c][0];
+        const half2v S = {(_Float16)0x1p15f, (_Float16)0x1p15f}, none = {(_Float16)0.f, (_Float16)0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            half8 af[2];
+#pragma unroll
+            for (int u = 0; u < 2; ++u)
+                af[u] = *(const half8 *)(buf + (i * 16 + r16) * SK + 8 * ((kq * 8 + 2 * q + u) ^ r16));
+            float4v xs = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0], ones, (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+            xs = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1], ones, xs, 0, 0, 0);
+#pragma unroll
+            for (int s = 0; s < NSUB; ++s)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) {
+                    const int row = 64 * s + 32 * wn + 16 * j + r16, at = s * 256 + (32 * wn + 16 * j + r16) * 2 + cs;
+                    const u32x2 w = *(const u32x2 *)&Wc[wb][c][row * 16 + (((2 * cs + (q >> 1)) ^ ((row >> 2) & 3)) << 2) +
+                                                                  (q & 1) * 2];
+                    float4v t = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[0], expand_nibbles_scaled(w[0], S, none),
+                                                                       (float4v){0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
+                    t = __builtin_amdgcn_mfma_f32_16x16x32_f16(af[1], expand_nibbles_scaled(w[1], S, none), t, 0, 0, 0);
+                    const float sc = bf16_to_f32(sp[at]), bi = bf16_to_f32(sp[at + 128]);
+#pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        acc[s][i][j][r] = fmaf(bi, xs[r], fmaf(sc, t[r] * 0x1p5f, acc[s][i][j][r]));
+                }
+        }
+    };
+
+    // a wide wave in a loop of its own (the same barriers)
+    auto stages = [&](auto f) __attribute__((always_inline)) {
+        for (uint32_t st = 0; st < nst; ++st) {
+            if (st + 1 < nst) issue(st + 1);   // block-uniform
+            f(st);
+            load_barrier();
+        }
+    };
+    if (BITS == 4 && wide) stages(compute_wide);
+    else stages(compute);
     if constexpr (TWO) {
 #pragma unroll
         for (int t = 0; t < NSUB * 8; ++t) acc[t / 8][(t / 2) % 4][t % 2] += acc1[t / 8][(t / 2) % 4][t % 2];

@@ -674,3 +674,64 @@ def test_dequant_gemm_precision_over_shapes(dev):
     base = error(n)
     for P in (1300, 2048, 2500):
         assert error(P) <= 1.1 * base, (P, error(P), base)
+
+
+@pytest.mark.parametrize("P,M,K", [(3, 64, 512), (65, 192, 1536), (45, 192, 2560), (70, 4096, 4608),
+                                   (1024, 1088, 512), (1030, 3136, 512), (833, 3840, 512)])
+def test_dequant_gemm_q4_wide_rows(dev, P, M, K):
+    """4-bit rows that the main kernel's scaled f16 weights cannot hold: scales
+    2^24 apart (every second token is zero where the large ones are, so only
+    the small ones show), scales far below the biases (denormal ones, and none
+    at all), and an infinite scale.  Blocks of 32 rows (a wave's) are of one
+    kind, the first of ordinary rows.  Every launch shape: four and two
+    k-phases, K split four and two ways, 64- and 128-row blocks, pairs."""
+    from nnzap_amd import formats as fm
+    from nnzap_amd.formats import QWeight
+    rng = np.random.default_rng([P, M, K])
+    G = K // 64
+    kind = (np.arange(M) // 32) % 4   # 0 ordinary, 1 spread, 2 tiny scales, 3 large scales
+
+    def weight():
+        s = rng.uniform(0.5, 1.0, (M, G)) / 64 * rng.choice([-1.0, 1.0], (M, G))
+        b = 8 * s * rng.uniform(-1.2, 0.2, s.shape)
+        s[kind == 1, 1::2] *= 2.0 ** -24
+        b[kind == 1, 1::2] *= 2.0 ** -24
+        s[kind == 2] *= np.where(rng.random((int((kind == 2).sum()), 1)) < 0.5, 2.0 ** -130, 0.0)
+        s[kind == 3] *= 2.0 ** 60
+        codes = rng.integers(0, 1 << 32, (M, K // 8), dtype=np.uint32)
+        return QWeight(4, M, K, 64, codes, S.f64_to_bf16_bits(s), S.f64_to_bf16_bits(b), fm.DT_BF16)
+
+    wa, wb = weight(), weight()
+    if M > 64:   # one more row: infinite in its first group, nibbles >= 1
+        wa.scales[40, 0] = 0x7F80
+        wa.codes[40] |= np.uint32(0x11111111)
+    a16 = (0.5 * rng.standard_normal((P, K))).astype(np.float16)
+    a16[0] = np.abs(a16[0]) + np.float16(0.125)
+    a16.reshape(P, G, 64)[1::2, 0::2] = 0.0
+    A, da, db, ad = a16.astype(np.float64), ops.DeviceQWeight(dev, wa), ops.DeviceQWeight(dev, wb), tdev(a16)
+
+    def ref_and_bound(w):
+        sc = S.bf16_bits_to_f32(w.scales).astype(np.float64)[:, :, None]
+        bi = S.bf16_bits_to_f32(w.biases).astype(np.float64)[:, :, None]
+        n = fm.unpack_q4(w.codes, K).reshape(M, G, 64).astype(np.float64)
+        terms = (n * np.abs(sc) + np.abs(bi) + 16 * np.abs(sc)).reshape(M, K)
+        # fp32 sums of s n and b, centred or not (random walk, 4 sigma)
+        return A @ (sc * n + bi).reshape(M, K).T, 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ terms.T)
+
+    out32 = torch.empty(P, M, dtype=torch.float32, device="cuda")
+    pair = torch.empty(P, M, dtype=torch.float16, device="cuda")
+    ops.dispatch_dequant_gemm(dev, da, ad, out32, L.GEMM_STORE_F32)
+    ops.dispatch_dequant_gemm(dev, da, ad, pair, L.GEMM_SILU_PAIR, wb=db)
+    dev.sync()
+    got, gp = host(out32), host(pair)
+    with np.errstate(invalid="ignore"):
+        ra, sa = ref_and_bound(wa)
+    rb, sb = ref_and_bound(wb)
+    rows = np.arange(M) != 40 if M > 64 else np.ones(M, bool)
+    if M > 64:
+        assert got[0, 40] == np.inf
+    assert_bf16_faithful(got[:, rows], ra[:, rows], "wide rows", sum_err=sa[:, rows])
+    rows &= kind < 2   # the others leave f16's range
+    ra, rb, sa, sb = (v[:, rows] for v in (ra, rb, sa, sb))
+    se = 1.1 * np.abs(rb) * sa + np.abs(O.silu(ra)) * sb + 1.1 * sa * sb
+    assert_bf16_faithful(gp[:, rows], O.silu(ra) * rb, "wide rows, pair", sum_err=se + 2.0 ** -24)
