@@ -659,6 +659,11 @@ int nnz_q1_mfma_launch(nnz_ctx *ctx, const NnzQ1Mfma &c) {
     const uint32_t gy = c.stack_count ? c.stack_count : 1u;
     uint32_t blocks = c.blocks_per_matrix ? c.blocks_per_matrix : ceil_div(256u, gy);
     if (c.K != KC) {
+        // One block per CU, and rows are long: a few blocks over 256 cost a
+        // second round, so as many per matrix as stay within one.  Rounded up /
+        // down: 24 of 1024 x 4096 16.8 / 11.0 us, 100 of 2048 x 6144 60.9 / 44.4,
+        // 129 79.1 / 71.2, 255 93.9 / 87.0.
+        if (!c.blocks_per_matrix) blocks = max(1u, 256u / gy);
         const uint32_t parts = c.K / KC;
         blocks = max(1u, min(blocks, ceil_div(tiles, 12u / parts)));
         if (parts == 2) qmv1_mfma_split_kernel<2><<<dim3(blocks, gy), 768, 0, ctx->stream>>>(a);

@@ -557,8 +557,8 @@ def test_q1_matrix_cores_qmv(dev, q1_cores, M):
 @pytest.mark.parametrize("M", [1, 65, 2048, 20011])
 def test_q1_matrix_cores_long_rows(dev, q1_cores, M, K):
     """Rows of two and three 2048-column parts (f32 in and out): partial
-    tiles, blocks with one round and with several (20011 rows over 256
-    blocks), the oracle within 1e-3 and the VALU kernel within float32
+    tiles, one tile a wave and two (20011 rows over 209 or 256 blocks; one
+    round of them: test_stacked_long_rows_rounds has more), the oracle within 1e-3 and the VALU kernel within float32
     rounding; the error against float64 is that of one rounding per group
     and part, below 2^-20 of the largest output."""
     w = cf.q1_matrix(M, K, 128, 720 + M % 97, 721)
@@ -577,6 +577,67 @@ def test_q1_matrix_cores_long_rows(dev, q1_cores, M, K):
     _near_valu(a, b, f"M={M} K={K}")
     err = np.max(np.abs(host(a).astype(np.float64) - ref)) / np.max(np.abs(ref))
     assert err <= 2.0 ** -20, f"M={M} K={K}: {err:.2e} of max |y|"
+
+
+@pytest.mark.parametrize("K", [4096, 6144])
+@pytest.mark.parametrize("M,n,bpm", [(2048, 3, 1), (2041, 3, 1), (2041, 2, 2), (1024, 24, 0), (16, 300, 0)])
+def test_stacked_long_rows_rounds(dev, q1_cores, M, n, bpm, K):
+    """Stacked rows of two and three parts with few blocks per matrix, so that a
+    wave runs up to 32 tiles and a block up to eight rounds (the double-buffered
+    sums and the ring of tiles come round), ragged and even row counts, and the
+    library's own grids: the oracle, and the single launch to the bit."""
+    q1_cores(1)
+    sw = ops.StackedQWeights(dev, M, K, 128, 1, n, 16, (0.01, 0.05))
+    x = torch.randn(n, K, device="cuda", generator=torch.Generator("cuda").manual_seed(17))
+    y = torch.full((n, M), float("nan"), device="cuda")
+    ops.dispatch_qmv_stacked(dev, sw, x, y, bpm)
+    dev.sync()
+    for i in (0, n - 1):
+        w = sw.host(i)
+        y1 = torch.empty(M, device="cuda")
+        ops.dispatch_qmv(dev, _dw(dev, w), x[i].contiguous(), y1)
+        dev.sync()
+        assert torch.equal(y[i], y1), f"matrix {i}: stacked != single launch"
+        assert_close(host(y[i]), O.qmv(w, x[i].cpu().numpy()), what=f"matrix {i}")
+
+
+@pytest.mark.parametrize("M,K,n,cores", [(1024, 4096, 13, 2), (1024, 4096, 14, 1), (512, 6144, 18, 2), (512, 6144, 19, 1)])
+def test_stacked_long_rows_default(dev, q1_cores, M, K, n, cores):
+    """Long stacked rows under the default option: the VALU kernel below 7 MB of
+    codes, the matrix cores from there on (to the bit what the option that
+    forces each gives)."""
+    sw = ops.StackedQWeights(dev, M, K, 128, 1, n, 18, (0.01, 0.05))
+    x = torch.randn(n, K, device="cuda", generator=torch.Generator("cuda").manual_seed(19))
+
+    def run(option):
+        q1_cores(option)
+        y = torch.full((n, M), float("nan"), device="cuda")
+        ops.dispatch_qmv_stacked(dev, sw, x, y)
+        dev.sync()
+        return y
+    assert torch.equal(run(0), run(cores)) and not torch.equal(run(0), run(3 - cores))
+
+
+def test_stacked_long_rows_one_round(dev, q1_cores):
+    """The library's grid stays within one round of blocks: 24 matrices take
+    about what 21 do (11.0 us against 10.2; 16.8 with a second round)."""
+    q1_cores(1)
+    M, K = 1024, 4096
+    x, y = torch.randn(24, K, device="cuda"), torch.empty(24, M, device="cuda")
+
+    def time_us(n):
+        sw = ops.StackedQWeights(dev, M, K, 128, 1, n, 20, (0.01, 0.05))
+        torch.cuda.synchronize()
+        best = []
+        for _ in range(5):
+            dev.mark(0)
+            for _ in range(50):
+                ops.dispatch_qmv_stacked(dev, sw, x, y)
+            dev.mark(1)
+            dev.sync()
+            best.append(dev.elapsed_ms(0, 1) * 1e3 / 50)
+        return min(best)
+    assert time_us(24) <= 1.3 * time_us(21)
 
 
 def test_q1_matrix_cores_long_rows_nonfinite(dev, q1_cores):
