@@ -1301,11 +1301,15 @@ int launch_qmv_ex(nnz_ctx *ctx, const nnz_qweight *const *w, const uint32_t *seg
     }
 
     // 1-bit rows of K = 2048, 4096 or 6144, group size 128: the block-scaled
-    // MFMA kernels (qmv_mfma.hip) where the context's policy picks them.
+    // MFMA kernels (qmv_mfma.hip) where the context's policy picks them and the
+    // scales are 4-byte aligned (those kernels load them 16 bytes at a time, the
+    // VALU kernel two).
     NNZ_REQUIRE(ctx, !top2 || (EPI == EPI_STORE && NMAT == 1 && ODT == NNZ_F32 && nw == 1 && !stk),
                 NNZ_EUNSUPPORTED, "%s: top-2 partials need one f32-output matrix", name);
     if constexpr (BITS == 1 && !FAITH && !MERGE) {
-        if (!top2 && q1_matrix_cores_wanted(ctx, d, stk) && (NMAT == 2 || nw == 1)) {
+        bool scales_ok = true;
+        for (int i = 0; i < NMAT; ++i) scales_ok = scales_ok && ((uintptr_t)w[i]->scales & 3) == 0;
+        if (!top2 && scales_ok && q1_matrix_cores_wanted(ctx, d, stk) && (NMAT == 2 || nw == 1)) {
             NnzQ1Mfma c;
             for (int i = 0; i < NMAT; ++i) {
                 c.codes[i] = w[i]->codes;

@@ -640,6 +640,27 @@ def test_stacked_long_rows_one_round(dev, q1_cores):
     assert time_us(24) <= 1.3 * time_us(21)
 
 
+@pytest.mark.parametrize("K", [2048, 4096, 6144])
+def test_stacked_scales_at_two_bytes(dev, q1_cores, K):
+    """Scales at an odd 2-byte address, which 1-bit QMVs take: not on the
+    matrix cores, whose loads are wider, whatever the option."""
+    from nnzap_amd import _lib as L
+    q1_cores(1)
+    M, n = 96, 3
+    sw = ops.StackedQWeights(dev, M, K, 128, 1, n, 21, (0.01, 0.05))
+    ref = [O.qmv(sw.host(i), np.ones(K, np.float32) * np.arange(K) / K) for i in range(n)]
+    moved = torch.zeros(sw.scales.numel() + 2, dtype=torch.int16, device="cuda")
+    moved[1:-1] = sw.scales.flatten()
+    sw.desc = L.QWeightDesc(sw.codes.data_ptr(), moved.data_ptr() + 2, None, M * K, 128, 1, sw.scale_dtype)
+    x = (torch.arange(K, device="cuda", dtype=torch.float64) / K).float().repeat(n, 1)
+    y = torch.full((n, M), float("nan"), device="cuda")
+    torch.cuda.synchronize()
+    ops.dispatch_qmv_stacked(dev, sw, x, y)
+    dev.sync()
+    for i in range(n):
+        assert_close(host(y[i]), ref[i], what=f"matrix {i}")
+
+
 def test_q1_matrix_cores_long_rows_nonfinite(dev, q1_cores):
     """An infinity or NaN in x reaches the outputs (the digit rows cannot hold
     one), and only those of its own matrix in a stacked launch."""
