@@ -1444,10 +1444,13 @@ int launch_qmv_ex(nnz_ctx *ctx, const nnz_qweight *const *w, const uint32_t *seg
         // -> 5.05).
         if (NMAT == 1 && nv == 2 && R >= 4) max_blocks = d.M <= 4u * 4u * 512u ? 256u : 512u;
         if (NMAT == 1 && nv == 1 && R == 8) max_blocks = 768u;
-        // a pair's 2048 waves: two-row steps where they come out as fewer rows
-        // (9728 x 2560: three steps of two against two of four, 7.4 -> 6.6 us;
-        // 12288 x 4096 8.3 either way)
-        if (NMAT == 2 && nv == 2 && R == 4 && blocks > max_blocks && ceil_div(d.M, 4096u) * 2 < ceil_div(d.M, 8192u) * 4) {
+        // a pair's 2048 waves: two-row steps where the last one is then at most
+        // half full, so that they come out as fewer rows than four-row steps
+        // (9728 x 2560: three steps of two against two of four, 7.1 -> 6.6 us;
+        // 10240 x 4096 7.9 -> 7.3; fuller ones lose what they save, 11264 x 3072
+        // 7.28 / 7.44, 12288 x 3072 7.36 / 7.54)
+        const uint32_t over = d.M % 8192u;
+        if (NMAT == 2 && nv == 2 && R == 4 && blocks > max_blocks && over > 0 && over <= 2048u) {
             R = 2;
             blocks = ceil_div(d.M, 4u * R * rpw);
         }

@@ -238,6 +238,21 @@ def test_fused_norm_long_rows_grids(dev, M, K):
     assert_close(host(h), _f16(O.qmv_pair_silu(wa, wb, xn)), what="norm pair silu")
 
 
+@pytest.mark.parametrize("M,K", [(10240, 2560), (10241, 2560), (12288, 2560), (18432, 4096)])
+def test_fused_norm_pair_two_row_steps(dev, M, K):
+    """Norm + gate/up of K > 2048 on both sides of the line where two-row steps
+    end: a last step that is half full, one row more, a full one, and the next
+    range's."""
+    wa, wb = cf.q1_matrix(M, K, 128, 374, 375), cf.q1_matrix(M, K, 128, 376, 377)
+    res = S.normal(378, K).astype(np.float32)
+    nw = (1.0 + 0.1 * S.normal(379, K)).astype(np.float32)
+    a, b, rd, nd = _dw(dev, wa), _dw(dev, wb), tdev(res), tdev(nw)
+    h = torch.full((M,), float("nan"), dtype=torch.float16, device="cuda")
+    ops.dispatch_fused_norm_pair_silu_f16io(dev, a, b, rd, h, nd)
+    dev.sync()
+    assert_close_f16(host(h), O.qmv_pair_silu(wa, wb, O.norm_to_half(res, nw)), what="norm pair silu")
+
+
 @pytest.mark.parametrize("qrows,kvrows,K", [(4096, 1024, 4096), (4096, 1024, 2560), (8192, 64, 4096)])
 def test_fused_norm_qkv_long_rows(dev, qrows, kvrows, K):
     """Norm + Q/K/V of K > 2048: fewer blocks than steps, segments met in one
