@@ -585,7 +585,7 @@ __global__ __launch_bounds__(256) void attn_split_kernel(AttnArgs a) {
 
 // ------------------------------------------------- fused decode attention --
 // The attention half of a decode step for one layer:
-//   attn_fused_kernel, grid (chunks of FCHUNK tokens, Hkv), 256 threads:
+//   attn_fused_kernel (head_dim 64), grid (chunks of FCHUNK tokens, Hkv), 256 threads:
 //     * first, every thread issues its K and V loads for the chunk (they do
 //       not depend on q), so the q prologue, the scores and P.V wait on one
 //       memory round trip instead of three;
@@ -638,9 +638,9 @@ __device__ __forceinline__ size_t part_ml_at(const FusedAttnArgs &a, uint32_t qh
     return a.unit_major ? (size_t)c * (a.kdim / D) + qh : (size_t)qh * a.nchunks + c;
 }
 
-template <int D, int G>
+template <int G>
 __global__ __launch_bounds__(256) void attn_fused_kernel(FusedAttnArgs a) {
-    static_assert(G * D <= 1024, "group too large");
+    constexpr int D = 64;   // a head is one wave wide
     constexpr int NQ = (G * D + 255) / 256;
     constexpr int TPT = 256 / FCHUNK;          // lanes per token in the score pass
     constexpr int KV4 = D / 8 / TPT;           // K: 16-byte vectors per lane
@@ -652,9 +652,8 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(FusedAttnArgs a) {
     __shared__ float ps[G][FCHUNK];   // scores
     __shared__ float pe[G][FCHUNK];   // exp(score - max)
     __shared__ float knew[D], vnew[D];
-    __shared__ float red[4][G];
     __shared__ float ored[PARTS][G][D];
-    __shared__ float hsum[G][4];
+    __shared__ float hsum[G];
 
     const int tid = threadIdx.x;
     // 1-D grid.  Unit u = (chunk c, KV head h); its `parts` blocks serve the
@@ -733,19 +732,13 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(FusedAttnArgs a) {
     for (int k = 0; k < NQ; ++k) {
         const int i = tid + 256 * k;
         if (i >= G * D) qv[k] = 0.f;
-        // lanes of one wave belong to one head (D >= 64)
         const float s = wave_sum(qv[k] * qv[k]);
-        if ((tid & 63) == 0 && i < G * D) hsum[i / D][(i % D) / 64] = s;
+        if ((tid & 63) == 0 && i < G * D) hsum[i / D] = s;
     }
     // new key: RMSNorm * k_norm, RoPE, f16; appended to the caches
     if (owns_new) {
         const float kv = tid < D ? kraw : 0.f;
-        float ss = wave_sum(kv * kv);
-        if (D > 64) {
-            if ((tid & 63) == 0) red[tid >> 6][0] = ss;
-        }
-        __syncthreads();
-        if (D > 64) ss = red[0][0] + red[1][0];
+        const float ss = wave_sum(kv * kv);   // the first wave's
         const float kn = kv * rsqrtf(ss / (float)D + a.eps) * knw;
         const float partner = __shfl_xor(kn, 1, 64);
         const float kr = f16_round(rope_rotate_f(kn, partner, tid, pos, kfreq));
@@ -764,10 +757,7 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(FusedAttnArgs a) {
         const int i = tid + 256 * k;
         const bool ok = i < G * D;
         const int g = ok ? i / D : 0, d = i % D;
-        float ss = 0.f;
-#pragma unroll
-        for (int w = 0; w < D / 64; ++w) ss += hsum[g][w];
-        const float v = ok ? qv[k] * rsqrtf(ss / (float)D + a.eps) * qnv[k] : 0.f;
+        const float v = ok ? qv[k] * rsqrtf(hsum[g] / (float)D + a.eps) * qnv[k] : 0.f;
         const float partner = __shfl_xor(v, 1, 64);  // all lanes take part
         if (ok) qs[g][d] = rope_rotate_f(v, partner, d, pos, qfreq[k]);
     }
@@ -806,32 +796,18 @@ __global__ __launch_bounds__(256) void attn_fused_kernel(FusedAttnArgs a) {
     }
     __syncthreads();
 
-    // ---- softmax over the chunk, all G heads at once: lane l holds tokens
-    // l, l + 64, ... so every wave sees the whole chunk and computes the
-    // same max and sum (no cross-wave step).
-    constexpr int TPL = (FCHUNK + 63) / 64;   // tokens per lane
+    // ---- softmax over the chunk, all G heads at once: lane l holds token l,
+    // so every wave sees the whole chunk and computes the same max and sum (no
+    // cross-wave step).
+    static_assert(FCHUNK == 64, "a token per lane");
     float mval[G], lval[G];
-    {
-        const int lane = tid & 63;
 #pragma unroll
-        for (int g = 0; g < G; ++g) {
-            float sc[TPL];
-            float m = -INFINITY;
-#pragma unroll
-            for (int k = 0; k < TPL; ++k) {
-                sc[k] = lane + 64 * k < FCHUNK ? ps[g][lane + 64 * k] : -INFINITY;
-                m = fmaxf(m, sc[k]);
-            }
-            mval[g] = wave_max(m);
-            float l = 0.f;
-#pragma unroll
-            for (int k = 0; k < TPL; ++k) {
-                const float e = lane + 64 * k < FCHUNK ? expf(sc[k] - mval[g]) : 0.f;
-                l += e;
-                if (tid < 64 && lane + 64 * k < FCHUNK) pe[g][lane + 64 * k] = e;
-            }
-            lval[g] = wave_sum(l);
-        }
+    for (int g = 0; g < G; ++g) {
+        const float sc = ps[g][tid & 63];
+        mval[g] = wave_max(sc);
+        const float e = expf(sc - mval[g]);
+        if (tid < 64) pe[g][tid] = e;
+        lval[g] = wave_sum(e);
     }
     __syncthreads();
 
@@ -2495,10 +2471,10 @@ int nnz_attn_fused1_launch(nnz_ctx *ctx, const void *q, const void *kr, const vo
         const uint32_t gb = (a.nchunks * hkv < 128) ? 1u : G;
         a.parts = G / gb;
         const dim3 grid(a.parts == 1 ? a.units : ceil_div(a.units, 8u) * 8u * a.parts);
-        if (gb == 1) attn_fused_kernel<64, 1><<<grid, 256, 0, ctx->stream>>>(a);
-        else if (G == 2) attn_fused_kernel<64, 2><<<grid, 256, 0, ctx->stream>>>(a);
-        else if (G == 4) attn_fused_kernel<64, 4><<<grid, 256, 0, ctx->stream>>>(a);
-        else attn_fused_kernel<64, 8><<<grid, 256, 0, ctx->stream>>>(a);
+        if (gb == 1) attn_fused_kernel<1><<<grid, 256, 0, ctx->stream>>>(a);
+        else if (G == 2) attn_fused_kernel<2><<<grid, 256, 0, ctx->stream>>>(a);
+        else if (G == 4) attn_fused_kernel<4><<<grid, 256, 0, ctx->stream>>>(a);
+        else attn_fused_kernel<8><<<grid, 256, 0, ctx->stream>>>(a);
     }
     NNZ_LAUNCHED(ctx);
     if (a.nchunks > 1 && !partials_only) {
