@@ -491,7 +491,8 @@ def test_dequant_gemm_q4_modes(dev, P, M, K, gs, sdt):
     """4-bit (q4_mlx) weights: s * (A . n) + b * sum(A) per group on the MFMA,
     every mode BF16-faithful like the Q4 decode kernels (one bf16 ulp bar).
     The last case has 320 blocks (more than one per CU), so the single-matrix
-    modes run the two-k-phase kernel real 4-bit prefill takes at hidden 2560."""
+    modes run the main kernel's two k-phases, as real 4-bit prefill does at
+    hidden 2560 (the general kernel's: test_dequant_gemm_q4_general_grids)."""
     from nnzap_amd import formats as fm
     sd = fm.DT_BF16 if sdt == 2 else fm.DT_F16
     wa = cf.q4_matrix(M, K, gs, 520, 521, 522, scale_dtype=sd)
@@ -526,6 +527,14 @@ def test_dequant_gemm_q4_modes(dev, P, M, K, gs, sdt):
     se_b = 4 * 2.0 ** -24 * np.sqrt(K) * (np.abs(A) @ np.abs(O.dequant(wb)).T)
     se_pair = 1.1 * np.abs(rb) * se + np.abs(O.silu(ra)) * se_b
     assert_bf16_faithful(host(pair), O.silu(ra) * rb, "q4 gemm silu pair", sum_err=se_pair)
+
+
+@pytest.mark.parametrize("P,M,K,gs,sdt", [(512, 2560, 2112, 64, 2), (512, 2560, 2048, 128, 1), (512, 2560, 2048, 64, 1)])
+def test_dequant_gemm_q4_general_grids(dev, P, M, K, gs, sdt):
+    """4-bit weights that the main kernel does not take (K not a multiple of
+    512, group size 128, f16 scales) on 320 blocks: the general kernel's
+    two-k-phase single-matrix forms, every mode."""
+    test_dequant_gemm_q4_modes(dev, P, M, K, gs, sdt)
 
 
 def test_dequant_gemm_split_under_capture(dev):
@@ -576,10 +585,11 @@ def test_gemm_row_equals_decode_qmv(dev):
                                         (4, 1, 64, 512), (4, 65, 192, 1536), (4, 64, 128, 4096),
                                         (4, 1030, 3136, 512), (4, 833, 3840, 512)])
 def test_dequant_gemm_main_shapes(dev, bits, P, M, K):
-    """The main prefill GEMM at the edges of its launch shapes: one token, one
-    past a token tile, one 64-row block, eight and four k-phases, two k-phases
-    on 64-row blocks (rows not a multiple of 128, and up to 768 blocks) and on
-    128-row ones, one W chunk and several, K split four and two ways with
+    """The prefill GEMM at the edges of its launch shapes (short 1-bit ones,
+    here of up to 128 blocks and K <= 1536, are the general kernel's): one
+    token, one past a token tile, one 64-row block, eight and four k-phases, two
+    k-phases on 64-row blocks (rows not a multiple of 128, and up to 768 blocks)
+    and on 128-row ones, one W chunk and several, K split four and two ways with
     parts of unequal length.  The 4-bit rows hold scales over
     eleven octaves, negative and zero ones among them, each row at a size of
     its own."""

@@ -93,8 +93,9 @@ def test_decode_stream_across_step_graphs(mdev):
     chunk counts each) and decode_steps, called in uneven batches, replays
     for each step the one sized for its length.  Tokens and margins equal
     the uncaptured loop's (which sizes every step exactly; partials past the
-    live length are never read, so the arithmetic is the same) bit for bit,
-    and the oracle's tokens up to its first near-tie step."""
+    live length are never read, and at head_dim 64 the kernel does not depend
+    on the length, so the arithmetic is the same) bit for bit, and the oracle's
+    tokens up to its first near-tie step."""
     cfg = cf.DecoderConfig(**{**cf.TINY.__dict__, "max_context_length": 1024,
                               "max_prefill_length": 512})
     w = cf.decoder_weights(cfg, norm_mode="unit")
@@ -125,6 +126,69 @@ def test_decode_stream_across_step_graphs(mdev):
           f"(first oracle near-tie at {first_tie})", flush=True)
     assert first_bad >= first_tie
     assert np.max(np.abs(margins[:first_bad] - ref_m[:first_bad])) < 2e-3
+
+
+@pytest.mark.parametrize("hq,hkv,prompt_len,n", [(16, 8, 980, 60), (32, 8, 490, 40), (32, 8, 1010, 24)])
+def test_decode_stream_across_attention_kernels(mdev, hq, hkv, prompt_len, n):
+    """A head_dim-128 decode plan over the lengths where its attention changes:
+    16 heads from 64-token chunks on the wave kernel to 128-token ones on the
+    matrix cores (1025 keys), 32 heads from the wave kernel to 64-token chunks
+    on the matrix cores (513) and from those to 128-token ones.  The O
+    projection merges the 128-token partials.  The captured stream sizes a step
+    by its graph, the uncaptured loop by its own length, so near such a line
+    they take different kernels: each is held against the oracle, tokens up to
+    its first near tie and margins throughout, and the decode logits at
+    positions on both sides."""
+    cfg = cf.DecoderConfig(**{**cf.TINY.__dict__, "max_context_length": 1200, "max_prefill_length": 1010,
+                              "num_query_heads": hq, "num_kv_heads": hkv, "head_dim": 128, "num_layers": 1})
+    w = cf.decoder_weights(cfg, norm_mode="unit")
+    prompt = cf.prompt_ids(cfg, prompt_len)
+    ref, ref_m = OracleDecoder(w).generate(prompt, n + 1)
+    m = DecoderModel(mdev, cfg)
+    try:
+        m.load(w)
+        m.decode_begin(prompt, n)
+        for k in (1, n // 2, n - 1 - n // 2):
+            m.decode_steps(k)
+        streams = [m.decode_read(n + 1)]
+        m.decode_end()
+        streams.append(m.generate(prompt, n + 1, use_graph=False)[:2])
+        # teacher-forced logits over the oracle's tokens
+        o = OracleDecoder(w)
+        o.forward(list(prompt), 0)
+        m.prefill(prompt, 0)
+        for i in range(n):
+            r = o.forward([int(ref[i])], prompt_len + i)[0]
+            g = m.forward_decode(int(ref[i]), prompt_len + i)
+            assert_close_normwise(g, r, what=f"decode pos {prompt_len + i}")
+    finally:
+        m.close()
+    # margins are logit differences: two logit errors of <= 1e-3 max|logit|
+    ties = np.flatnonzero(ref_m < 2e-3)
+    first_tie = int(ties[0]) if len(ties) else n + 1
+    for toks, margins in streams:
+        bad = np.flatnonzero(toks[:n + 1] != ref)
+        first_bad = int(bad[0]) if len(bad) else n + 1
+        assert first_bad >= first_tie
+        assert np.max(np.abs(margins[:first_bad] - ref_m[:first_bad])) < 2e-3
+
+
+@pytest.mark.parametrize("P", [45, 129])
+def test_prefill_split_segments(mdev, P):
+    """Wide layers with few heads: a Q/K/V launch (three row segments) that splits
+    K, four ways at 4096 columns and 32 blocks, two ways at 6144 and 96, the
+    sum over the parts finding each segment's output; against the oracle."""
+    cfg = cf.DecoderConfig(**{**cf.TINY.__dict__, "hidden_size": 4096 if P == 45 else 6144, "num_layers": 1,
+                              "num_query_heads": 8, "num_kv_heads": 4, "head_dim": 128, "max_prefill_length": P})
+    w = cf.decoder_weights(cfg, norm_mode="unit")
+    ids = cf.prompt_ids(cfg, P)
+    ref = OracleDecoder(w).forward(list(ids), 0)
+    m = DecoderModel(mdev, cfg)
+    try:
+        m.load(w)
+        assert_close_normwise(m.prefill(ids, 0), ref[-1], what=f"{P}-token prefill")
+    finally:
+        m.close()
 
 
 def test_tiny_prefill_chunks_match_single_prefill(mdev, tiny):
