@@ -1085,14 +1085,16 @@ __global__ __launch_bounds__(256) void attn_fused_wave_kernel(FusedAttnArgs a) {
 //     so that lane group g's eight B slots are eight consecutive keys and a
 //     lane's V operand is one 16-byte load of its dim's row.
 //   * q is normalised and rotated by the wave w + 4 n of head w + 4 n (lane l
-//     on dims 2l, 2l + 1, a RoPE pair) and scaled by log2(e) / sqrt(D).  Its
-//     24 bits go into three f16 parts, and so do the probabilities': scaled by
-//     a power of two first (q by one that its largest possible value, from the
-//     norm weights, allows; p by 2^15), so that the last parts stay above the
-//     smallest f16 and the three products add up to the float32 ones.  Error
-//     of the merged partials against float64, three parts / float32 on the VALU
-//     / two parts: 16 query heads, 1500 tokens 2.1e-7 / 2.3e-7 / 3.1e-7; 32,
-//     3001 2.4e-7 / 2.3e-7 / 3.2e-7 (the third parts cost 0.35-0.4 us).
+//     on dims 2l, 2l + 1, a RoPE pair) and scaled by log2(e) / sqrt(D).  It goes
+//     into two f16 parts, both rounded to nearest (within 2^-24 of the value,
+//     a float32 rounding), and so do the probabilities, after a scaling by a
+//     power of two (q by one that its largest possible value, from the norm
+//     weights, allows; p by 2^15) that keeps the second parts above the smallest
+//     f16; their products are summed apart.  Error of the merged partials
+//     against float64, this / float32 on the VALU / truncated parts without the
+//     scaling: 16 query heads, 1500 tokens 2.0e-7 / 2.3e-7 / 3.1e-7; 32, 3001
+//     2.2e-7 / 2.3e-7 / 3.2e-7 (over 39 shapes and score spreads 0.93 and 1.39
+//     times the VALU's; the scaling and the infinities cost 0.4 us).
 //   * The block whose chunk holds position seq - 1 normalises, rotates and
 //     f16-rounds the new key (wave 3), appends it and the value to the caches
 //     and puts both into their lanes' operands.
@@ -1101,16 +1103,28 @@ __global__ __launch_bounds__(256) void attn_fused_wave_kernel(FusedAttnArgs a) {
 // (with its merge, which had one block per head): 32 query and 8 KV heads, 1500
 // tokens 14.8 -> 8.0 us, 3001 23.9 -> 8.3, 8192 57.4 -> 11.4; 16 query heads,
 // 1025 tokens 10.5 -> 7.4, 4096 26.8 -> 8.9.
+// A sum's products with the first parts and with the second ones.  Where a cache
+// holds an infinity the first alone decide, as the whole value would: a second
+// part may be zero (0 inf is NaN) or of the other sign.  The median of (v, v,
+// hi) is v, and hi where v is NaN.
+__device__ __forceinline__ float join_parts(float hi, float lo) {
+    float v = hi + lo;
+    asm("v_med3_f32 %0, %0, %0, %1" : "+v"(v) : "v"(hi));
+    return v;
+}
+
 template <int GM, int KW>
 __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     typedef _Float16 half8 __attribute__((ext_vector_type(8)));
+    typedef _Float16 half2v __attribute__((ext_vector_type(2)));
+    typedef float float2v __attribute__((ext_vector_type(2)));
     typedef float float4v __attribute__((ext_vector_type(4)));
     typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
     typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
     constexpr int D = 128, CH = 4 * KW, NT = KW / 16, NK = KW >= 32 ? KW / 32 : 1, NH = (GM + 3) / 4;
     constexpr int QP = D + 8;   // LDS pitch (halves) of a query part
     constexpr float PSC = 0x1p15f;   // of the probabilities' f16 parts
-    __shared__ __align__(16) _Float16 qs[GM][3][QP];
+    __shared__ __align__(16) _Float16 qs[GM][2][QP];
     __shared__ __align__(16) _Float16 knew[D];
     __shared__ uint16_t vnew[D];
     __shared__ __align__(16) float osh[4][GM][D];
@@ -1195,7 +1209,7 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
         float qe = fmaf(x0, cs, -x1 * sn) * sl, qo = fmaf(x0, sn, x1 * cs) * sl;
         if (hh < GM) {
 #pragma unroll
-            for (int i = 0; i < 3; ++i) {
+            for (int i = 0; i < 2; ++i) {
                 const f16_t he = (f16_t)qe, ho = (f16_t)qo;
                 *(uint32_t *)&qs[hh][i][2 * lane] =
                     (uint32_t)__builtin_bit_cast(uint16_t, he) | (uint32_t)__builtin_bit_cast(uint16_t, ho) << 16;
@@ -1223,12 +1237,12 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     __syncthreads();
 
     // ---- S^T = K . Q^T (log2 units)
-    half8 qf[3][4];
+    half8 qf[2][4];
     {
         const bool live = (uint32_t)c16 < heads;
         const int hc = c16 < GM ? c16 : 0;
 #pragma unroll
-        for (int i = 0; i < 3; ++i)
+        for (int i = 0; i < 2; ++i)
 #pragma unroll
             for (int ks = 0; ks < 4; ++ks) {
                 const half8 zero = {}, v = *(const half8 *)&qs[hc][i][32 * ks + 8 * g];
@@ -1254,13 +1268,12 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
             const half8 ka = __builtin_bit_cast(half8, kreg[t][ks]);
-            lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[2][ks], lo, 0, 0, 0);
             s[t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[0][ks], s[t], 0, 0, 0);
             lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(ka, qf[1][ks], lo, 0, 0, 0);
         }
         const float unit = __builtin_ldexpf(1.f, -qexp);
 #pragma unroll
-        for (int r = 0; r < 4; ++r) s[t][r] = (s[t][r] + lo[r]) * unit;
+        for (int r = 0; r < 4; ++r) s[t][r] = join_parts(s[t][r], lo[r]) * unit;
     }
     // ---- softmax of head c16 over the wave's tokens
     const bool tail = wt0 + KW > seq;   // wave-uniform
@@ -1291,7 +1304,7 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     l += __shfl_xor(l, 32);
 
     // P^T: slot 8 g + e is the wave's key 32 kk + 8 g + e (KW 16: 4 g + e, e < 4)
-    half8 pf[3][NK];
+    half8 pf[2][NK];
 #pragma unroll
     for (int kk = 0; kk < NK; ++kk)
 #pragma unroll
@@ -1300,14 +1313,13 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
             for (int r = 0; r < 4; r += 2) {
                 const int t = KW >= 32 ? 2 * kk + sb : 0;
                 const bool z = KW < 32 && sb == 1;
-                float p0 = z ? 0.f : s[t][r] * PSC, p1 = z ? 0.f : s[t][r + 1] * PSC;
+                float2v p = {z ? 0.f : s[t][r] * PSC, z ? 0.f : s[t][r + 1] * PSC};
 #pragma unroll
-                for (int i = 0; i < 3; ++i) {
-                    const auto v = __builtin_amdgcn_cvt_pkrtz(p0, p1);
+                for (int i = 0; i < 2; ++i) {
+                    const half2v v = __builtin_convertvector(p, half2v);
                     pf[i][kk][4 * sb + r] = v[0];
                     pf[i][kk][4 * sb + r + 1] = v[1];
-                    p0 -= (float)v[0];
-                    p1 -= (float)v[1];
+                    p = (float2v){p[0] - (float)v[0], p[1] - (float)v[1]};
                 }
             }
     if (tail || wnew) {
@@ -1335,13 +1347,15 @@ __global__ __launch_bounds__(256) void attn_fused_mfma_kernel(FusedAttnArgs a) {
     // ---- O^T = V^T . P^T: lane (g, c16) holds dims 16 dt + 4 g + r of head c16
 #pragma unroll
     for (int dt = 0; dt < 8; ++dt) {
-        float4v o = {0.f, 0.f, 0.f, 0.f};
+        float4v o = {0.f, 0.f, 0.f, 0.f}, lo = o;
 #pragma unroll
         for (int kk = 0; kk < NK; ++kk) {
             const half8 va = __builtin_bit_cast(half8, vreg[kk][dt]);
-#pragma unroll
-            for (int i = 2; i >= 0; --i) o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pf[i][kk], o, 0, 0, 0);
+            o = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pf[0][kk], o, 0, 0, 0);
+            lo = __builtin_amdgcn_mfma_f32_16x16x32_f16(va, pf[1][kk], lo, 0, 0, 0);
         }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) o[r] = join_parts(o[r], lo[r]);
         if (c16 < GM) *(float4v *)&osh[w][c16][16 * dt + 4 * g] = o;
     }
     if (g == 0 && c16 < GM) mlsh[w][c16] = make_float2(m, l);
@@ -2383,7 +2397,7 @@ int nnz_attn_launch(nnz_ctx *ctx, const void *q, int qdt, const void *kc, const 
 // query head).  Measured, the attention launch alone, wave / MFMA kernel: 16
 // query and 8 KV heads, 100 tokens 3.52 / 3.96 us, 640 4.02 / 4.29, 1000 4.17 /
 // 4.20; 32 query heads, 200 tokens (128 blocks) 3.65 / 4.13, 640 (320 blocks)
-// 4.85 / 4.37 (the MFMA kernel before its third f16 parts, now 0.35 more).
+// 4.85 / 4.37 (the MFMA kernel before its parts were scaled, now 0.4 more).
 static bool attn_fused_by_wave(uint32_t chunks, uint32_t hq) { return chunks * hq <= 256; }
 
 // Chunk length (tokens per partial) of the fused decode attention: 64 while
@@ -2392,7 +2406,7 @@ static bool attn_fused_by_wave(uint32_t chunks, uint32_t hq) { return chunks * h
 // and merge together, 3001 tokens 9.2 -> 8.1 us, 8192 13.9 -> 11.5; 1500 tokens
 // 7.1 -> 7.5, but then its 12 chunks need no merge launch in the decode step.
 // (256-token chunks, 64 per wave: 10.9 us at 3001, 12.5 at 8192; all of these
-// before the third f16 parts, which cost every length 0.35-0.4 us.)
+// before the f16 parts were scaled, which costs every length 0.4 us.)
 uint32_t nnz_attn_fused_chunk(uint32_t max_seq, uint32_t hq, uint32_t head_dim) {
     const uint32_t n64 = ceil_div(max_seq, (uint32_t)FCHUNK);
     if (head_dim != 128 || n64 <= NNZ_O_MERGE_MAX_CHUNKS || attn_fused_by_wave(n64, hq)) return (uint32_t)FCHUNK;

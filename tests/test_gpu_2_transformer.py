@@ -187,6 +187,38 @@ def test_gqa_fused_1pass_kernels(dev, hq, hkv, seq, ctx):
     assert np.isnan(host(kcd)[:, seq:]).all() and np.isnan(host(vcd)[:, :, seq:]).all()
 
 
+def test_gqa_fused_1pass_infinite_cache(dev):
+    """An infinity in the caches of a long context does what it does to a
+    float32 product: a key whose score is -inf has no weight (the output is
+    finite and the other tokens'), a value of +inf makes its dim +inf."""
+    hq, hkv, d, seq, ctx, theta = 16, 8, 128, 1100, 1104, 1e6
+    pos = seq - 1
+    rng = np.random.default_rng(2202)
+    qn, kn = ((1 + 0.1 * rng.standard_normal(d)).astype(np.float32) for _ in range(2))
+    kc = np.zeros((hkv, ctx, d), np.float16)
+    vc = np.zeros((hkv, d, ctx), np.float16)
+    kc[:, :pos] = rng.standard_normal((hkv, pos, d))
+    vc[:, :, :pos] = rng.standard_normal((hkv, d, pos))
+    q = rng.standard_normal((hkv, 1, d)).repeat(hq // hkv, 1).reshape(hq, d).astype(np.float16)
+    kr, vr = (rng.standard_normal((hkv, d)).astype(np.float16) for _ in range(2))
+    rot = O.head_norm_rope(q.astype(np.float64), qn, pos, theta)
+    kc[0, 500, 3] = -np.inf * np.sign(rot[0, 3])
+    kc[2, 1098, 70] = -np.inf * np.sign(rot[4, 70])
+    vc[1, 7, 20] = np.inf
+    dims = L.GQAFusedDims(hq, hkv, d, seq, ctx, hq // hkv, pos, 1e-6, theta)
+    scr = torch.zeros(ops.gqa_scratch_bytes(L.GQADims(hq, hkv, d, seq, ctx, hq // hkv)), dtype=torch.uint8, device="cuda")
+    out = torch.empty(hq, d, dtype=torch.float16, device="cuda")
+    ops.dispatch_gqa_attention_fused_1pass(dev, tdev(q), tdev(kc), tdev(vc), out, tdev(kr), tdev(vr), tdev(qn),
+                                           tdev(kn), scr, dims)
+    dev.sync()
+    got = host(out)
+    ref = O.gqa_fused_step(q.astype(np.float64), kr.astype(np.float64), vr.astype(np.float64),
+                           kc[:, :seq].astype(np.float64), vc[:, :, :seq].astype(np.float64), qn, kn, pos, theta)
+    assert (got[2:4, 7] == np.inf).all() and (ref[2:4, 7] == np.inf).all()
+    got[2:4, 7] = ref[2:4, 7] = 0.0
+    assert_close(got, O.f16(ref), what="infinite cache")
+
+
 @pytest.mark.parametrize("form,qscale,kscale", [("plain", 1.0, 1.0), ("small norms", 2.0 ** -10, 2.0 ** 10),
                                                 ("large norms", 2.0 ** 20, 2.0 ** -17), ("sink", 1.0, 1.0)])
 def test_attention_partials_precision(dev, form, qscale, kscale):
