@@ -136,7 +136,8 @@ int nnz_graph_destroy(nnz_graph *g);
 
 /* Context options (new; the reference has no counterpart).
  * NNZ_OPT_Q1_MATRIX_CORES selects the kernel of 1-bit QMVs with group size 128
- * and K = 2048 (or K = 4096 or 6144, f32 in and out, one matrix): 0 = the library's choice by shape (default), 1 = the
+ * and K = 2048 (or K = 4096 or 6144, f32 in and out, one matrix) and 4-byte
+ * aligned scales: 0 = the library's choice by shape (default), 1 = the
  * block-scaled MFMA kernel wherever it applies, 2 = never it (the VALU
  * kernels).  Results agree to float32 rounding either way; a captured graph
  * keeps the kernels chosen at capture. */
@@ -297,7 +298,14 @@ int nnz_dispatch_dequant(nnz_ctx *ctx, const nnz_qweight *w, float *output, nnz_
  * aligned): every result is BF16-truncated before its store, += or the
  * SiLU*mul product's store, like the Q4 decode kernels
  * (q4mv_bf16_specialized.metal:52-57).  M, K and the group size multiples of
- * 64, the group size a power of two. */
+ * 64, the group size a power of two.
+ *
+ * A long K with few output tiles may be split, the partial sums meeting in a
+ * 4 MiB workspace of the context (allocated with it).  Not while the stream is
+ * captured: a graph may be replayed beside the context's other work, or after
+ * its end.  A captured call of such a shape therefore runs unsplit: slower
+ * (M = 4096, K = 12288, P = 45: 29 us against 15), and its fp32 sums are in
+ * another order, equal to the eager call's to rounding but not to the bit. */
 #define NNZ_GEMM_STORE_F16 0
 #define NNZ_GEMM_STORE_F32 1
 #define NNZ_GEMM_RESADD    2
