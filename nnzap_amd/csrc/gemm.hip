@@ -672,8 +672,8 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(2))) v
 // the VALU.  Measured before -> now, weights rotated: 1-bit gate/up 2 x 6144 x
 // 2048 at P = 512 33.8 -> 30.5 us (845 TFLOP/s), 2 x 9728 x 2560 at P = 3001
 // 295 -> 268 (1113 TFLOP/s; the library's bf16 GEMM of that size without any
-// dequantisation 1161); 2560 x 9728 at P = 3001 190 -> 148, 2560 x 4096 82 ->
-// 68, 6144 x 2560 120 -> 97; 4-bit gate/up 2 x 6144 x 2048 at P = 512 59.7 ->
+// dequantisation 1161); 2560 x 9728 at P = 3001 190 -> 144, 2560 x 4096 82 ->
+// 63, 6144 x 2560 120 -> 86; 4-bit gate/up 2 x 6144 x 2048 at P = 512 59.7 ->
 // 47, 2 x 9728 x 2560 at P = 1500 290 -> 230.  Bounds now: 1-bit, one round of
 // blocks at P = 512 (first loads and epilogue overlap nothing), at large P the
 // L2-to-LDS rate of A (8.7 TB/s over the chip) and MFMA issue; 4-bit, VALU
@@ -704,6 +704,13 @@ __device__ __forceinline__ T *uniform_ptr(T *p) {
     const uint32_t lo = __builtin_amdgcn_readfirstlane((uint32_t)v);
     const uint32_t hi = __builtin_amdgcn_readfirstlane((uint32_t)(v >> 32));
     return (T *)((uint64_t)hi << 32 | lo);
+}
+// Low half of a lane value times a uniform one, in one register: the compiler's
+// multiply-add has a 64-bit result, whose other half would live as long.
+__device__ __forceinline__ uint32_t mul_lo(uint32_t v, uint32_t s) {
+    uint32_t r;
+    asm("v_mul_lo_u32 %0, %1, %2" : "=v"(r) : "v"(v), "s"(s));
+    return r;
 }
 template <class T>
 __device__ __forceinline__ uint32_t lds_addr(T *p) {
@@ -771,12 +778,12 @@ constexpr size_t qgemm_lds() {
     return 2 * (size_t)(BM * BK * KQ) * 2 + 2 * (size_t)cpb * (64 * NSUB) * (64 + 8) + (BITS == 4 ? 4 * 64 * NSUB : 4);
 }
 constexpr size_t LDS_CU = 160 * 1024;
-static_assert(qgemm_lds<1, 1, 8>() <= LDS_CU && 2 * qgemm_lds<1, 1, 4>() <= LDS_CU && 3 * qgemm_lds<1, 1, 2>() <= LDS_CU && 2 * qgemm_lds<1, 2, 2>() <= LDS_CU &&
+static_assert(qgemm_lds<1, 1, 8>() <= LDS_CU && 2 * qgemm_lds<1, 1, 4>() <= LDS_CU && 3 * qgemm_lds<1, 2, 2>() <= LDS_CU &&
               qgemm_lds<4, 2, 4>() <= LDS_CU && 2 * qgemm_lds<4, 1, 4>() > LDS_CU && 3 * qgemm_lds<4, 2, 2>() <= LDS_CU,
               "blocks per CU");
 
 template <int BITS, int MODE, int NSUB, int KQ, bool SPLIT>
-__global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
+__global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(3))) void qgemm_kernel(GemmArgs ga) {
     constexpr bool PAIR = MODE == NNZ_GEMM_SILU_PAIR;
     static_assert(!PAIR || (NSUB == 2 && !SPLIT), "a pair has two sub-blocks, and is not split");
     constexpr int SK = BK * KQ, PIECES = SK / 8, THREADS = 128 * KQ, A_LOADS = 4, ROWS = 64 * NSUB;
@@ -848,13 +855,10 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     uint32_t avoff[A_LOADS];
 #pragma unroll
     for (int u = 0; u < A_LOADS; ++u)
-        avoff[u] = (min(p0 + (uint32_t)(lr + 16 * u), ga.P - 1) - p0) * K * 2u + (uint32_t)(lp ^ (lr & 15)) * 16u;
+        avoff[u] = mul_lo(min(p0 + (uint32_t)(lr + 16 * u), ga.P - 1) - p0, K * 2u) + (uint32_t)(lp ^ (lr & 15)) * 16u;
     const char *const abase = (const char *)(ga.A + (size_t)p0 * K + kb);
     // W chunk: 64 bytes per row as 4 pieces, piece p of row r at slot
     // p ^ ((r >> 2) & 3); instruction i fills rows 16 i .. 16 i + 15.
-    const int wrow = lane >> 2;
-    const uint32_t wvoff = (uint32_t)wrow * rowbytes + (uint32_t)((lane & 3) ^ ((wrow >> 2) & 3)) * 16u;
-
     auto issue_a = [&](uint32_t st) __attribute__((always_inline)) {
         const char *const sb = abase + (size_t)st * (SK * 2);
         const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(As[st & 1] + 8 * (wave * 64)));
@@ -862,7 +866,14 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
         for (int u = 0; u < A_LOADS; ++u) load_lds_b128(uniform_ptr(sb), avoff[u], l0 + 16u * (uint32_t)(u * THREADS));
     };
     // buffer b of W: chunks b CPS .. of every row
+    // (the lane's number and offsets are computed here each time: three
+    // registers fewer in the loop)
     auto issue_w = [&](uint32_t b) __attribute__((always_inline)) {
+        uint32_t ln;
+        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+        const uint32_t wvoff = mul_lo(ln >> 2, rowbytes) + ((ln & 3u) ^ (ln >> 4)) * 16u;
+        // scales: 2 dwords of a row (1-bit), or one
+        const uint32_t svoff = BITS == 1 ? mul_lo(ln >> 1, G * 2u) + (ln & 1u) * 4u : mul_lo(ln, G * 2u);
 #pragma unroll
         for (int i0 = 0; i0 < W_INSTR; i0 += WAVES) {
             const int i = i0 + wave;
@@ -880,14 +891,14 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
                 const int c = i / (2 * NSUB), j = i % (2 * NSUB), sub = j >> 1, h = j & 1;
                 const uint32_t l0 = __builtin_amdgcn_readfirstlane(lds_addr(&Sc[b & 1][c][sub * 128 + h * 64]));
                 if constexpr (BITS == 1) {   // 4 scales of a row = 2 dwords: rows 32 h .. of the sub-block
-                    const char *const sb = (const char *)(sub ? sbase1 : sbase0) + (size_t)(b * CPS + c) * 8;
-                    load_lds_b32(uniform_ptr(sb), (uint32_t)(32 * h + (lane >> 1)) * G * 2u + (uint32_t)(lane & 1) * 4u, l0);
+                    const char *const sb = (const char *)(sub ? sbase1 : sbase0) + (size_t)(32 * h) * G * 2 + (size_t)(b * CPS + c) * 8;
+                    load_lds_b32(uniform_ptr(sb), svoff, l0);
                 } else {                     // 2 scales (h = 0) or biases (h = 1) of a row = 1 dword
                     const uint16_t *const s0 = uniform_ptr(sbase0), *const s1 = uniform_ptr(sbase1);
                     const uint16_t *const b0 = uniform_ptr(bbase0), *const b1 = uniform_ptr(bbase1);
                     const uint16_t *const t0 = h ? b0 : s0, *const t1 = h ? b1 : s1;
                     const char *const sb = (const char *)(sub ? t1 : t0) + (size_t)(b * CPS + c) * 4;
-                    load_lds_b32(uniform_ptr(sb), (uint32_t)lane * G * 2u, l0);
+                    load_lds_b32(uniform_ptr(sb), svoff, l0);
                 }
             }
         }
@@ -903,8 +914,9 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
     // 1-bit launches on two k-phases keep a second set, for the u = 1 MFMAs, so
     // that a float32 chain is no longer than four k-phases make it: with one
     // set the result was 1.4 times as far from float64 (2048 x 6144, P = 1500:
-    // 3.5e-7 against 2.5e-7).  On 128-row blocks (179 registers) that leaves
-    // two blocks per CU instead of three.
+    // 3.5e-7 against 2.5e-7).  Three 128-row blocks per CU leave a lane 168
+    // registers, 128 of them these sums: the loop's addresses are held down to
+    // that (with spills, or two blocks per CU, it is 1.1 to 1.8 times slower).
     constexpr bool TWO = BITS == 1 && KQ == 2 && !PAIR;
     float4v acc1[TWO ? NSUB : 1][4][2];
     if constexpr (TWO) {
@@ -991,14 +1003,17 @@ __global__ __launch_bounds__(128 * KQ) void qgemm_kernel(GemmArgs ga) {
             for (int i = 0; i < 4; ++i)
                 af[u][i] = *(const half8 *)(buf + (i * 16 + r16) * SK + 8 * ((kq * 8 + 2 * q + u) ^ r16));
         if constexpr (BITS == 1) {
+            // the lane's codes and scale of row 32 wn + r16; its other rows lie
+            // at constant offsets (multiples of 16 rows swizzle alike)
+            const char *const wp = (const char *)&Wc[wb][c][0] + (32 * wn + r16) * 64 +
+                                   (((cs >> 1) ^ ((r16 >> 2) & 3)) << 4) + (cs & 1) * 8 + 2 * q;
+            const char *const sp = (const char *)&Sc[wb][c][0] + (32 * wn + r16) * 8 + (cs >> 1) * 2;
 #pragma unroll
             for (int s = 0; s < NSUB; ++s)
 #pragma unroll
                 for (int j = 0; j < 2; ++j) {
-                    const int row = 64 * s + 32 * wn + 16 * j + r16;
-                    const uint32_t h = *((const uint16_t *)&Wc[wb][c][row * 16 + (((cs >> 1) ^ ((row >> 2) & 3)) << 2)] +
-                                         (cs & 1) * 4 + q);
-                    const uint32_t sc = *((const uint16_t *)&Sc[wb][c][row * 2] + (cs >> 1));
+                    const uint32_t h = *(const uint16_t *)(wp + (64 * s + 16 * j) * 64);
+                    const uint32_t sc = *(const uint16_t *)(sp + (64 * s + 16 * j) * 8);
                     half8 b0, b1;
                     expand_bits16(h, (sc | (sc << 16)) ^ 0x80008000u, b0, b1);
 #pragma unroll
@@ -1274,16 +1289,13 @@ void qgemm_split(nnz_ctx *ctx, GemmArgs ga, uint32_t rows, uint32_t splits) {
 }
 
 // Shape of a single-matrix launch (one or more row segments), by how many
-// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (42 KB of LDS; of 128
-// rows two 1-bit ones, by registers, or three 4-bit ones), of KQ = 4 two 1-bit
-// ones (75 KB) or one 4-bit one (84 KB), one of KQ = 8 (140 KB).
+// 64-row blocks g it has: a CU holds 3 blocks of KQ = 2 (42 KB of LDS, 51 with
+// 128 rows), of KQ = 4 two 1-bit ones (75 KB) or one 4-bit one (84 KB), one of
+// KQ = 8 (140 KB).
 //   * More than one round of KQ = 2 64-row blocks: 128-row blocks, half the A
-//     traffic (1-bit 2560 x 4096, P = 3001: 66 us against 72 with 64 rows; 6144
-//     x 2560 97 against 104; 2560 x 9728, P = 1500 77 against 104) -- except
-//     1-bit grids of 1025 to 1536, whose 513 to 768 128-row blocks leave the
-//     second round of 512 half empty (6144 x 2560, P = 768: 31.1 us on 64 rows
-//     against 36.9; 4096 x 12288, P = 1280 139 against 156; at 1536, P = 1024,
-//     37.2 against 37.1).
+//     traffic (1-bit 2560 x 4096, P = 3001: 63 us against 72 with 64 rows; 6144
+//     x 2560 86 against 104, P = 768 29.5 against 31.1; 2560 x 9728, P = 1500 74
+//     against 104).
 //   * Up to 768, from 512 (1-bit) or 256 (4-bit), where KQ = 4 takes a second
 //     round: one round of KQ = 2 64-row blocks (2048 x 2048, P = 1500: 18.0 us
 //     against 23.7 on KQ = 4; 6144 x 2560, P = 512: 22.6 against 25.0; 4-bit
@@ -1314,7 +1326,7 @@ void qgemm_single(nnz_ctx *ctx, const GemmArgs &ga, uint32_t rows, bool rows128)
         return qgemm_split<BITS, MODE, 1, 4>(ctx, ga, rows, S);
     }
     if (g > 768) {
-        if (rows128 && (BITS == 4 || g <= 1024 || g > 1536)) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
+        if (rows128) qgemm_start<BITS, MODE, 2, 2>(ctx, ga, rows);
         else qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
     } else if (g > (BITS == 1 ? 512u : 256u)) {
         qgemm_start<BITS, MODE, 1, 2>(ctx, ga, rows);
