@@ -790,6 +790,7 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(3))) v
     constexpr int CSTEPS = BITS == 1 ? 8 : 2;                    // 64-k steps per W chunk
     constexpr int CPS = KQ > CSTEPS ? KQ / CSTEPS : 1;           // chunks per buffer
     constexpr int SPC = CSTEPS > KQ ? CSTEPS / KQ : 1;           // stages per buffer
+    constexpr bool TWO = BITS == 1 && KQ == 2 && !PAIR;          // two accumulator sets
     constexpr int W_INSTR = 4 * NSUB * CPS, S_INSTR = 2 * NSUB * CPS, WAVES = 2 * KQ;
     __shared__ __attribute__((aligned(16))) f16_t As[2][BM * SK];
     __shared__ __attribute__((aligned(16))) uint32_t Wc[2][CPS][ROWS * 16];
@@ -866,11 +867,13 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(3))) v
         for (int u = 0; u < A_LOADS; ++u) load_lds_b128(uniform_ptr(sb), avoff[u], l0 + 16u * (uint32_t)(u * THREADS));
     };
     // buffer b of W: chunks b CPS .. of every row
-    // (the lane's number and offsets are computed here each time: three
-    // registers fewer in the loop)
+    // (with two accumulator sets on 128 rows, once in four stages, the lane's
+    // number and offsets are computed here each time: three registers fewer in
+    // the loop)
     auto issue_w = [&](uint32_t b) __attribute__((always_inline)) {
-        uint32_t ln;
-        asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
+        uint32_t ln = (uint32_t)lane;
+        if constexpr (TWO && NSUB == 2)
+            asm volatile("v_mbcnt_lo_u32_b32 %0, -1, 0\n\tv_mbcnt_hi_u32_b32 %0, -1, %0" : "=v"(ln));
         const uint32_t wvoff = mul_lo(ln >> 2, rowbytes) + ((ln & 3u) ^ (ln >> 4)) * 16u;
         // scales: 2 dwords of a row (1-bit), or one
         const uint32_t svoff = BITS == 1 ? mul_lo(ln >> 1, G * 2u) + (ln & 1u) * 4u : mul_lo(ln, G * 2u);
@@ -911,13 +914,12 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(3))) v
         for (int i = 0; i < 4; ++i)
 #pragma unroll
             for (int j = 0; j < 2; ++j) acc[s][i][j] = (float4v){0.f, 0.f, 0.f, 0.f};
-    // 1-bit launches on two k-phases keep a second set, for the u = 1 MFMAs, so
-    // that a float32 chain is no longer than four k-phases make it: with one
+    // 1-bit launches on two k-phases (TWO) keep a second set, for the u = 1
+    // MFMAs, so that a float32 chain is no longer than four k-phases make it: with one
     // set the result was 1.4 times as far from float64 (2048 x 6144, P = 1500:
     // 3.5e-7 against 2.5e-7).  Three 128-row blocks per CU leave a lane 168
     // registers, 128 of them these sums: the loop's addresses are held down to
     // that (with spills, or two blocks per CU, it is 1.1 to 1.8 times slower).
-    constexpr bool TWO = BITS == 1 && KQ == 2 && !PAIR;
     float4v acc1[TWO ? NSUB : 1][4][2];
     if constexpr (TWO) {
 #pragma unroll
@@ -946,7 +948,8 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(3))) v
         const int row = tid / TPR, sub = row >> 6;
         const uint16_t *const s0 = uniform_ptr(sbase0), *const s1 = uniform_ptr(sbase1);
         const auto *const rs = (const __attribute__((address_space(1))) u32x4 *)((sub ? s1 : s0) + (size_t)(row & 63) * G);
-        uint32_t mx = 0, mn1 = 0xFFFFFFFFu;    // largest |s|, smallest nonzero |s| less 1 (bits)
+        typedef uint16_t u16x2 __attribute__((ext_vector_type(2)));
+        u16x2 mx2 = {0, 0}, mn2 = {0xFFFF, 0xFFFF};   // largest |s|, smallest nonzero |s| less 1 (bits)
         const uint32_t np = (ke - kb) / 512;   // 16-byte pieces of the row's scales
         for (uint32_t p = tid % TPR; p < np; p += 4 * TPR) {
             u32x4 v[4];   // four loads in flight; past the end the last piece again
@@ -954,11 +957,12 @@ __global__ __launch_bounds__(128 * KQ) __attribute__((amdgpu_waves_per_eu(3))) v
             for (int e = 0; e < 4; ++e) v[e] = rs[min(p + (uint32_t)(e * TPR), np - 1)];
 #pragma unroll
             for (int e = 0; e < 16; ++e) {
-                const uint32_t a = v[e / 4][e % 4] & 0x7FFFu, b = (v[e / 4][e % 4] >> 16) & 0x7FFFu;
-                mx = max(mx, max(a, b));
-                mn1 = min(mn1, min(a - 1u, b - 1u));
+                const u16x2 a = __builtin_bit_cast(u16x2, v[e / 4][e % 4] & 0x7FFF7FFFu);
+                mx2 = __builtin_elementwise_max(mx2, a);
+                mn2 = __builtin_elementwise_min(mn2, a - (u16x2){1, 1});
             }
         }
+        uint32_t mx = max(mx2[0], mx2[1]), mn1 = min(mn2[0], mn2[1]);
 #pragma unroll
         for (int o = 1; o < TPR; o *= 2) {
             mx = max(mx, (uint32_t)__shfl_xor((int)mx, o, 64));
